@@ -195,8 +195,10 @@ typedef struct piper_prepare_args {
 #define PIPER_PLAN_CAUSAL_FORWARD 2 /* causal: query tiles in forward order */
 #define PIPER_PLAN_NO_XCD_REMAP 4   /* hardware workgroup order */
 #define PIPER_PLAN_CAUSAL_INTERLEAVE 8 /* causal, longest first: query tiles dispatched longest first
-                                          across the heads of each XCD (across all heads with
-                                          PIPER_PLAN_NO_XCD_REMAP) instead of head by head */
+                                          across heads (with PIPER_PLAN_WORK_QUEUE across each
+                                          queue's) instead of head by head.  Without the bit, grids
+                                          without work queues go across heads while the tile
+                                          records fit the last-level cache */
 #define PIPER_PLAN_THREE_WORKGROUPS 16 /* three 4-wave workgroups per CU (three waves per SIMD, 2-stage LDS
                                           rings); overrides PIPER_PLAN_FOUR_WAVES.  Both operators */
 /* Key-range split (Piper Attention, non-causal, with PIPER_PLAN_THREE_WORKGROUPS): the key tiles

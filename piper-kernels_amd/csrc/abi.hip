@@ -201,7 +201,11 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
   ap.score_multiplier = ap.scale_log2e * 67108864.0f;  // x 2^26: exact
   ap.causal_forward = (plan & PIPER_PLAN_CAUSAL_FORWARD) ? 1 : 0;
   ap.xcd_remap = (plan & PIPER_PLAN_NO_XCD_REMAP) ? 0 : 1;
-  ap.causal_interleave = (plan & PIPER_PLAN_CAUSAL_INTERLEAVE) ? 1 : 0;
+  // the work queues' order is the plan's; a hardware-dispatched grid's is chosen by size where the plan
+  // does not ask for the one across heads
+  ap.across_heads = (plan & PIPER_PLAN_CAUSAL_INTERLEAVE) != 0 ||
+                    (!work_queue && piper::order_across_heads(ap.batch_heads, ap.nkb,
+                                                              piper::kv_tile_bytes(static_cast<int>(s.head_dim))));
   ap.heads = static_cast<int>(s.heads);
   ap.per_thread = (flags & PIPER_ATTENTION_QK_PER_THREAD) ? 1 : 0;
   if (query != nullptr) {
@@ -545,7 +549,8 @@ int piper_sage_attention_forward(const piper_sage_attention_args* a, void* strea
   sp.scale_log2e = static_cast<float>(static_cast<double>(a->scale) * 1.4426950408889634);
   sp.causal_forward = (a->plan & PIPER_PLAN_CAUSAL_FORWARD) ? 1 : 0;
   sp.xcd_remap = (a->plan & PIPER_PLAN_NO_XCD_REMAP) ? 0 : 1;
-  sp.causal_interleave = (a->plan & PIPER_PLAN_CAUSAL_INTERLEAVE) ? 1 : 0;
+  sp.across_heads = (a->plan & PIPER_PLAN_CAUSAL_INTERLEAVE) != 0 ||
+                    piper::order_across_heads(sp.batch_heads, sp.nkb, piper::sage_tile_bytes(static_cast<int>(s.head_dim)));
   sp.per_thread = (a->flags & PIPER_ATTENTION_QK_PER_THREAD) ? 1 : 0;
   sp.fp16_partials = (a->flags & PIPER_SAGE_FP16_PARTIALS) ? 1 : 0;
   if (static_cast<int64_t>(sp.query_tiles) * sp.batch_heads > 0x7fffffff)

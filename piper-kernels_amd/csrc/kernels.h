@@ -128,6 +128,18 @@ struct AttnParams {
   void* output;
   int batch_heads;
   int query_length;
+// Order of a causal longest-first grid whose plan leaves it open: across heads while all K/V tile
+// records fit the 256 MiB last-level cache, head by head beyond (then only a few heads' records are
+// live at a time).  Measured, head by head against across heads, Piper Attention at D = 128: B2 H16
+// S1531 48.4 -> 41.8 us, B1 H32 S4096 168 -> 126, B1 H24 S16384 (126 MB of records) 1409 -> 1302, B1 H42
+// S20000 (269 MB) 3866 -> 3765, B1 H48 S24000 (369 MB) 5693 -> 5873, B1 H40 S32768 (419 MB) 8605 -> 9065;
+// batch-heads not divisible by 8, B1 H12 S20000 1212 -> 1015; D = 64, B4 H40 S8192 (231 MB) 1709 ->
+// 1501; SageAttention2++ B1 H24 S4096 143 -> 95, B1 H10 S16384 678 -> 467.
+constexpr long kAcrossHeadsBytes = 256L << 20;
+inline bool order_across_heads(long batch_heads, long key_tiles, int tile_bytes) {
+  return batch_heads * key_tiles * tile_bytes <= kAcrossHeadsBytes;
+}
+
   int key_length;
   int sq32;
   int sk64;
@@ -137,7 +149,7 @@ struct AttnParams {
   float scale_log2e;
   int causal_forward;  // causal grids: 1 = query tiles in forward order, 0 = longest first
   int xcd_remap;       // 1 = consecutive workgroups of a head share an XCD, 0 = hardware order
-  int causal_interleave;  // causal, longest first: 1 = across the heads of an XCD, 0 = head by head
+  int across_heads;    // causal, longest first: 1 = across heads, 0 = head by head
   // Fused query quantisation: each wave quantises its own 32-row query block from `query`
   // (query_code and query_scale are then unused).
   int fused_query;
@@ -206,7 +218,7 @@ struct SageParams {
   float scale_log2e;
   int causal_forward;
   int xcd_remap;
-  int causal_interleave;
+  int across_heads;
   int per_thread;  // Q/K scales per thread group (the tile's four K slots, per-row-group Q scales)
   int fp16_partials;  // round each block's FP8 product to FP16 (the reference's arithmetic)
 };

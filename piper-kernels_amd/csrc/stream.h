@@ -50,13 +50,12 @@ struct Ring {
 
 // Workgroup -> (batch-head, query tile) of both attention kernels.  With the XCD remap the
 // logical ids of one XCD are contiguous (xcd_remap).  Non-causal grids and causal grids in
-// forward order walk the query tiles of one head after another; causal grids in longest-first
-// order (the work of a query tile grows with its index) walk each head's tiles longest first.
-// With causal_interleave they instead go in longest-processing-time order across the heads
-// that share an L2: when the batch-heads split evenly over the 8 XCDs, each XCD's range covers
-// its own batch-heads and walks the query tiles longest first across all of them (without the
-// remap the whole grid does).  That shortens the tail of short and medium sequences; for long
-// sequences with many heads the head-by-head order keeps more of the K/V reuse in L2.
+// forward order walk the query tiles of one head after another.  Causal grids in longest-first
+// order (the work of a query tile grows with its index) walk each head's tiles longest first or, with
+// across_heads, longest first across heads: when the batch-heads split evenly over the 8 XCDs each
+// XCD's range covers its own batch-heads, otherwise the whole grid walks all heads in hardware order.
+// Head by head, the grid ends with the last heads' long tiles running beside empty slots; across
+// heads, more tile records are live at once (across_heads in kernels.h has the rule and both sides).
 struct TileCoord {
   int bh;
   int qtile;
@@ -64,13 +63,13 @@ struct TileCoord {
 
 template <bool kCausal, class Params>
 __device__ __forceinline__ TileCoord workgroup_tile(const Params& p) {
-  const int logical = p.xcd_remap ? xcd_remap(blockIdx.x, gridDim.x) : static_cast<int>(blockIdx.x);
   const int qt = p.query_tiles;
-  if (kCausal && !p.causal_forward && p.causal_interleave && !(p.xcd_remap && (p.batch_heads & 7) != 0)) {
+  if (kCausal && !p.causal_forward && p.across_heads) {
     int heads = p.batch_heads;
     int base_bh = 0;
-    int r = logical;
-    if (p.xcd_remap) {  // batch_heads % 8 == 0: one group of heads per XCD
+    int r = static_cast<int>(blockIdx.x);
+    if (p.xcd_remap && (p.batch_heads & 7) == 0) {  // one group of heads per XCD
+      const int logical = xcd_remap(blockIdx.x, gridDim.x);
       heads = p.batch_heads >> 3;
       const int group = logical / (heads * qt);
       base_bh = group * heads;
@@ -79,6 +78,7 @@ __device__ __forceinline__ TileCoord workgroup_tile(const Params& p) {
     const int rank = r / heads;
     return {base_bh + (r - rank * heads), qt - 1 - rank};
   }
+  const int logical = p.xcd_remap ? xcd_remap(blockIdx.x, gridDim.x) : static_cast<int>(blockIdx.x);
   const int bh = logical / qt;
   const int qtile = logical - bh * qt;
   return {bh, kCausal && !p.causal_forward ? qt - 1 - qtile : qtile};
@@ -86,12 +86,12 @@ __device__ __forceinline__ TileCoord workgroup_tile(const Params& p) {
 
 // Logical id -> (batch-head, query tile) of the work-queue plan, whose `queues` queues hold
 // consecutive logical ranges (queue q: what XCC q runs under the XCD-aware order); qt and
-// batch_heads are p.query_tiles and p.batch_heads, passed in by the caller.  The same order
-// as workgroup_tile with the XCD remap: with causal_interleave and batch-heads divisible by the
-// queues, each queue walks its own batch-heads' query tiles longest first across them.
+// batch_heads are p.query_tiles and p.batch_heads, passed in by the caller.  Longest first, each
+// queue walks its batch-heads one after another; with across_heads and batch-heads divisible by
+// the queues, it walks its own batch-heads' query tiles longest first across them.
 template <bool kCausal, class Params>
 __device__ __forceinline__ TileCoord queue_tile(const Params& p, int logical, int queues, int qt, int batch_heads) {
-  if (kCausal && !p.causal_forward && p.causal_interleave && batch_heads % queues == 0) {
+  if (kCausal && !p.causal_forward && p.across_heads && batch_heads % queues == 0) {
     const int heads = batch_heads / queues;
     const int group = logical / (heads * qt);
     const int r = logical - group * heads * qt;

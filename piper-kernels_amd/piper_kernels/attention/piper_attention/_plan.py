@@ -48,13 +48,15 @@ class MI355XPlan:
     LDS ring). ``causal_longest_first``: causal
     grids dispatch the query tiles with the most key blocks first. ``xcd_remap``: consecutive
     workgroups of one head run on one XCD (its L2 then serves the head's K/V tiles).
-    ``causal_interleave``: causal, longest first, across the heads of an XCD rather than head
-    by head (a shorter tail for short and medium sequences; less L2 reuse for long ones).
-    ``three_per_cu`` (4-wave workgroups only): three workgroups per CU, so three waves share each
-    SIMD (a 2-stage LDS ring per workgroup and no score look-ahead, to fit 168 VGPRs) instead of
-    two.  ``key_parts`` (three per CU, non-causal): the key tiles of each query tile are cut into
-    that many ranges, one workgroup each, whose FP32 partial sums a merge kernel combines; for
-    grids with too few query waves to give every SIMD three (results equal to rounding).
+    ``causal_interleave``: causal, longest first, across heads (of an XCD, or of a queue) rather than
+    head by head; without it, grids without work queues still go across heads while the tile records
+    fit the last-level cache (csrc/kernels.h order_across_heads).
+    ``three_per_cu`` (4-wave workgroups only): three workgroups per CU (four at head size 64), so three
+    waves share each SIMD (a 2-stage LDS ring per workgroup and no score look-ahead, to fit 168 VGPRs)
+    instead of two.  ``key_parts`` (three per CU, non-causal): the key tiles of the query tiles beyond
+    whole rounds of resident workgroups are cut into that many ranges, one workgroup each, whose FP32
+    partial sums a merge kernel combines; for grids, or last rounds, with too few query waves to give
+    every SIMD three (results equal to rounding).
     ``work_queue`` (three per CU, no split): a persistent grid takes the query tiles from one
     queue per XCC instead of the hardware dispatching one workgroup per tile (bit-identical).
     """
