@@ -200,7 +200,8 @@ typedef struct piper_prepare_args {
                                           without work queues go across heads while the tile
                                           records fit the last-level cache */
 #define PIPER_PLAN_THREE_WORKGROUPS 16 /* three 4-wave workgroups per CU (three waves per SIMD, 2-stage LDS
-                                          rings); overrides PIPER_PLAN_FOUR_WAVES.  Both operators */
+                                          rings); four at head_dim 64.  Overrides
+                                          PIPER_PLAN_FOUR_WAVES.  Both operators */
 /* Key-range split (Piper Attention, non-causal, with PIPER_PLAN_THREE_WORKGROUPS): the key tiles
  * of each query tile are cut into `parts` ranges (2..8), one workgroup each, which write their
  * FP32 partial numerator, denominator and reference maximum to the call's workspace; a merge
@@ -210,7 +211,7 @@ typedef struct piper_prepare_args {
 #define PIPER_PLAN_KEY_PARTS(parts) (((parts) - 1) << 5)
 #define PIPER_PLAN_KEY_PARTS_OF(plan) ((((plan) >> 5) & 7) + 1)
 /* Work queues (Piper Attention, with PIPER_PLAN_THREE_WORKGROUPS, no key-range split): a
- * persistent grid of at most three workgroups per CU takes the query tiles, in the order the
+ * persistent grid that fills the CUs' workgroup slots takes the query tiles, in the order the
  * other bits give, from one queue per XCC (relaxed atomic counters in the call's workspace,
  * piper_attention_workspace_bytes) instead of one workgroup per tile dispatched by the hardware,
  * whose in-order round-robin over the XCCs leaves slots idle when tiles differ in length (causal).

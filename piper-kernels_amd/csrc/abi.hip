@@ -179,7 +179,7 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
   if (!aligned16(o.kv_tiles) || !aligned16(o.value_mean) || (reinterpret_cast<uintptr_t>(output) & 7u) != 0)
     return fail(PIPER_ERROR_INVALID_ARGUMENT, "prepared buffers must be 16-byte and the output 8-byte aligned");
 
-  // 3: three 4-wave workgroups per CU (attention_w3_kernel)
+  // 3: three 4-wave workgroups per CU (four at D = 64; attention_w3_kernel)
   const int waves = (plan & PIPER_PLAN_THREE_WORKGROUPS) ? 3 : (plan & PIPER_PLAN_FOUR_WAVES) ? 4 : 8;
   const int block_m = 32 * (waves == 3 ? 4 : waves);
   piper::AttnParams ap{};
@@ -224,12 +224,13 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
     return fail(PIPER_ERROR_UNSUPPORTED, "too many workgroups");
   if (work_queue) {
     // one queue per XCC of the device (one queue if the runtime reports no XCC count), a
-    // persistent grid of three workgroups per CU, or fewer when there are fewer tiles
+    // persistent grid that fills every CU's workgroup slots, or one workgroup per tile when there are fewer tiles
     int cus = 0, xccs = 0;
     if (int st = device_topology(&cus, &xccs)) return st;
     const long tiles = static_cast<long>(ap.query_tiles) * ap.batch_heads;
     ap.queue_xccs = std::max(1, std::min(xccs, piper::kQueueCounters));
-    ap.queue_workers = static_cast<int>(std::max(1L, std::min(tiles, 3L * std::max(cus, 1))));
+    const long slots = static_cast<long>(piper::waves_per_simd(static_cast<int>(s.head_dim))) * std::max(cus, 1);
+    ap.queue_workers = static_cast<int>(std::max(1L, std::min(tiles, slots)));
     ap.queue = static_cast<uint32_t*>(workspace);
   }
 
@@ -532,7 +533,7 @@ int piper_sage_attention_forward(const piper_sage_attention_args* a, void* strea
   if (!aligned16(o.kv_tiles) || !aligned16(o.value_scale) || (reinterpret_cast<uintptr_t>(a->output) & 7u) != 0)
     return fail(PIPER_ERROR_INVALID_ARGUMENT, "prepared buffers must be 16-byte and the output 8-byte aligned");
 
-  // 3: three 4-wave workgroups per CU (sage_attention_w3_kernel)
+  // 3: three 4-wave workgroups per CU (four at D = 64; sage_attention_w3_kernel)
   const int waves = (a->plan & PIPER_PLAN_THREE_WORKGROUPS) ? 3 : (a->plan & PIPER_PLAN_FOUR_WAVES) ? 4 : 8;
   piper::SageParams sp{};
   sp.kv_tiles = static_cast<const uint8_t*>(o.kv_tiles);

@@ -21,7 +21,7 @@
 // * K, V^T, per-key log2 scales, inverse multipliers and column sums of a tile form one
 //   record laid out exactly like its LDS stage (padded rows against bank conflicts); it is
 //   copied with direct global -> LDS loads into an LDS ring: two stages, one block ahead, with
-//   three workgroups per CU (the default); four or six stages in the two-waves-per-SIMD plans.
+//   three workgroups per CU (the default; four at D = 64); four or six stages in the two-waves-per-SIMD plans.
 #include "common.h"
 #include "kernels.h"
 #include "quant.h"
@@ -549,7 +549,7 @@ __device__ __forceinline__ void w3_tile(const AttnParams& p, char* smem, TileCoo
 }
 
 template <int D, bool kCausal, int kOut, bool kPerThread>
-__global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(3, 3)))
+__global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D))))
 attention_w3_kernel(const AttnParams p) {
   __shared__ __attribute__((aligned(16))) char smem[2 * TileLayout<D, 4>::kStageBytes];
   int part = 0;
@@ -571,7 +571,7 @@ attention_w3_kernel(const AttnParams p) {
   w3_tile<D, kCausal, kOut, kPerThread, kCausal>(p, smem, tc, part, threadIdx.x & 63);
 }
 
-// The work-queue plan: a persistent grid (at most three workgroups per CU) whose workgroups take
+// The work-queue plan: a persistent grid (at most waves_per_simd(D) workgroups per CU) whose workgroups take
 // query tiles from one queue per XCC instead of waiting for the hardware to dispatch them.  The
 // hardware deals workgroups round-robin over the XCCs in id order, so a workgroup that cannot be
 // placed on a full XCC holds back the next ones for every XCC: with causal tiles of unequal
@@ -582,7 +582,7 @@ attention_w3_kernel(const AttnParams p) {
 // attention_w3_kernel, so the output is bit-identical.  Every claim increments a counter, so each
 // workgroup ends after at most (tiles + queues) claims; no workgroup waits for another.
 template <int D, bool kCausal, int kOut, bool kPerThread>
-__global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(3, 3)))
+__global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D))))
 attention_w3_queue_kernel(const AttnParams p) {
   static_assert(kOut != kPartials, "the work-queue plan has no key-range split");
   __shared__ __attribute__((aligned(16))) char smem[2 * TileLayout<D, 4>::kStageBytes];

@@ -58,6 +58,15 @@ constexpr int sage_tile_bytes(int head_dim) {
   return (sage_v_offset(head_dim) + head_dim * kv_v_stride() + 1023) / 1024 * 1024;
 }
 
+// Workgroups of four waves resident per CU, so waves per SIMD, under PIPER_PLAN_THREE_WORKGROUPS.
+// D = 128: three (64 numerator registers of a wave leave room for 168 VGPRs per wave).  D = 64: four
+// (32 numerator registers; every instantiation fits 128 VGPRs without a spill, five waves' 96 do not,
+// and four two-stage rings take 88 KiB of LDS).  Measured at D = 64 against three: B1 H16 S8192
+// (1024 query tiles, one round instead of 1.33) 350 -> 301 us, SageAttention2++ 284 -> 256 us; B2 H24
+// S8192 (three rounds instead of four) 901 -> 884 us; B4 H16 S4096 causal 214 -> 208 us,
+// SageAttention2++ 210 -> 197 us.
+constexpr int waves_per_simd(int head_dim) { return head_dim == 64 ? 4 : 3; }
+
 struct InputTensor {
   const void* data;  // 16-bit floats; the head_dim axis is contiguous
   long stride_batch;  // element strides
@@ -171,7 +180,7 @@ inline bool order_across_heads(long batch_heads, long key_tiles, int tile_bytes)
   // tiles from queue_xccs queues of consecutive logical ids, counters in `queue` (zero before the
   // launch).  queue_xccs = 0: the hardware dispatches one workgroup per query tile.
   int queue_xccs;
-  int queue_workers;  // the persistent grid (at most three workgroups per CU)
+  int queue_workers;  // the persistent grid (at most waves_per_simd workgroups per CU)
   float score_multiplier;  // scale_log2e * 2^26 (kScoreUnit), exact: the logits' multiplier per query scale
   uint32_t* queue;
 };

@@ -24,7 +24,7 @@
 // in that order, is directly the B operand of the FP8 MFMA (which contracts over any key order
 // the A operand shares: V^T rows are read at bytes [16h, +16) and [32 + 16h, +16)); the query
 // is quantised in the prologue; tile records are copied straight into an LDS ring (two stages per
-// workgroup with three workgroups per CU, the default; four or six in the two-waves-per-SIMD plans).
+// workgroup with three workgroups per CU, four at D = 64, the default; four or six in the two-waves-per-SIMD plans).
 #include "common.h"
 #include "kernels.h"
 #include "quant.h"
@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(NW * 64, 8 / NW) sage_attention_kernel(const S
 // tile t - 1 used, then the scores, head and tail of tile t.  Same per-block arithmetic as
 // sage_attention_kernel, in the same order, so the output is bit-identical to the other plans.
 template <int D, bool kCausal, int kOut, bool kPerThread, bool kFp16Partials>
-__global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(3, 3)))
+__global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D))))
 sage_attention_w3_kernel(const SageParams p) {
   constexpr int NW = 4;
   using L = SageLayout<D, NW>;
