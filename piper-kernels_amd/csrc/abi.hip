@@ -213,11 +213,20 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
     ap.query_bf16 = query_dtype == PIPER_BFLOAT16 ? 1 : 0;
     ap.query = to_input(*query);
   }
-  // key-range split: part_tiles tiles per part, and no empty part
+  // key-range split: part_tiles tiles per part, and no empty part; only the query tiles beyond whole
+  // rounds of resident workgroups are split
   ap.key_parts = 1;
   if (key_parts > 1) {
+    int cus = 0, xccs = 0;
+    if (int st = device_topology(&cus, &xccs)) return st;
+    const int64_t tiles = static_cast<int64_t>(ap.query_tiles) * ap.batch_heads;
+    const int64_t slots = static_cast<int64_t>(piper::waves_per_simd(static_cast<int>(s.head_dim))) * std::max(cus, 1);
     ap.part_tiles = static_cast<int>(ceil_div(ap.nkb, key_parts));
     ap.key_parts = static_cast<int>(ceil_div(ap.nkb, ap.part_tiles));
+    ap.whole_tiles = static_cast<int>(std::min<int64_t>(tiles / slots * slots, 0x7fffffff));
+    if (ap.whole_tiles == tiles) ap.key_parts = 1;
+    ap.split_row0 = static_cast<long>(ap.whole_tiles / ap.query_tiles) * s.query_length +
+                    static_cast<long>(ap.whole_tiles % ap.query_tiles) * block_m;
     ap.partials = static_cast<float*>(workspace);
   }
   if (static_cast<int64_t>(ap.query_tiles) * ap.batch_heads * ap.key_parts > 0x7fffffff)

@@ -386,20 +386,19 @@ __global__ void __launch_bounds__(NW * 64, 8 / NW) attention_kernel(const AttnPa
 // of tile t - 1 done), start the copy of tile t + 1 into the stage tile t - 1 used, then the
 // scores, softmax and PV of tile t.  The arithmetic is block_update's, so the output is
 // bit-identical to the other plans.
-// kOut: 0, 1, 2 = fp16, bf16, fp32 output; kPartials = the key-range split's partial sums
-// (non-causal only): the workgroup covers key tiles [part * part_tiles, +part_tiles) of its query
-// tile and writes its numerator, denominator and reference maximum for attention_merge_kernel.
-constexpr int kPartials = 3;
+// kOut: 0, 1, 2 = fp16, bf16, fp32 output.  kSplit (non-causal): the key-range split, whose last
+// workgroups cover key tiles [part * part_tiles, +part_tiles) of a query tile and write the numerator,
+// denominator and reference maximum for attention_merge_kernel; part < 0 is a whole tile.
 
 // One query tile (and, for the key-range split, one key part) of attention_w3_kernel or of the
 // work-queue kernel below: the whole prologue, key loop and epilogue of one workgroup.  The caller
 // provides the LDS stages and the lane id; every wave of the workgroup calls it with the same tile.
-template <int D, bool kCausal, int kOut, bool kPerThread, bool kFreshLane = false>
+template <int D, bool kCausal, int kOut, bool kPerThread, bool kFreshLane = false, bool kSplit = false>
 __device__ __forceinline__ void w3_tile(const AttnParams& p, char* smem, TileCoord tc, int part, int lane) {
   constexpr int NW = 4;
   using L = TileLayout<D, NW>;
   constexpr int kChunksD = D / 32;
-  static_assert(kOut != kPartials || !kCausal, "the key-range split is non-causal");
+  static_assert(!kSplit || !kCausal, "the key-range split is non-causal");
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = lane >> 5;
@@ -413,9 +412,11 @@ __device__ __forceinline__ void w3_tile(const AttnParams& p, char* smem, TileCoo
   // key tiles [t0, t0 + tiles) of this workgroup, local index i = t - t0
   int t0 = 0;
   int tiles = p.nkb;
-  if constexpr (kOut == kPartials) {
-    t0 = part * p.part_tiles;
-    tiles = max(0, min(p.part_tiles, p.nkb - t0));
+  if constexpr (kSplit) {
+    if (part >= 0) {
+      t0 = part * p.part_tiles;
+      tiles = max(0, min(p.part_tiles, p.nkb - t0));
+    }
   }
   int wave_tiles = wave_live ? tiles : 0;
   if constexpr (kCausal) {
@@ -517,58 +518,68 @@ __device__ __forceinline__ void w3_tile(const AttnParams& p, char* smem, TileCoo
   const int en = epilogue_lane & 31;
   const int query = q0 + en;
   if (!wave_live || query >= p.query_length) return;
-  if constexpr (kOut == kPartials) {
-    const long rows = static_cast<long>(p.batch_heads) * p.query_length;
-    const long row = static_cast<long>(part) * rows + static_cast<long>(bh) * p.query_length + query;
-    float* dst = p.partials + row * D;
+  if constexpr (kSplit) {
+    if (part >= 0) {
+      const long rows = split_rows(p);
+      const long row =
+          static_cast<long>(part) * rows + static_cast<long>(bh) * p.query_length + query - p.split_row0;
+      float* dst = p.partials + row * D;
 #pragma unroll
-    for (int j = 0; j < kChunksD; ++j)
+      for (int j = 0; j < kChunksD; ++j)
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<float4*>(dst + 32 * j + 8 * g + 4 * eh) =
-            make_float4(num[j][4 * g + 0], num[j][4 * g + 1], num[j][4 * g + 2], num[j][4 * g + 3]);
-    // both lane halves hold the row's den_total and mref
-    if (eh == 0) reinterpret_cast<float2*>(p.partials + p.key_parts * rows * D)[row] = make_float2(den_total, mref);
-    return;
-  } else {
-    const float rden = (1.0f / 255.0f) / fmaxf(den_total, 1e-30f);  // the numerator holds 255 x the reference's
-    const float* vmean = p.value_mean + static_cast<long>(bh) * D;
-    const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<float4*>(dst + 32 * j + 8 * g + 4 * eh) =
+              make_float4(num[j][4 * g + 0], num[j][4 * g + 1], num[j][4 * g + 2], num[j][4 * g + 3]);
+      // both lane halves hold the row's den_total and mref
+      if (eh == 0) reinterpret_cast<float2*>(p.partials + p.key_parts * rows * D)[row] = make_float2(den_total, mref);
+      return;
+    }
+  }
+  const float rden = (1.0f / 255.0f) / fmaxf(den_total, 1e-30f);  // the numerator holds 255 x the reference's
+  const float* vmean = p.value_mean + static_cast<long>(bh) * D;
+  const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
 #pragma unroll
-    for (int j = 0; j < kChunksD; ++j) {
+  for (int j = 0; j < kChunksD; ++j) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d0 = 32 * j + 8 * g + 4 * eh;
-        float4 m = make_float4(0.f, 0.f, 0.f, 0.f);
-        if constexpr (!kCausal) m = *reinterpret_cast<const float4*>(vmean + d0);
-        store4<kOut>(p.output, out_row + d0, fmaf(num[j][4 * g + 0], rden, m.x), fmaf(num[j][4 * g + 1], rden, m.y),
-                     fmaf(num[j][4 * g + 2], rden, m.z), fmaf(num[j][4 * g + 3], rden, m.w));
-      }
+    for (int g = 0; g < 4; ++g) {
+      const int d0 = 32 * j + 8 * g + 4 * eh;
+      float4 m = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (!kCausal) m = *reinterpret_cast<const float4*>(vmean + d0);
+      store4<kOut>(p.output, out_row + d0, fmaf(num[j][4 * g + 0], rden, m.x), fmaf(num[j][4 * g + 1], rden, m.y),
+                   fmaf(num[j][4 * g + 2], rden, m.z), fmaf(num[j][4 * g + 3], rden, m.w));
     }
   }
 }
 
-template <int D, bool kCausal, int kOut, bool kPerThread>
+template <int D, bool kCausal, int kOut, bool kPerThread, bool kSplit = false>
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D))))
 attention_w3_kernel(const AttnParams p) {
   __shared__ __attribute__((aligned(16))) char smem[2 * TileLayout<D, 4>::kStageBytes];
-  int part = 0;
+  int part = -1;
   TileCoord tc;
-  if constexpr (kOut == kPartials) {
-    // logical id -> (batch-head, key part, query tile): the workgroups of one key range of a
-    // head are neighbours, so an XCD's workgroups stream the same tiles through its L2
-    const int logical = p.xcd_remap ? xcd_remap(blockIdx.x, gridDim.x) : static_cast<int>(blockIdx.x);
-    const int per_head = p.key_parts * p.query_tiles;
-    tc.bh = logical / per_head;
-    const int rem = logical - tc.bh * per_head;
-    part = rem / p.query_tiles;
-    tc.qtile = rem - part * p.query_tiles;
+  if constexpr (kSplit) {
+    // workgroups [0, whole_tiles): query tiles [0, whole_tiles), whole; then the parts of the other
+    // tiles, part by part, so that the workgroups an XCD runs stream one key range through its L2
+    const int block = static_cast<int>(blockIdx.x);
+    const int rest = static_cast<int>(gridDim.x) - p.whole_tiles;
+    int tile;
+    if (block < p.whole_tiles) {
+      tile = p.xcd_remap ? xcd_remap(block, p.whole_tiles) : block;
+    } else {
+      const int i = block - p.whole_tiles;
+      const int logical = p.xcd_remap ? xcd_remap(i, rest) : i;
+      const int split_tiles = p.query_tiles * p.batch_heads - p.whole_tiles;
+      part = logical / split_tiles;
+      tile = p.whole_tiles + logical - part * split_tiles;
+    }
+    tc.bh = tile / p.query_tiles;
+    tc.qtile = tile - tc.bh * p.query_tiles;
   } else {
     tc = workgroup_tile<kCausal>(p);
   }
-  // causal: the lane id read again for the epilogue (kept through the key loop, its half bit
-  // spills at 168 VGPRs)
-  w3_tile<D, kCausal, kOut, kPerThread, kCausal>(p, smem, tc, part, threadIdx.x & 63);
+  // causal and split: the lane id read again for the epilogue (kept through the key loop, its half
+  // bit spills)
+  w3_tile<D, kCausal, kOut, kPerThread, kCausal || kSplit, kSplit>(p, smem, tc, part, threadIdx.x & 63);
 }
 
 // The work-queue plan: a persistent grid (at most waves_per_simd(D) workgroups per CU) whose workgroups take
@@ -584,7 +595,6 @@ attention_w3_kernel(const AttnParams p) {
 template <int D, bool kCausal, int kOut, bool kPerThread>
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(waves_per_simd(D), waves_per_simd(D))))
 attention_w3_queue_kernel(const AttnParams p) {
-  static_assert(kOut != kPartials, "the work-queue plan has no key-range split");
   __shared__ __attribute__((aligned(16))) char smem[2 * TileLayout<D, 4>::kStageBytes];
   // The claim state lives in LDS (state[0]: the tile claimed, state[1]: the queue being taken
   // from).  Nothing of the claim may stay in registers across the tiles: at 168 VGPRs the key loop
@@ -668,12 +678,12 @@ __global__ void __launch_bounds__(64) queue_init_kernel(uint32_t* counters, int 
 // sequential pass, so split plans agree with the others to rounding, not bit for bit.
 template <int D, int kOut>
 __global__ void __launch_bounds__(256) attention_merge_kernel(const AttnParams p) {
-  const long rows = static_cast<long>(p.batch_heads) * p.query_length;
+  const long rows = split_rows(p);
   const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= rows * (D / 4)) return;
-  const long row = i / (D / 4);
+  const long row = i / (D / 4);  // among the split tiles' rows, which are consecutive
   const int d0 = static_cast<int>(i - row * (D / 4)) * 4;
-  const int bh = static_cast<int>(row / p.query_length);
+  const int bh = static_cast<int>((p.split_row0 + row) / p.query_length);
   const float2* stats = reinterpret_cast<const float2*>(p.partials + p.key_parts * rows * D);
   float top = -__builtin_inff();
   for (int q = 0; q < p.key_parts; ++q) top = fmaxf(top, stats[q * rows + row].y);
@@ -691,7 +701,7 @@ __global__ void __launch_bounds__(256) attention_merge_kernel(const AttnParams p
   }
   const float rden = (1.0f / 255.0f) / fmaxf(den, 1e-30f);
   const float4 m = *reinterpret_cast<const float4*>(p.value_mean + static_cast<long>(bh) * D + d0);
-  store4<kOut>(p.output, row * D + d0, fmaf(acc.x, rden, m.x), fmaf(acc.y, rden, m.y), fmaf(acc.z, rden, m.z),
+  store4<kOut>(p.output, (p.split_row0 + row) * D + d0, fmaf(acc.x, rden, m.x), fmaf(acc.y, rden, m.y), fmaf(acc.z, rden, m.z),
                fmaf(acc.w, rden, m.w));
 }
 
@@ -713,11 +723,16 @@ static hipError_t launch_w3(int out_dtype, const AttnParams& ap, hipStream_t str
   }
   if constexpr (!kCausal) {
     if (ap.key_parts > 1) {
-      const dim3 grid(static_cast<unsigned>(ap.query_tiles * ap.batch_heads * ap.key_parts));
-      hipLaunchKernelGGL((attention_w3_kernel<D, false, kPartials, kPerThread>), grid, block, 0, stream, ap);
+      const dim3 grid(static_cast<unsigned>(
+          ap.whole_tiles + (ap.query_tiles * ap.batch_heads - ap.whole_tiles) * ap.key_parts));
+      switch (out_dtype) {
+        case 0: hipLaunchKernelGGL((attention_w3_kernel<D, false, 0, kPerThread, true>), grid, block, 0, stream, ap); break;
+        case 1: hipLaunchKernelGGL((attention_w3_kernel<D, false, 1, kPerThread, true>), grid, block, 0, stream, ap); break;
+        default: hipLaunchKernelGGL((attention_w3_kernel<D, false, 2, kPerThread, true>), grid, block, 0, stream, ap); break;
+      }
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
-      const long threads = static_cast<long>(ap.batch_heads) * ap.query_length * (D / 4);
+      const long threads = split_rows(ap) * (D / 4);
       const dim3 merge_grid(static_cast<unsigned>((threads + 255) / 256));
       switch (out_dtype) {
         case 0: hipLaunchKernelGGL((attention_merge_kernel<D, 0>), merge_grid, block, 0, stream, ap); break;

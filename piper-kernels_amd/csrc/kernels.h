@@ -128,15 +128,6 @@ struct QuantParams {
   uint8_t* kv_tiles;  // [batch_heads][nkb][kv_tile_bytes(D)] (layout in piper_mi355x.h)
 };
 
-struct AttnParams {
-  const int8_t* query_code;
-  const float* query_scale;
-  const float* key_scale;
-  const uint8_t* kv_tiles;
-  const float* value_mean;
-  void* output;
-  int batch_heads;
-  int query_length;
 // Order of a causal longest-first grid whose plan leaves it open: across heads while all K/V tile
 // records fit the 256 MiB last-level cache, head by head beyond (then only a few heads' records are
 // live at a time).  Measured, head by head against across heads, Piper Attention at D = 128: B2 H16
@@ -149,6 +140,15 @@ inline bool order_across_heads(long batch_heads, long key_tiles, int tile_bytes)
   return batch_heads * key_tiles * tile_bytes <= kAcrossHeadsBytes;
 }
 
+struct AttnParams {
+  const int8_t* query_code;
+  const float* query_scale;
+  const float* key_scale;
+  const uint8_t* kv_tiles;
+  const float* value_mean;
+  void* output;
+  int batch_heads;
+  int query_length;
   int key_length;
   int sq32;
   int sk64;
@@ -168,13 +168,17 @@ inline bool order_across_heads(long batch_heads, long key_tiles, int tile_bytes)
   int query_bf16;
   int heads;
   InputTensor query;
-  // Key-range split (non-causal, three workgroups per CU): each query tile's key tiles are cut
-  // into key_parts ranges of part_tiles tiles, one workgroup per range, which writes its
-  // unnormalised numerator (x 255), denominator and reference maximum to `partials`
-  // ([key_parts][batch_heads][query_length][D] floats, then [key_parts][batch_heads][query_length]
-  // float2 (den, mref)); attention_merge_kernel combines them.  key_parts = 1: no split.
+  // Key-range split (non-causal, PIPER_PLAN_THREE_WORKGROUPS): query tiles [0, whole_tiles), whole
+  // rounds of resident workgroups, run unsplit; the key tiles of each later query tile are cut into
+  // key_parts ranges of part_tiles tiles, one workgroup per range, which writes its unnormalised
+  // numerator (x 255), denominator and reference maximum to `partials` ([key_parts][split rows][D]
+  // floats, then [key_parts][split rows] float2 (den, mref)); attention_merge_kernel combines them.
+  // The split rows are the output's rows from split_row0 on (rows of [batch_heads * query_length]).
+  // key_parts = 1: no split.
   int key_parts;
   int part_tiles;
+  int whole_tiles;
+  long split_row0;
   float* partials;
   // Work-queue plan (three workgroups per CU, no key-range split): a persistent grid takes query
   // tiles from queue_xccs queues of consecutive logical ids, counters in `queue` (zero before the
@@ -184,6 +188,10 @@ inline bool order_across_heads(long batch_heads, long key_tiles, int tile_bytes)
   float score_multiplier;  // scale_log2e * 2^26 (kScoreUnit), exact: the logits' multiplier per query scale
   uint32_t* queue;
 };
+
+__host__ __device__ inline long split_rows(const AttnParams& p) {
+  return static_cast<long>(p.batch_heads) * p.query_length - p.split_row0;
+}
 
 // The workspace bytes of a key-range split (0 without one).
 inline long attention_partial_bytes(long batch_heads, long query_length, int head_dim, int key_parts) {

@@ -181,49 +181,66 @@ def heuristic_plan(batch: int, heads: int, query_length: int) -> MI355XPlan:
     return MI355XPlan(waves=4)
 
 
-def split_parts(batch: int, heads: int, query_length: int, key_length: int) -> int:
-    """Key parts for an untuned non-causal shape (1: no split).  A grid whose 128-query tiles
-    fall short of one round of three workgroups per CU (768) and whose 256-query tiles leave CUs
-    idle splits into 2-4 parts, each of at least two key tiles (c1, 64 tiles: 4 parts, 0.017 vs
-    0.029 ms).  A long key range (>= 32768 keys,
-    where the partial sums' HBM round trip is small against the work) splits in the 2-4 parts
-    that fill the last round best, when that beats the unsplit grid's last round by 10% of a
-    round (B1 H1 N131072: 1024 tiles = 1.33 rounds; 3 parts = 4 full rounds, 7.14 vs 7.97 ms).
-    At 8192 keys the round trip costs more than the fuller round gains (r1: 3 parts 0.262 vs
-    0.254 ms), so mid-length grids stay whole."""
-    tiles = batch * heads * (-(-query_length // MI355XPlan(waves=4, three_per_cu=True).block_m))
+# Microseconds one 64-key tile takes a query wave when 1, 2, ... waves share its SIMD (measured on grids
+# of 1 to 3, at head size 64 to 4, workgroups per CU), the partial sums' round trip through memory in
+# bytes per microsecond, and the merge kernel's launch.
+_TILE_US = {128: (1.5, 1.75, 2.5), 64: (1.2, 1.4, 1.8, 2.3)}
+_PARTIAL_BYTES_PER_US = 4e6
+_MERGE_US = 2.2
+
+
+def _split_us(tiles: int, rows: int, key_tiles: int, parts: int, head_dim: int) -> float:
+    """Estimated time of a non-causal grid of `tiles` query tiles whose last, unfilled round of resident
+    workgroups (`rows` query rows) is split into `parts` key ranges (csrc/kernels.h AttnParams)."""
+    steps = _TILE_US[head_dim]
+    slots = len(steps) * COMPUTE_UNITS
+    whole, rest = divmod(tiles, slots)
+    part_rounds, part_rest = divmod(rest * parts, slots)
+    part_tiles = -(-key_tiles // parts)
+    us = (whole * key_tiles + part_rounds * part_tiles) * steps[-1]
+    if part_rest:
+        us += part_tiles * steps[-(-part_rest // COMPUTE_UNITS) - 1]
+    if parts > 1:
+        us += _MERGE_US + 2 * parts * rows * (head_dim + 2) * 4 / _PARTIAL_BYTES_PER_US
+    return us
+
+
+@lru_cache(maxsize=4096)
+def split_parts(batch: int, heads: int, query_length: int, key_length: int, head_dim: int = 128) -> int:
+    """Key parts for an untuned non-causal shape (1: no split): what ``_split_us`` finds fastest, if that
+    gains 5% of the whole grid's time.  Small grids split to give every SIMD more waves, larger ones
+    only the query tiles beyond whole rounds of resident workgroups.  Measured, unsplit against split: c1
+    (64 tiles of 16 key tiles) 22.4 -> 16.7 us in 4 parts; B1 H24 Sq256 Sk16384 (48 tiles of 256) 371 ->
+    74 us in 8 (105 in 4); B2 H12 Sq1000 Sk333 (192 tiles of 6) stays whole: 16.4 against 28.4 us in 2."""
+    block_m = MI355XPlan(waves=4, three_per_cu=True).block_m
+    tiles = batch * heads * (-(-query_length // block_m))
     key_tiles = -(-key_length // KEY_BLOCK)
-    round_slots = 3 * COMPUTE_UNITS
-    if tiles < round_slots and MI355XPlan(waves=8).workgroups(batch, heads, query_length) < COMPUTE_UNITS:
-        parts = min(4, max(2, round_slots // tiles), key_tiles // 2)
-        return parts if parts >= 2 else 1
-    if key_length >= 32768:
-        def fill(p: int) -> float:
-            rounds = tiles * p / round_slots
-            return rounds / -(-rounds // 1)
-        best = max((2, 3, 4), key=lambda p: (round(fill(p), 6), -p))
-        if fill(best) >= fill(1) + 0.1 and key_tiles >= 2 * best:
-            return best
-    return 1
+    rest = tiles % (len(_TILE_US[head_dim]) * COMPUTE_UNITS)
+    if rest == 0:
+        return 1
+    rows = min(rest * block_m, batch * heads * query_length)
+    us = {p: _split_us(tiles, rows, key_tiles, p, head_dim) for p in range(1, min(MAX_KEY_PARTS, max(1, key_tiles // 2)) + 1)}
+    best = min(us, key=us.get)
+    return best if us[best] <= 0.95 * us[1] else 1
 
 
 def piper_heuristic_plan(batch: int, heads: int, query_length: int, is_causal: bool,
-                         key_length: int | None = None) -> MI355XPlan:
+                         key_length: int | None = None, head_dim: int = 128) -> MI355XPlan:
     """Piper Attention's plan for an untuned shape: three 4-wave workgroups per CU.  With three
     waves per SIMD from three independent workgroups, one wave's MFMA, LDS and barrier waits are
     filled by the other two: measured 7-24% faster than the two-waves-per-SIMD plans at c2-c5.
-    Non-causal grids too small or too ragged for whole rounds of three workgroups per CU split
-    their key range (``split_parts``).  Otherwise a non-causal grid whose 128-query tiles cannot
-    fill three slots per CU, but whose 256-query tiles give every CU one, runs two waves per SIMD
-    either way; one 8-wave workgroup per CU is then 1-2% faster (measured at r1, B1 H8 N8192)."""
+    Non-causal grids too small or too ragged for whole rounds of resident workgroups split their key
+    range (``split_parts``).  Otherwise a non-causal grid of head size 128 whose 256-query tiles give
+    every CU exactly one runs two waves per SIMD either way; one 8-wave workgroup per CU is then 1-2%
+    faster (measured at r1, B1 H8 N8192; one 256-query tile more costs a round: B1 H10 N8192 474 us
+    against 320)."""
     three = MI355XPlan(waves=4, three_per_cu=True)
     wide = MI355XPlan(waves=8)
     if not is_causal:
-        parts = split_parts(batch, heads, query_length, query_length if key_length is None else key_length)
+        parts = split_parts(batch, heads, query_length, query_length if key_length is None else key_length, head_dim)
         if parts > 1:
             return MI355XPlan(waves=4, three_per_cu=True, key_parts=parts)
-        if (three.workgroups(batch, heads, query_length) < 3 * COMPUTE_UNITS
-                and wide.workgroups(batch, heads, query_length) >= COMPUTE_UNITS):
+        if head_dim == 128 and wide.workgroups(batch, heads, query_length) == COMPUTE_UNITS:
             return wide
     return three
 
@@ -239,7 +256,8 @@ def sage_plan(batch: int, heads: int, query_length: int) -> MI355XPlan:
 def select_plan(batch: int, heads: int, query_length: int, key_length: int, head_dim: int, is_causal: bool) -> MI355XPlan:
     """The frozen table's plan for a tuned shape, else Piper Attention's heuristic."""
     plan = frozen_plans().get(shape_key(batch, heads, query_length, key_length, head_dim, is_causal))
-    return plan if plan is not None else piper_heuristic_plan(batch, heads, query_length, is_causal, key_length)
+    return plan if plan is not None else piper_heuristic_plan(
+        batch, heads, query_length, is_causal, key_length, head_dim)
 
 
 def select_sage_plan(batch: int, heads: int, query_length: int, key_length: int, head_dim: int,
