@@ -492,7 +492,7 @@ int piper_sage_prepare(const piper_sage_prepare_args* a, void* stream) {
   mp.value_absmax = 1;
   mp.value_scale = o.value_scale;
 
-  piper::SageQuantParams qp{};
+  piper::QuantParams qp{};
   qp.key = to_input(a->key);
   qp.value = to_input(a->value);
   qp.batch_heads = bh;
@@ -502,13 +502,17 @@ int piper_sage_prepare(const piper_sage_prepare_args* a, void* stream) {
   qp.k_blocks_wg = static_cast<int>(ceil_div(static_cast<int64_t>(bh) * nkb, 4));
   qp.v_blocks_wg = qp.k_blocks_wg;
   qp.key_mean = o.key_mean;
-  qp.value_scale = o.value_scale;
   qp.key_scale = o.key_scale;
   qp.kv_tiles = static_cast<uint8_t*>(o.kv_tiles);
   qp.per_thread = (a->flags & PIPER_PREPARE_QK_PER_THREAD) ? 1 : 0;
 
+  piper::PrepDevice dev{};
+  if (int st = device_topology(&dev.cus, &dev.xccs)) return st;
+  dev.spin_limit = piper::kPrepSpinLimit;
+
   const hipError_t err =
-      piper::launch_sage_prep(a->dtype == PIPER_BFLOAT16, static_cast<int>(s.head_dim), mp, qp, static_cast<hipStream_t>(stream));
+      piper::launch_sage_prep(a->dtype == PIPER_BFLOAT16, static_cast<int>(s.head_dim), mp, qp, dev,
+                              static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(PIPER_ERROR_HIP, "prep launch failed: %s", hipGetErrorString(err));
   g_last_error[0] = '\0';
   return PIPER_OK;

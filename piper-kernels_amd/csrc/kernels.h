@@ -102,6 +102,8 @@ struct MeanParams {
 constexpr int kQueryScaleSlots = 8;
 constexpr int kKeyScaleSlots = 4;
 
+// Both operators' prep quantisation.  SageAttention2++ has no query blocks and no value means: it
+// quantises K (per 64-row block, after K smoothing) and V (FP8 per channel) into its own tile records.
 struct QuantParams {
   InputTensor query;
   InputTensor key;
@@ -124,8 +126,8 @@ struct QuantParams {
   int8_t* query_code;
   float* query_scale;
   float* key_scale;
-  float* value_scale;
-  uint8_t* kv_tiles;  // [batch_heads][nkb][kv_tile_bytes(D)] (layout in piper_mi355x.h)
+  float* value_scale;  // Piper Attention's per-key scales (SageAttention2++'s per channel: MeanParams)
+  uint8_t* kv_tiles;  // [batch_heads][nkb][kv_tile_bytes(D) or sage_tile_bytes(D)] (layout in piper_mi355x.h)
 };
 
 // Order of a causal longest-first grid whose plan leaves it open: across heads while all K/V tile
@@ -202,24 +204,6 @@ inline long attention_partial_bytes(long batch_heads, long query_length, int hea
 constexpr int kQueueCounters = 64;
 constexpr long kQueueBytes = kQueueCounters * 4;
 
-// SageAttention2++: the prep quantises K (per 64-row block, after K smoothing) and V (FP8
-// per channel) into tile records; the attention kernel quantises each query block itself.
-struct SageQuantParams {
-  InputTensor key;
-  InputTensor value;
-  int batch_heads;
-  int heads;
-  int key_length;
-  int nkb;
-  int k_blocks_wg;  // workgroups (4 units each) per unit kind
-  int v_blocks_wg;
-  const float* key_mean;
-  const float* value_scale;
-  float* key_scale;   // [batch_heads][nkb][kKeyScaleSlots]
-  uint8_t* kv_tiles;  // [batch_heads][nkb][sage_tile_bytes(D)]
-  int per_thread;     // 1: K scales per thread group; 0: one per block, repeated in every slot
-};
-
 struct SageParams {
   const uint8_t* kv_tiles;
   const float* value_scale;  // [batch_heads][D]
@@ -258,7 +242,7 @@ __host__ __device__ inline bool single_pass_resident(int chunks, int cus, int xc
 
 hipError_t launch_prep(bool bf16, int head_dim, const MeanParams& mp, const QuantParams& qp, const PrepDevice& dev,
                        hipStream_t stream);
-hipError_t launch_sage_prep(bool bf16, int head_dim, const MeanParams& mp, const SageQuantParams& qp,
+hipError_t launch_sage_prep(bool bf16, int head_dim, const MeanParams& mp, const QuantParams& qp, const PrepDevice& dev,
                             hipStream_t stream);
 hipError_t launch_sage_attention(int head_dim, bool causal, int out_dtype, int waves, const SageParams& sp,
                                  hipStream_t stream);

@@ -16,6 +16,25 @@
 
 namespace piper {
 
+// Which path a call takes (launch_prep_typed has the rule):
+//   short      one kernel, every workgroup computes the sequence statistics it needs itself
+//   two-pass   partial sums, then quantisation whose waves finish the statistics
+//   single     K and V read from memory once, the chunks of a sequence waiting for their statistics
+//   three-pass as two-pass with a kernel of its own for the finish (very long sequences)
+
+// K and V bytes up to which the two-pass prep, which reads them twice (the second time from the last-level
+// cache), beats the single pass, whose chunks wait for one another.  At D = 64 a chunk in flight is half
+// as large and the waits weigh more: B2 H24 S8192 (100 MB) 50.8 us against 54.7, B4 H24 S8192 (200 MB)
+// 106.6 against 103.8 (causal 104.8 against 89.3).  At D = 128 the two tie up to 50 MB (B1 H24 S2048 and
+// S4096) and the single pass wins from there: B2 H24 S4096 (100 MB) 45.3 us against 50.9,
+// SageAttention2++ 40.7 against 48.6.
+constexpr long two_pass_bytes(int head_dim) { return (head_dim == 64 ? 128L : 32L) << 20; }
+
+template <int D, bool kSage>
+constexpr int record_bytes() {
+  return kSage ? sage_tile_bytes(D) : kv_tile_bytes(D);
+}
+
 // ---------------------------------------------------------------------------------------
 // Means, pass 1: one workgroup per chunk of L^2 rows of K (tensor 0) or V (tensor 1) of one
 // batch-head.  Thread (slot, column group) sums L-row blocks slot, slot + kSlots, ... of eight
@@ -110,12 +129,14 @@ __global__ void __launch_bounds__(256) mean_partial_kernel(const MeanParams p) {
 }
 
 
+// SageAttention2++'s V scale of a channel (sage_attention_2pp/reference.py:22-23: FP32 division and add).
+__device__ __forceinline__ float channel_scale(float amax) { return __fadd_rn(amax / 2.25f, 1e-7f); }
+
 // Means, pass 2, one thread per (tensor, batch-head, column): the complete chunks' level-1 sums
 // are added in groups of L (level 2), the group sums in order (level 3); then
 // ((trailing rows + short chunk's blocks) + unfinished level 2) + level 3, divided by the length
 // in FP32.  Causal calls write a zero V mean.  SageAttention2++ (value_absmax): the V column's
-// max |v| over the chunks gives its FP8 scale amax / 2.25 + 1e-7
-// (sage_attention_2pp/reference.py:22-23: FP32 division, FP32 add).
+// max |v| over the chunks gives its FP8 scale.
 __device__ __forceinline__ void finalize_column(const MeanParams& p, int tensor, int bh, int d, int head_dim) {
   const int rem = bh * head_dim + d;
   float* dst = tensor == 0 ? p.key_mean : p.value_mean;
@@ -128,7 +149,7 @@ __device__ __forceinline__ void finalize_column(const MeanParams& p, int tensor,
   if (tensor == 1 && p.value_absmax) {
     float amax = 0.0f;
     for (int c = 0; c <= p.chunks; ++c) amax = fmaxf(amax, src[static_cast<long>(c) * head_dim]);
-    p.value_scale[rem] = __fadd_rn(amax / 2.25f, 1e-7f);
+    p.value_scale[rem] = channel_scale(amax);
     return;
   }
   const int block = p.block_rows;
@@ -170,6 +191,62 @@ __global__ void __launch_bounds__(64) mean_finalize_kernel(const MeanParams p, i
   const int tensor = gid / per_tensor;
   const int rem = gid - tensor * per_tensor;
   finalize_column(p, tensor, rem / head_dim, rem % head_dim, head_dim);
+}
+
+// Means, pass 2, by the waves of the quantisation itself (two-pass prep, at most kWaveChunks chunks of
+// 16-row blocks): the wave that owns a unit finishes its batch-head's statistics in registers, lane l
+// the columns [l D / 64, +D / 64), every partial loaded before the first addition, into `out` (this
+// wave's D floats of LDS).  The same order of additions as finalize_column.  A kernel of its own for this
+// took 4.6-11 us (B2 H20 S4096 D64, B4 H32 S8192 D128) and a launch on a chain of three.
+constexpr int kWaveChunks = 32;  // 8192 keys: the partials a wave reads stay below its unit's rows
+
+template <int D, bool kAbsMax>
+__device__ __forceinline__ void wave_statistics(const MeanParams& p, int tensor, int bh, int lane, float* out) {
+  constexpr int kCols = D / 64;
+  typedef float cols_t __attribute__((ext_vector_type(kCols)));
+  constexpr int L = 16;
+  const float* src =
+      p.partials + (static_cast<long>(tensor) * p.batch_heads + bh) * (p.chunks + 1) * D + lane * kCols;
+  const auto at = [&](int c) { return *reinterpret_cast<const cols_t*>(src + static_cast<long>(c) * D); };
+  cols_t result;
+  if constexpr (kAbsMax) {
+    cols_t amax = 0.0f;
+    for (int c0 = 0; c0 <= p.chunks; c0 += L) {
+      cols_t part[L];
+#pragma unroll
+      for (int i = 0; i < L; ++i) part[i] = c0 + i <= p.chunks ? at(c0 + i) : cols_t(0.0f);
+#pragma unroll
+      for (int i = 0; i < L; ++i)
+#pragma unroll
+        for (int k = 0; k < kCols; ++k) amax[k] = fmaxf(amax[k], part[i][k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kCols; ++k) result[k] = channel_scale(amax[k]);
+  } else {
+    const int full = p.length / (L * L);  // complete chunks
+    const cols_t level0 = at(p.chunks);
+    const cols_t level1 = full < p.chunks ? at(full) : cols_t(0.0f);
+    cols_t level2 = 0.0f, level3 = 0.0f;
+    for (int c0 = 0; c0 < full; c0 += L) {
+      cols_t part[L];
+#pragma unroll
+      for (int i = 0; i < L; ++i) part[i] = c0 + i < full ? at(c0 + i) : cols_t(0.0f);
+      level2 = 0.0f;
+#pragma unroll
+      for (int i = 0; i < L; ++i)
+        if (c0 + i < full) level2 += part[i];
+      if (c0 + L <= full) {
+        level3 += level2;
+        level2 = 0.0f;
+      }
+    }
+    const cols_t total = ((level0 + level1) + level2) + level3;
+#pragma unroll
+    for (int k = 0; k < kCols; ++k) result[k] = total[k] / static_cast<float>(p.length);
+  }
+  *reinterpret_cast<cols_t*>(out + lane * kCols) = result;
+  // the wave's own reads follow its writes in order; the compiler must keep them so
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
 // ---------------------------------------------------------------------------------------
@@ -332,27 +409,6 @@ __device__ __forceinline__ void load_unit_rows(const InputTensor& in, int b, int
   }
 }
 
-template <bool kBf16, int D, bool kGuard>
-__device__ __forceinline__ void quantize_value_rows(const QuantParams& p, int unit, int lane,
-                                                    uint4 (&raw)[kKeyBlock / (kWave / (D / 8))],
-                                                    const float (&mu)[8]);
-
-template <bool kBf16, int D, bool kGuard>
-__device__ __forceinline__ void quantize_value_tile(const QuantParams& p, int unit, int lane) {
-  constexpr int kGroups = D / 8;
-  const int bh = unit / p.nkb;
-  const int kb = unit - bh * p.nkb;
-  const int b = bh / p.heads;
-  const int h = bh - b * p.heads;
-  const int group = lane % kGroups;
-  uint4 raw[kKeyBlock / (kWave / kGroups)];
-  load_unit_rows<D, kGuard>(p.value, b, h, kb, p.key_length, lane, raw);
-  float mu[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) mu[i] = p.center_value ? p.value_mean[static_cast<long>(bh) * D + group * 8 + i] : 0.0f;
-  quantize_value_rows<kBf16, D, kGuard>(p, unit, lane, raw, mu);
-}
-
 // The V tile `unit` from lane (group, sub)'s rows `raw` (load_unit_rows) centred by `mu` (its
 // eight columns' means, zeros when uncentred).
 template <bool kBf16, int D, bool kGuard>
@@ -447,14 +503,13 @@ __device__ __forceinline__ void quantize_query_unit(const QuantParams& p, int un
         p.query, b, h, qb * kQueryBlock, p.query_length, nullptr, codes, scales, p.per_thread);
 }
 
-template <bool kBf16, int D>
-__device__ __forceinline__ void quantize_key_unit(const QuantParams& p, int unit) {  // one 64-row K block
+template <bool kBf16, int D, bool kSage>
+__device__ __forceinline__ void quantize_key_unit(const QuantParams& p, int unit, const float* mean) {  // one 64-row K block
   const int bh = unit / p.nkb;
   const int kb = unit - bh * p.nkb;
   const int b = bh / p.heads;
   const int h = bh - b * p.heads;
-  int8_t* tile = reinterpret_cast<int8_t*>(p.kv_tiles) + static_cast<long>(unit) * kv_tile_bytes(D);
-  const float* mean = p.key_mean + static_cast<long>(bh) * D;
+  int8_t* tile = reinterpret_cast<int8_t*>(p.kv_tiles) + static_cast<long>(unit) * record_bytes<D, kSage>();
   float* scales = p.key_scale + static_cast<long>(unit) * kKeyScaleSlots;
   if ((kb + 1) * kKeyBlock <= p.key_length)
     quantize_block<kBf16, D, kKeyBlock, true, kv_k_stride(D), kKeyScaleSlots, false>(
@@ -464,44 +519,150 @@ __device__ __forceinline__ void quantize_key_unit(const QuantParams& p, int unit
         p.key, b, h, kb * kKeyBlock, p.key_length, mean, tile, scales, p.per_thread);
 }
 
+// SageAttention2++'s V tile `unit` from lane (group, sub)'s rows `raw` (load_unit_rows; rows past the end
+// are zero and get code 0) and its eight channels' scales: FP8 E4M3 codes of v / scale (the correctly
+// rounded FP32 quotient, then v_cvt_pk_fp8_f32: round to nearest even, bit-identical to torch's
+// float8_e4m3fn cast; sage_attention_2pp/reference.py:22-25, 44-49), four keys of a column packed per
+// word: the 16-byte (D = 128) or 8-byte (D = 64) pieces of the lane's eight V^T rows.
 template <bool kBf16, int D>
-__device__ __forceinline__ void quantize_value_unit(const QuantParams& p, int unit, int lane) {  // one 64-key V tile
-  if ((unit % p.nkb + 1) * kKeyBlock <= p.key_length)
-    quantize_value_tile<kBf16, D, false>(p, unit, lane);
-  else
-    quantize_value_tile<kBf16, D, true>(p, unit, lane);
+__device__ __forceinline__ void quantize_channel_rows(const QuantParams& p, int unit, int lane,
+                                                      const uint4 (&raw)[kKeyBlock / (kWave / (D / 8))],
+                                                      const float (&scale)[8]) {
+  constexpr int kGroups = D / 8;
+  constexpr int kKeys = kKeyBlock / (kWave / kGroups);
+  const int group = lane % kGroups;
+  const int key0 = (lane / kGroups) * kKeys;
+  Divisor divisor[8];  // this lane's 8 channels
+#pragma unroll
+  for (int i = 0; i < 8; ++i) divisor[i] = Divisor(scale[i]);
+  uint32_t packed[8][kKeys / 4];  // [column][four keys]
+#pragma unroll
+  for (int j4 = 0; j4 < kKeys / 4; ++j4) {
+    float q[4][8];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float f[8];
+      widen8<kBf16>(raw[4 * j4 + u], f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) q[u][i] = divisor[i].quotient(f[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0][i], q[1][i], 0, false);
+      packed[i][j4] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(q[2][i], q[3][i], lo, true));
+    }
+  }
+  uint8_t* tile = p.kv_tiles + static_cast<long>(unit) * sage_tile_bytes(D);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    uint8_t* dst = tile + sage_v_offset(D) + (group * 8 + i) * kv_v_stride() + key0;
+    if constexpr (kKeys == 16)
+      *reinterpret_cast<uint4*>(dst) = make_uint4(packed[i][0], packed[i][1], packed[i][2], packed[i][3]);
+    else
+      *reinterpret_cast<uint2*>(dst) = make_uint2(packed[i][0], packed[i][1]);
+  }
 }
+
+// A V tile's codes from its rows and the statistic of the lane's eight columns: the means that centre
+// them (zeros when uncentred) or, SageAttention2++, the channel scales.
+template <bool kBf16, int D, bool kSage, bool kGuard>
+__device__ __forceinline__ void quantize_value_codes(const QuantParams& p, int unit, int lane,
+                                                     uint4 (&raw)[kKeyBlock / (kWave / (D / 8))],
+                                                     const float (&stat)[8]) {
+  if constexpr (kSage) quantize_channel_rows<kBf16, D>(p, unit, lane, raw, stat);
+  else quantize_value_rows<kBf16, D, kGuard>(p, unit, lane, raw, stat);
+}
+
+// One 64-key V tile; `stat`: the batch-head's D column statistics (NULL: uncentred).
+template <bool kBf16, int D, bool kSage, bool kGuard>
+__device__ __forceinline__ void quantize_value_tile(const QuantParams& p, int unit, int lane, const float* stat) {
+  constexpr int kGroups = D / 8;
+  const int bh = unit / p.nkb;
+  const int kb = unit - bh * p.nkb;
+  const int b = bh / p.heads;
+  const int h = bh - b * p.heads;
+  uint4 raw[kKeyBlock / (kWave / kGroups)];
+  load_unit_rows<D, kGuard>(p.value, b, h, kb, p.key_length, lane, raw);
+  float mu[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) mu[i] = stat != nullptr ? stat[(lane % kGroups) * 8 + i] : 0.0f;
+  quantize_value_codes<kBf16, D, kSage, kGuard>(p, unit, lane, raw, mu);
+}
+
+template <bool kBf16, int D, bool kSage>
+__device__ __forceinline__ void quantize_value_unit(const QuantParams& p, int unit, int lane, const float* stat) {
+  if ((unit % p.nkb + 1) * kKeyBlock <= p.key_length)
+    quantize_value_tile<kBf16, D, kSage, false>(p, unit, lane, stat);
+  else
+    quantize_value_tile<kBf16, D, kSage, true>(p, unit, lane, stat);
+}
+
+struct PrepParams {
+  QuantParams q;
+  MeanParams m;
+};
 
 // One wave per unit, four units of one kind per workgroup: Q blocks (two-step path), K blocks,
 // V tiles.  Four waves per SIMD (at most 128 VGPRs) overlap one another's loads with their
 // arithmetic.  Causal calls take the K blocks last-read-first: the mean pass has just read K (and
-// only K), so the most recently read rows are still in the last-level cache.
-template <bool kBf16, int D>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) quantize_kernel(const QuantParams p) {
-  const int wave = threadIdx.x >> 6;
+// only K), so the most recently read rows are still in the last-level cache.  kFinish: the partials are
+// not finished yet, each wave finishes its batch-head's (wave_statistics) and the first unit's wave of
+// each batch-head writes them out; otherwise mean_finalize_kernel has.
+template <bool kBf16, int D, bool kSage, bool kFinish>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) quantize_kernel(const PrepParams a) {
+  __shared__ __attribute__((aligned(16))) float statistics[4][D];
+  const QuantParams& p = a.q;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   int block = blockIdx.x;
-  if (block < p.q_blocks_wg) {
-    const int unit = block * 4 + wave;
-    if (unit < p.batch_heads * p.nqb) quantize_query_unit<kBf16, D>(p, unit);
-    return;
+  if (kFinish && !kSage && block == 0 && threadIdx.x == 0) *a.m.status = 0u;  // this path never waits
+  if constexpr (!kSage) {
+    if (block < p.q_blocks_wg) {
+      const int unit = block * 4 + wave;
+      if (unit < p.batch_heads * p.nqb) quantize_query_unit<kBf16, D>(p, unit);
+      return;
+    }
+    block -= p.q_blocks_wg;
   }
-  block -= p.q_blocks_wg;
   if (block < p.k_blocks_wg) {
-    const int unit = (p.center_value ? block : p.k_blocks_wg - 1 - block) * 4 + wave;
-    if (unit < p.batch_heads * p.nkb) quantize_key_unit<kBf16, D>(p, unit);
+    const int unit = (kSage || p.center_value ? block : p.k_blocks_wg - 1 - block) * 4 + wave;
+    if (unit >= p.batch_heads * p.nkb) return;
+    const int bh = unit / p.nkb;
+    const float* mean = p.key_mean + static_cast<long>(bh) * D;
+    if constexpr (kFinish) {
+      wave_statistics<D, false>(a.m, 0, bh, lane, statistics[wave]);
+      if (unit == bh * p.nkb)
+        for (int col = lane; col < D; col += 64) a.m.key_mean[static_cast<long>(bh) * D + col] = statistics[wave][col];
+      mean = statistics[wave];
+    }
+    quantize_key_unit<kBf16, D, kSage>(p, unit, mean);
     return;
   }
   const int unit = (block - p.k_blocks_wg) * 4 + wave;
-  if (unit < p.batch_heads * p.nkb) quantize_value_unit<kBf16, D>(p, unit, lane);
+  if (unit >= p.batch_heads * p.nkb) return;
+  const int bh = unit / p.nkb;
+  const bool used = kSage || p.center_value;
+  float* out = (kSage ? a.m.value_scale : a.m.value_mean) + static_cast<long>(bh) * D;
+  const float* stat = used ? out : nullptr;
+  if constexpr (kFinish) {
+    if (used) {
+      wave_statistics<D, kSage>(a.m, 1, bh, lane, statistics[wave]);
+      stat = statistics[wave];
+    }
+    if (unit == bh * p.nkb)
+      for (int col = lane; col < D; col += 64) out[col] = used ? statistics[wave][col] : 0.0f;
+  }
+  quantize_value_unit<kBf16, D, kSage>(p, unit, lane, stat);
 }
 
 // ---------------------------------------------------------------------------------------
-// Single-pass prep (D = 128, cascade blocks of L = 16 rows, at most kSinglePassChunks chunks per
+// Single-pass prep (cascade blocks of L = 16 rows, at most kSinglePassChunks chunks per
 // sequence): K and V are read from HBM once.  One workgroup per 256-row chunk of one batch-head's
 // K or V: wave w holds rows [64 w, +64) of the chunk (the chunk's K block or V tile 4 c + w) in
-// registers, lane (group, sub) the columns [8 group, +8) of rows [16 sub, +16) -- exactly one
-// cascade level-0 block, which it sums in row order.  The chunk's level-1 sums are published
+// registers, lane (group, sub) the columns [8 group, +8) of rows [16 sub, +16) (D = 128: exactly one
+// cascade level-0 block, which it sums in row order) or [8 sub, +8) (D = 64: half a block, the odd
+// lane goes on from the even lane's sum).  The chunk's level-1 sums (SageAttention2++'s V: its column
+// maxima of |v|) are published
 // (write-through stores) and counted on the batch-head tensor's arrival counter; the chunk that
 // arrives last computes the mean (levels 2 and 3, the torch order of the mean pass above) and
 // writes it over the pending marks the launch left in the mean buffer; the other chunks poll
@@ -528,21 +689,22 @@ __device__ __forceinline__ void store_coherent(float* p, float v) {  // agent-sc
                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// K block from registers (load_unit_rows at D = 128): centred by `mu`, per-thread-group scales
-// (group of row r: (r % 8) / 2, i.e. (j % 8) / 2 for this lane's row 16 sub + j) or one per
+// K block from registers (load_unit_rows): centred by `mu`, per-thread-group scales
+// (group of row r: (r % 8) / 2, i.e. (j % 8) / 2 for this lane's row kKeys sub + j) or one per
 // block, codes into the tile's K rows, scales to scale_out and to the padding of K row 0 --
 // the same values as quantize_block, which takes the rows in another lane order.
-template <bool kBf16, bool kGuard>
-__device__ __forceinline__ void quantize_key_rows(uint4 (&raw)[16], const float (&mu)[8], int valid_rows,
-                                                  int8_t* __restrict__ tile, float* __restrict__ scale_out,
-                                                  bool per_thread, int lane) {
-  constexpr int D = 128;
+template <bool kBf16, int D, bool kGuard>
+__device__ __forceinline__ void quantize_key_rows(uint4 (&raw)[kKeyBlock / (kWave / (D / 8))], const float (&mu)[8],
+                                                  int valid_rows, int8_t* __restrict__ tile,
+                                                  float* __restrict__ scale_out, bool per_thread, int lane) {
+  constexpr int kGroups = D / 8;
+  constexpr int kKeys = kKeyBlock / (kWave / kGroups);
   constexpr int kStride = kv_k_stride(D);
-  const int group = lane & 15;
-  const int sub = lane >> 4;
+  const int group = lane % kGroups;
+  const int sub = lane / kGroups;
   float am[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
+  for (int j = 0; j < kKeys; ++j) {
     float f[8];
     widen8<kBf16>(raw[j], f);
 #pragma unroll
@@ -562,9 +724,9 @@ __device__ __forceinline__ void quantize_key_rows(uint4 (&raw)[16], const float 
   const Divisor divisor[4] = {Divisor(scale[0]), Divisor(scale[1]), Divisor(scale[2]), Divisor(scale[3])};
   // widen and centre again from the packed rows (as quantize_block: keeps 128 floats out of VGPRs)
 #pragma unroll
-  for (int j = 0; j < 16; ++j) asm volatile("" : "+v"(raw[j].x), "+v"(raw[j].y), "+v"(raw[j].z), "+v"(raw[j].w));
+  for (int j = 0; j < kKeys; ++j) asm volatile("" : "+v"(raw[j].x), "+v"(raw[j].y), "+v"(raw[j].z), "+v"(raw[j].w));
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
+  for (int j = 0; j < kKeys; ++j) {
     float f[8];
     widen8<kBf16>(raw[j], f);
     uint32_t c[8];
@@ -573,7 +735,7 @@ __device__ __forceinline__ void quantize_key_rows(uint4 (&raw)[16], const float 
       const float x = !kGuard || j < valid_rows ? f[i] - mu[i] : 0.0f;
       c[i] = code_word(x, divisor[(j & 7) >> 1]);
     }
-    *reinterpret_cast<uint2*>(tile + (16 * sub + j) * kStride + 8 * group) =
+    *reinterpret_cast<uint2*>(tile + (kKeys * sub + j) * kStride + 8 * group) =
         make_uint2(pack_low_bytes(c[0], c[1], c[2], c[3]), pack_low_bytes(c[4], c[5], c[6], c[7]));
   }
   if (lane == 0) {
@@ -586,8 +748,9 @@ __device__ __forceinline__ void quantize_key_rows(uint4 (&raw)[16], const float 
 struct SinglePassParams {
   QuantParams q;
   MeanParams m;
-  uint32_t* arrivals;  // [batch_heads][2] chunks arrived (zero before the launch)
-  uint32_t* status;    // chunks whose wait gave up and computed the mean themselves (zero before the launch)
+  uint32_t* arrivals;  // chunks arrived of batch-head bh's tensor t, at [bh * arrival_stride + t] (zero before the launch)
+  long arrival_stride;
+  uint32_t* status;    // (Piper Attention) chunks whose wait gave up and computed the mean themselves (zero before the launch)
   int kv_workgroups;   // batch_heads * 2 * chunks; Q-block workgroups (4 blocks each) follow
   int xccs;            // XCCs the workgroups are dealt over (the remap's stride)
   int spin_limit;      // polls before a wait gives up (0: no wait, every waiter computes the mean)
@@ -614,6 +777,18 @@ __device__ float block_rows_sum(const uint16_t* rows, long stride, int n) {
   for (int r = 0; r < 16; ++r)
     if (r < n) acc += v[r];
   return acc;
+}
+
+// SageAttention2++'s V scale of column `col` straight from its rows.
+template <bool kBf16>
+__device__ float column_scale_from_rows(const InputTensor& in, int b, int h, int col, int length) {
+  const uint16_t* base = static_cast<const uint16_t*>(in.data) + b * in.stride_batch + h * in.stride_head + col;
+  float amax = 0.0f;
+  for (int r = 0; r < length; ++r) {
+    const uint32_t bits = base[static_cast<long>(r) * in.stride_seq];
+    amax = fmaxf(amax, fabsf(kBf16 ? __uint_as_float(bits << 16) : half_bits_to_float(bits)));
+  }
+  return channel_scale(amax);
 }
 
 template <bool kBf16>
@@ -648,394 +823,473 @@ __device__ float column_mean_from_rows(const InputTensor& in, int b, int h, int 
 }
 constexpr uint32_t kMeanPending = 0x7fa5a5a5u;  // a signalling NaN: the mean slot before it is published
 
-// The mean of one column from the published partials, torch's cascade order (finalize_column),
-// with two threads per column: thread `half` sums the level-2 groups half, half + 2, ... of L
-// chunks each (one group's loads in flight together, the groups one after another to keep the
-// chunk's rows in registers), the groups meet in LDS and thread 0 of the pair combines them in
-// order.
-__device__ __forceinline__ float single_pass_mean(const MeanParams& p, const float* src, int col, int half,
-                                                  float (*group_sums)[128]) {
+// The statistic of one column from the published partials: the mean in torch's cascade order
+// (finalize_column) or the channel scale, with kParts = 256 / D threads per column.  Thread `part` sums
+// the level-2 groups part, part + kParts, ... of L chunks each (one group's loads in flight together,
+// the groups one after another to keep the chunk's rows in registers), the groups meet in LDS and
+// thread 0 of the column combines them in order.
+template <int D, bool kAbsMax>
+__device__ __forceinline__ float single_pass_statistic(const MeanParams& p, const float* src, int col, int part,
+                                                       float (*group_sums)[D]) {
   constexpr int L = 16;
-  const int full = p.length / (L * L);  // complete chunks
+  constexpr int kParts = 256 / D;
+  const int full = kAbsMax ? p.chunks : p.length / (L * L);  // complete chunks (a maximum takes every chunk alike)
   const int groups = (full + L - 1) / L;  // level-2 groups (the last may be unfinished)
 #pragma unroll 1
-  for (int g = half; g < groups; g += 2) {
+  for (int g = part; g < groups; g += kParts) {
     const int c0 = g * L;
     const int n = min(L, full - c0);
-    float part[L];
+    float value[L];
 #pragma unroll
-    for (int i = 0; i < L; ++i) part[i] = i < n ? load_coherent(src + static_cast<long>(c0 + i) * 128) : 0.0f;
+    for (int i = 0; i < L; ++i) value[i] = i < n ? load_coherent(src + static_cast<long>(c0 + i) * D) : 0.0f;
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < L; ++i)
-      if (i < n) s += part[i];
+      if (i < n) s = kAbsMax ? fmaxf(s, value[i]) : s + value[i];
     group_sums[g][col] = s;
   }
   __syncthreads();
-  if (half != 0) return 0.0f;
+  if (part != 0) return 0.0f;
+  if constexpr (kAbsMax) {
+    float amax = 0.0f;
+    for (int g = 0; g < groups; ++g) amax = fmaxf(amax, group_sums[g][col]);
+    return channel_scale(amax);
+  }
   float level3 = 0.0f, level2 = 0.0f;
   for (int g = 0; g < groups; ++g) {
     if ((g + 1) * L <= full) level3 += group_sums[g][col];
     else level2 = group_sums[g][col];
   }
-  const float level1 = full < p.chunks ? load_coherent(src + static_cast<long>(full) * 128) : 0.0f;
-  const float level0 = load_coherent(src + static_cast<long>(p.chunks) * 128);
+  const float level1 = full < p.chunks ? load_coherent(src + static_cast<long>(full) * D) : 0.0f;
+  const float level0 = load_coherent(src + static_cast<long>(p.chunks) * D);
   const float total = ((level0 + level1) + level2) + level3;
   return total / static_cast<float>(p.length);
 }
 
 // LDS of a single-pass workgroup.
+template <int D>
 struct SinglePassShared {
-  float block_sums[16][128];  // the chunk's level-0 sums
-  float group_sums[kSinglePassChunks / 16][128];
-  float mean[128];
+  float block_sums[2048 / D][D];  // the chunk's level-0 sums (16 used) or one row of maxima per (wave, sub)
+  float group_sums[kSinglePassChunks / 16][D];
+  float statistic[D];
   int last;
 };
 
-// One chunk of tensor kTensor (0: K, 1: V) of batch-head bh: load, cascade sums, mean, codes.
-// The whole pipeline is inlined once per tensor so that each keeps its 64 VGPRs of rows in
-// registers without the other's code in between; a unit that reaches past the end of the
-// sequence (at most one per batch-head) loads its rows again, guarded, inside its own branch.
-template <bool kBf16, int kTensor>
-__device__ __forceinline__ void single_pass_chunk(const SinglePassParams& p, SinglePassShared& sh, int bh, int chunk,
+// The codes of this wave's unit of tensor kTensor from its rows in registers and its columns' statistic;
+// a unit that reaches past the end of the sequence (at most one per batch-head) loads its rows again,
+// guarded, inside its own branch.
+template <bool kBf16, int D, bool kSage, int kTensor>
+__device__ __forceinline__ void quantize_unit_rows(const QuantParams& p, int bh, int kb, int lane, bool full_unit,
+                                                   uint4 (&raw)[kKeyBlock / (kWave / (D / 8))], const float (&stat)[8]) {
+  constexpr int kKeys = kKeyBlock / (kWave / (D / 8));
+  const int b = bh / p.heads;
+  const int h = bh - b * p.heads;
+  const int unit = bh * p.nkb + kb;
+  if constexpr (kTensor == 0) {
+    int8_t* tile = reinterpret_cast<int8_t*>(p.kv_tiles) + static_cast<long>(unit) * record_bytes<D, kSage>();
+    float* scales = p.key_scale + static_cast<long>(unit) * kKeyScaleSlots;
+    if (full_unit) {
+      quantize_key_rows<kBf16, D, false>(raw, stat, kKeys, tile, scales, p.per_thread, lane);
+    } else {
+      const int valid_rows = max(0, min(kKeys, p.key_length - kb * kKeyBlock - lane / (D / 8) * kKeys));
+      uint4 rows[kKeys];
+      load_unit_rows<D, true>(p.key, b, h, kb, p.key_length, lane, rows);
+      quantize_key_rows<kBf16, D, true>(rows, stat, valid_rows, tile, scales, p.per_thread, lane);
+    }
+  } else {
+    if (full_unit) {
+      quantize_value_codes<kBf16, D, kSage, false>(p, unit, lane, raw, stat);
+    } else {
+      uint4 rows[kKeys];
+      load_unit_rows<D, true>(p.value, b, h, kb, p.key_length, lane, rows);
+      quantize_value_codes<kBf16, D, kSage, true>(p, unit, lane, rows, stat);
+    }
+  }
+}
+
+// One chunk of tensor kTensor (0: K, 1: V) of batch-head bh: load, level-0 and level-1 statistics, the
+// sequence's statistic, codes.  The whole pipeline is inlined once per tensor so that each keeps its
+// rows (64 VGPRs at D = 128) in registers without the other's code in between.
+template <bool kBf16, int D, bool kSage, int kTensor>
+__device__ __forceinline__ void single_pass_chunk(const SinglePassParams& p, SinglePassShared<D>& sh, int bh, int chunk,
                                                   int wave, int lane) {
-  constexpr int D = 128;
   constexpr int L = 16;
+  constexpr int kGroups = D / 8;
+  constexpr int kSubs = kWave / kGroups;
+  constexpr int kKeys = kKeyBlock / kSubs;
+  constexpr bool kAbsMax = kSage && kTensor == 1;
   const int chunks = p.m.chunks;
-  const int pair = 2 * bh + kTensor;
   const int b = bh / p.q.heads;
   const int h = bh - b * p.q.heads;
   const int length = p.q.key_length;
   const InputTensor& in = kTensor == 0 ? p.q.key : p.q.value;
   const int kb = chunk * 4 + wave;  // this wave's K block / V tile
-  const int group = lane & 15;
-  const int sub = lane >> 4;
-  const int first_row = kb * kKeyBlock + sub * 16;  // this lane's rows [first_row, +16)
-  const int valid_rows = max(0, min(16, length - first_row));
+  const int group = lane % kGroups;
+  const int sub = lane / kGroups;
+  const int first_row = kb * kKeyBlock + sub * kKeys;  // this lane's rows [first_row, +kKeys)
   const bool full_unit = (kb + 1) * kKeyBlock <= length;
 
-  uint4 raw[16];
+  uint4 raw[kKeys];
   if (full_unit) {
     load_unit_rows<D, false>(in, b, h, kb, length, lane, raw);
   } else {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) raw[j] = make_uint4(0, 0, 0, 0);
+    for (int j = 0; j < kKeys; ++j) raw[j] = make_uint4(0, 0, 0, 0);
   }
 
-  float* mean_out = (kTensor == 0 ? p.m.key_mean : p.m.value_mean) + static_cast<long>(bh) * D;
-  const bool centred = kTensor == 0 || p.q.center_value;
-  if (centred) {
-    // level 0: this lane's block of L rows, in row order from +0.0 (a partial unit reads its
-    // rows here with guards; they are read again for the codes)
+  float* out = (kTensor == 0 ? p.m.key_mean : kSage ? p.m.value_scale : p.m.value_mean) + static_cast<long>(bh) * D;
+  const bool used = kTensor == 0 || kSage || p.q.center_value;
+  if (used) {
+    // level 0: this lane's rows, in row order (a partial unit reads its rows here with guards; they
+    // are read again for the codes)
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (full_unit) {
+    const auto add_rows = [&]() {
+      if (full_unit) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        float f[8];
-        widen8<kBf16>(raw[j], f);
+        for (int j = 0; j < kKeys; ++j) {
+          float f[8];
+          widen8<kBf16>(raw[j], f);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += f[i];
+          for (int i = 0; i < 8; ++i) acc[i] = kAbsMax ? fmaxf(acc[i], fabsf(f[i])) : acc[i] + f[i];
+        }
+      } else {
+        const int valid_rows = max(0, min(kKeys, length - first_row));
+        const uint16_t* rows = static_cast<const uint16_t*>(in.data) + b * in.stride_batch + h * in.stride_head +
+                               static_cast<long>(first_row) * in.stride_seq + 8 * group;
+        for (int j = 0; j < valid_rows; ++j) {
+          float f[8];
+          widen8<kBf16>(*reinterpret_cast<const uint4*>(rows + static_cast<long>(j) * in.stride_seq), f);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i] = kAbsMax ? fmaxf(acc[i], fabsf(f[i])) : acc[i] + f[i];
+        }
       }
-    } else if (valid_rows > 0) {
-      const uint16_t* rows = static_cast<const uint16_t*>(in.data) + b * in.stride_batch + h * in.stride_head +
-                             static_cast<long>(first_row) * in.stride_seq + 8 * group;
-      for (int j = 0; j < valid_rows; ++j) {
-        float f[8];
-        widen8<kBf16>(*reinterpret_cast<const uint4*>(rows + static_cast<long>(j) * in.stride_seq), f);
+    };
+    add_rows();
+    if constexpr (!kAbsMax && kKeys == 8) {
+      // half a level-0 block per lane: the odd lane adds its rows to the even lane's sum
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += f[i];
+      for (int i = 0; i < 8; ++i) {
+        const float below = __shfl_up(acc[i], kGroups, kWave);
+        acc[i] = (sub & 1) != 0 ? below : 0.0f;
       }
+      add_rows();
     }
-    float4* dst = reinterpret_cast<float4*>(&sh.block_sums[4 * wave + sub][8 * group]);
-    dst[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    dst[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
-    // the K codes widen the packed rows again: the 128 floats of this pass stay dead (the V
+    const int slot = kAbsMax ? kSubs * wave + sub : (kSubs * wave + sub) * kKeys / L;
+    if (kAbsMax || kKeys == L || (sub & 1) != 0) {
+      float4* dst = reinterpret_cast<float4*>(&sh.block_sums[slot][8 * group]);
+      dst[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      dst[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    }
+    // the K codes widen the packed rows again: the widened floats of this pass stay dead (the V
     // tile's register reuse needs no such hint)
     if constexpr (kTensor == 0) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) asm volatile("" : "+v"(raw[j].x), "+v"(raw[j].y), "+v"(raw[j].z), "+v"(raw[j].w));
+      for (int j = 0; j < kKeys; ++j) asm volatile("" : "+v"(raw[j].x), "+v"(raw[j].y), "+v"(raw[j].z), "+v"(raw[j].w));
     }
     __syncthreads();
     // level 1: the chunk's complete blocks in order; a short last chunk's trailing rows go to
-    // slot `chunks` (mean_chunk's layout)
+    // slot `chunks` (mean_chunk's layout).  A maximum takes every row of the chunk.
     const int rows = min(L * L, length - chunk * L * L);
     const int full = rows / L;
     const int tail = rows - full * L;
+    const int pair = kTensor * p.m.batch_heads + bh;
     float* src = p.m.partials + (static_cast<long>(pair) * (chunks + 1)) * D;
     if (threadIdx.x < D) {
       const int col = threadIdx.x;
       float s = 0.0f;
-      for (int blk = 0; blk < full; ++blk) s += sh.block_sums[blk][col];
+      if constexpr (kAbsMax) {
+#pragma unroll
+        for (int blk = 0; blk < 4 * kSubs; ++blk) s = fmaxf(s, sh.block_sums[blk][col]);
+      } else {
+        for (int blk = 0; blk < full; ++blk) s += sh.block_sums[blk][col];
+      }
       store_coherent(src + static_cast<long>(chunk) * D + col, s);
-      if (chunk == chunks - 1)
+      if (!kAbsMax && chunk == chunks - 1)
         store_coherent(src + static_cast<long>(chunks) * D + col, tail > 0 ? sh.block_sums[full][col] : 0.0f);
     }
     __builtin_amdgcn_s_waitcnt(0);  // the stores are complete before the arrival is counted
     __syncthreads();
     if (threadIdx.x == 0)
-      sh.last = __hip_atomic_fetch_add(p.arrivals + pair, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                static_cast<uint32_t>(chunks - 1);
+      sh.last = __hip_atomic_fetch_add(p.arrivals + bh * p.arrival_stride + kTensor, 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT) == static_cast<uint32_t>(chunks - 1);
     __syncthreads();
     if (sh.last) {
-      const int col = threadIdx.x & (D - 1);
-      const float m = single_pass_mean(p.m, src + col, col, threadIdx.x >> 7, sh.group_sums);
+      const int col = threadIdx.x % D;
+      const float m = single_pass_statistic<D, kAbsMax>(p.m, src + col, col, threadIdx.x / D, sh.group_sums);
       if (threadIdx.x < D) {
-        sh.mean[col] = m;
-        store_coherent(mean_out + col, m);  // replaces the pending mark: the other chunks go on
+        sh.statistic[col] = m;
+        store_coherent(out + col, m);  // replaces the pending mark: the other chunks go on
       }
     } else {
-      // wait for this column's mean to replace the pending mark (kMeanPending, a signalling NaN
+      // wait for this column's statistic to replace the pending mark (kMeanPending, a signalling NaN
       // that no arithmetic produces), at most spin_limit polls
       bool waiting = false;
       if (threadIdx.x < D) {
         uint32_t bits = kMeanPending;
         for (int polls = 0; polls < p.spin_limit; ++polls) {
-          bits = __hip_atomic_load(reinterpret_cast<const uint32_t*>(mean_out) + threadIdx.x, __ATOMIC_RELAXED,
+          bits = __hip_atomic_load(reinterpret_cast<const uint32_t*>(out) + threadIdx.x, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
           if (bits != kMeanPending) break;
           __builtin_amdgcn_s_sleep(2);
         }
         waiting = bits == kMeanPending;
-        sh.mean[threadIdx.x] = __builtin_bit_cast(float, bits);
+        sh.statistic[threadIdx.x] = __builtin_bit_cast(float, bits);
       }
-      // a column still pending: the chunk computes every column's mean from the rows itself
+      // a column still pending: the chunk computes every column's statistic from the rows itself
       if (__syncthreads_or(waiting)) {
-        if (threadIdx.x < D) sh.mean[threadIdx.x] = column_mean_from_rows<kBf16>(in, b, h, threadIdx.x, length);
-        if (threadIdx.x == 0) __hip_atomic_fetch_add(p.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x < D)
+          sh.statistic[threadIdx.x] = kAbsMax ? column_scale_from_rows<kBf16>(in, b, h, threadIdx.x, length)
+                                              : column_mean_from_rows<kBf16>(in, b, h, threadIdx.x, length);
+        if (!kSage && threadIdx.x == 0) __hip_atomic_fetch_add(p.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
     __syncthreads();
   } else if (chunk == 0 && threadIdx.x < D) {
-    mean_out[threadIdx.x] = 0.0f;  // causal: V is not centred, its mean slot reads zero
+    out[threadIdx.x] = 0.0f;  // causal: V is not centred, its mean slot reads zero
   }
   if (kb >= p.q.nkb) return;
 
-  float mu[8];
+  float stat[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) mu[i] = centred ? sh.mean[8 * group + i] : 0.0f;
-  const int unit = bh * p.q.nkb + kb;
-  if constexpr (kTensor == 0) {
-    int8_t* tile = reinterpret_cast<int8_t*>(p.q.kv_tiles) + static_cast<long>(unit) * kv_tile_bytes(D);
-    float* scales = p.q.key_scale + static_cast<long>(unit) * kKeyScaleSlots;
-    if (full_unit) {
-      quantize_key_rows<kBf16, false>(raw, mu, valid_rows, tile, scales, p.q.per_thread, lane);
-    } else {
-      uint4 rows[16];
-      load_unit_rows<D, true>(in, b, h, kb, length, lane, rows);
-      quantize_key_rows<kBf16, true>(rows, mu, valid_rows, tile, scales, p.q.per_thread, lane);
-    }
-  } else {
-    if (full_unit) {
-      quantize_value_rows<kBf16, D, false>(p.q, unit, lane, raw, mu);
-    } else {
-      uint4 rows[16];
-      load_unit_rows<D, true>(in, b, h, kb, length, lane, rows);
-      quantize_value_rows<kBf16, D, true>(p.q, unit, lane, rows, mu);
-    }
-  }
+  for (int i = 0; i < 8; ++i) stat[i] = used ? sh.statistic[8 * group + i] : 0.0f;
+  quantize_unit_rows<kBf16, D, kSage, kTensor>(p.q, bh, kb, lane, full_unit, raw, stat);
 }
 
-template <bool kBf16>
+template <bool kBf16, int D, bool kSage>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 prep_single_pass_kernel(const SinglePassParams p) {
-  __shared__ __attribute__((aligned(16))) SinglePassShared sh;
+  __shared__ __attribute__((aligned(16))) SinglePassShared<D> sh;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: index math stays scalar
   const int lane = threadIdx.x & 63;
   const int logical = xcc_remap(blockIdx.x, gridDim.x, p.xccs);
-  if (logical >= p.kv_workgroups) {  // the two-step path's Q blocks: no mean, no wait
-    const int unit = (logical - p.kv_workgroups) * 4 + wave;
-    if (unit < p.q.batch_heads * p.q.nqb) quantize_query_unit<kBf16, 128>(p.q, unit);
-    return;
+  if constexpr (!kSage) {
+    if (logical >= p.kv_workgroups) {  // the two-step path's Q blocks: no mean, no wait
+      const int unit = (logical - p.kv_workgroups) * 4 + wave;
+      if (unit < p.q.batch_heads * p.q.nqb) quantize_query_unit<kBf16, D>(p.q, unit);
+      return;
+    }
   }
   const int pair = logical / p.m.chunks;  // (batch-head, tensor): K and V of a batch-head are neighbours
   const int chunk = logical - pair * p.m.chunks;
-  if (pair & 1) single_pass_chunk<kBf16, 1>(p, sh, pair >> 1, chunk, wave, lane);
-  else single_pass_chunk<kBf16, 0>(p, sh, pair >> 1, chunk, wave, lane);
+  if (pair & 1) single_pass_chunk<kBf16, D, kSage, 1>(p, sh, pair >> 1, chunk, wave, lane);
+  else single_pass_chunk<kBf16, D, kSage, 0>(p, sh, pair >> 1, chunk, wave, lane);
 }
 
-// Before the single-pass prep: arrival counters and status word cleared, the means marked
-// pending (the V mean only when V is centred).
-__global__ void __launch_bounds__(256) prep_clear_kernel(uint32_t* words, int count, float* key_mean, float* value_mean,
-                                                         int means, int centre_value) {
+// Before the single-pass prep: arrival counters (batch-head bh's at [bh * stride], `words` of them) and
+// status word cleared, the statistics marked pending (`value` only where V has one).
+__global__ void __launch_bounds__(256) prep_clear_kernel(uint32_t* arrivals, long stride, int batch_heads, uint32_t* status,
+                                                         float* key, float* value, int columns) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < count) words[i] = 0u;
-  if (i < means) {
-    key_mean[i] = __builtin_bit_cast(float, kMeanPending);
-    if (centre_value) value_mean[i] = __builtin_bit_cast(float, kMeanPending);
+  if (i < 2 * batch_heads) arrivals[(i >> 1) * stride + (i & 1)] = 0u;
+  if (i == 0 && status != nullptr) *status = 0u;
+  if (i < columns) {
+    key[i] = __builtin_bit_cast(float, kMeanPending);
+    if (value != nullptr) value[i] = __builtin_bit_cast(float, kMeanPending);
   }
 }
 
 // ---------------------------------------------------------------------------------------
-// SageAttention2++ quantisation (sage_attention_2pp/reference.py:22-25, 44-49).  Each wave
-// owns a 64-row K block (the Piper K path, into the SageAttention2++ tile record) or a
-// 64-key V tile: FP8 E4M3 codes of v / scale[channel] (the correctly rounded FP32 quotient,
-// then v_cvt_pk_fp8_f32: round to nearest even, bit-identical to torch's float8_e4m3fn
-// cast), written transposed into the record's V^T rows.  Keys past the end get code 0.
+// Short prep (sequences of at most kShortChunks chunks): one launch, no workspace, no waiting.  One
+// workgroup per 256-row chunk of one batch-head's K or V, its units' rows loaded first; then the workgroup
+// sums the whole sequence itself (every chunk's workgroup the same sums, from L2), so nothing is handed
+// between workgroups, and quantises its rows from registers.  A call of this size is bound by its chain of
+// launches and memory round trips: B1 H8 S1024 D64 3.8 + 3.9 + 5.6 us in three kernels, 8.0 in this one
+// (SageAttention2++ 3.7 + 3.7 + 4.5 and 6.4); B2 H12 S333 D128 2.1 + 12.2 in the single pass, 10.1 here.
+// Longer sequences would read too much per workgroup, and more workgroups than two per CU are no longer
+// a matter of latency (B4 H20 S1024 D128, 640 workgroups: two-pass).
 // ---------------------------------------------------------------------------------------
-template <bool kBf16, int D>
-__global__ void __launch_bounds__(256) sage_quantize_kernel(const SageQuantParams p) {
+constexpr int kShortChunks = 4;
 
-  const int wave = threadIdx.x >> 6;
+template <int D>
+struct ShortShared {
+  float block_sums[kShortChunks * 16][D];
+  float statistic[D];
+};
+
+template <bool kBf16, int D, bool kSage, int kTensor>
+__device__ __forceinline__ void short_chunk(const PrepParams& p, ShortShared<D>& sh, int bh, int chunk, int wave, int lane) {
+  constexpr int L = 16;
+  constexpr int kGroups = D / 8;
+  constexpr int kKeys = kKeyBlock / (kWave / kGroups);
+  constexpr bool kAbsMax = kSage && kTensor == 1;
+  const int b = bh / p.q.heads;
+  const int h = bh - b * p.q.heads;
+  const int length = p.q.key_length;
+  const InputTensor& in = kTensor == 0 ? p.q.key : p.q.value;
+  const int kb = chunk * 4 + wave;
+  const bool full_unit = (kb + 1) * kKeyBlock <= length;
+  uint4 raw[kKeys];
+  if (full_unit) {
+    load_unit_rows<D, false>(in, b, h, kb, length, lane, raw);
+  } else {
+#pragma unroll
+    for (int j = 0; j < kKeys; ++j) raw[j] = make_uint4(0, 0, 0, 0);
+  }
+  float* out = (kTensor == 0 ? p.m.key_mean : kSage ? p.m.value_scale : p.m.value_mean) + static_cast<long>(bh) * D;
+  const bool used = kTensor == 0 || kSage || p.q.center_value;
+  if (used) {
+    const int full = length / L;  // complete level-0 blocks
+    const int tail = length - full * L;
+    const uint16_t* base = static_cast<const uint16_t*>(in.data) + b * in.stride_batch + h * in.stride_head +
+                           8 * (threadIdx.x % kGroups);
+    chunk_block_sums<kBf16, D, kAbsMax>(base, in.stride_seq, L, full, full + (tail > 0 ? 1 : 0), tail,
+                                        threadIdx.x / kGroups, threadIdx.x % kGroups, &sh.block_sums[0][0]);
+    __syncthreads();
+    if (threadIdx.x < D) {
+      const int col = threadIdx.x;
+      float m;
+      if constexpr (kAbsMax) {
+        float amax = 0.0f;
+        for (int blk = 0; blk < full + (tail > 0 ? 1 : 0); ++blk) amax = fmaxf(amax, sh.block_sums[blk][col]);
+        m = channel_scale(amax);
+      } else {
+        // levels 1 to 3 (finalize_column): fewer than 16 chunks, so level 3 stays empty
+        float level2 = 0.0f;
+        int blk = 0;
+        for (int c = 0; c < full / L; ++c) {
+          float level1 = 0.0f;
+#pragma unroll
+          for (int i = 0; i < L; ++i) level1 += sh.block_sums[blk + i][col];
+          blk += L;
+          level2 += level1;
+        }
+        float level1 = 0.0f;
+        for (; blk < full; ++blk) level1 += sh.block_sums[blk][col];
+        const float level0 = tail > 0 ? sh.block_sums[full][col] : 0.0f;
+        m = (((level0 + level1) + level2) + 0.0f) / static_cast<float>(length);
+      }
+      sh.statistic[col] = m;
+      if (chunk == 0) out[col] = m;
+    }
+    __syncthreads();
+  } else if (chunk == 0 && threadIdx.x < D) {
+    out[threadIdx.x] = 0.0f;  // causal: V is not centred, its mean slot reads zero
+  }
+  if (kb >= p.q.nkb) return;
+  float stat[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) stat[i] = used ? sh.statistic[8 * (lane % kGroups) + i] : 0.0f;
+  quantize_unit_rows<kBf16, D, kSage, kTensor>(p.q, bh, kb, lane, full_unit, raw, stat);
+}
+
+// Two waves per SIMD: the unit's rows and the sums' loads in flight together need over 128 VGPRs, and a
+// grid of this path is small.
+template <bool kBf16, int D, bool kSage>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) prep_short_kernel(const PrepParams p) {
+  __shared__ __attribute__((aligned(16))) ShortShared<D> sh;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int block = blockIdx.x;
-
-  if (block < p.k_blocks_wg) {
-    const int unit = block * 4 + wave;
-    if (unit >= p.batch_heads * p.nkb) return;
-    const int bh = unit / p.nkb;
-    const int kb = unit - bh * p.nkb;
-    const int b = bh / p.heads;
-    const int h = bh - b * p.heads;
-    int8_t* tile = reinterpret_cast<int8_t*>(p.kv_tiles) + static_cast<long>(unit) * sage_tile_bytes(D);
-    const float* mean = p.key_mean + static_cast<long>(bh) * D;
-    float* scales = p.key_scale + static_cast<long>(unit) * kKeyScaleSlots;
-    if ((kb + 1) * kKeyBlock <= p.key_length)
-      quantize_block<kBf16, D, kKeyBlock, true, kv_k_stride(D), kKeyScaleSlots, false>(
-          p.key, b, h, kb * kKeyBlock, p.key_length, mean, tile, scales, p.per_thread);
-    else
-      quantize_block<kBf16, D, kKeyBlock, true, kv_k_stride(D), kKeyScaleSlots, true>(
-          p.key, b, h, kb * kKeyBlock, p.key_length, mean, tile, scales, p.per_thread);
-    return;
-  }
-
-  // V tile: lane (group, sub) owns columns [8 group, +8) of the kKeys consecutive keys
-  // [kKeys sub, +kKeys), converts them with the per-channel divisors and packs four keys of a
-  // column per word: the 16-byte (D = 128) or 8-byte (D = 64) pieces of its eight V^T rows.
-  const int unit = (block - p.k_blocks_wg) * 4 + wave;
-  if (unit >= p.batch_heads * p.nkb) return;
-  const int bh = unit / p.nkb;
-  const int kb = unit - bh * p.nkb;
-  const int b = bh / p.heads;
-  const int h = bh - b * p.heads;
-  constexpr int kGroups = D / 8;
-  constexpr int kSubs = kWave / kGroups;
-  constexpr int kKeys = kKeyBlock / kSubs;
-  const int group = lane % kGroups;
-  const int sub = lane / kGroups;
-  const int key0 = sub * kKeys;
-  const uint16_t* base = static_cast<const uint16_t*>(p.value.data) + b * p.value.stride_batch +
-                         h * p.value.stride_head + group * 8;
-  uint4 raw[kKeys];
-#pragma unroll
-  for (int j = 0; j < kKeys; ++j) {
-    const int row = kb * kKeyBlock + key0 + j;
-    raw[j] = row < p.key_length ? *reinterpret_cast<const uint4*>(base + static_cast<long>(row) * p.value.stride_seq)
-                                : make_uint4(0, 0, 0, 0);
-  }
-  Divisor divisor[8];  // this lane's 8 channels
-#pragma unroll
-  for (int i = 0; i < 8; ++i) divisor[i] = Divisor(p.value_scale[static_cast<long>(bh) * D + group * 8 + i]);
-  uint32_t packed[8][kKeys / 4];  // [column][four keys]
-#pragma unroll
-  for (int j4 = 0; j4 < kKeys / 4; ++j4) {
-    float q[4][8];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      float f[8];
-      widen8<kBf16>(raw[4 * j4 + u], f);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) q[u][i] = divisor[i].quotient(f[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0][i], q[1][i], 0, false);
-      packed[i][j4] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(q[2][i], q[3][i], lo, true));
+  const int kv_workgroups = 2 * p.q.batch_heads * p.m.chunks;
+  if (!kSage && block == 0 && threadIdx.x == 0) *p.m.status = 0u;  // this path never waits
+  if constexpr (!kSage) {
+    if (block >= kv_workgroups) {  // the two-step path's Q blocks
+      const int unit = (block - kv_workgroups) * 4 + wave;
+      if (unit < p.q.batch_heads * p.q.nqb) quantize_query_unit<kBf16, D>(p.q, unit);
+      return;
     }
   }
-  uint8_t* tile = p.kv_tiles + static_cast<long>(unit) * sage_tile_bytes(D);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    uint8_t* dst = tile + sage_v_offset(D) + (group * 8 + i) * kv_v_stride() + key0;
-    if constexpr (kKeys == 16)
-      *reinterpret_cast<uint4*>(dst) = make_uint4(packed[i][0], packed[i][1], packed[i][2], packed[i][3]);
-    else
-      *reinterpret_cast<uint2*>(dst) = make_uint2(packed[i][0], packed[i][1]);
-  }
+  const int pair = block / p.m.chunks;
+  const int chunk = block - pair * p.m.chunks;
+  if (pair & 1) short_chunk<kBf16, D, kSage, 1>(p, sh, pair >> 1, chunk, wave, lane);
+  else short_chunk<kBf16, D, kSage, 0>(p, sh, pair >> 1, chunk, wave, lane);
 }
 
 // ---------------------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------------------
-template <bool kBf16, int D>
-static hipError_t launch_mean_partials(const MeanParams& mp, hipStream_t stream) {
+static bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
+
+template <bool kBf16, int D, bool kSage>
+static hipError_t launch_single_pass(const PrepParams& pp, const PrepDevice& dev, hipStream_t stream) {
+  SinglePassParams sp{};
+  sp.q = pp.q;
+  sp.m = pp.m;
+  const int bh = pp.m.batch_heads;
+  if constexpr (kSage) {
+    // the arrival counters sit in the V tensor's partial slots for trailing rows, which a maximum
+    // leaves unused: two words per batch-head at [1][bh][chunks][0]
+    sp.arrival_stride = static_cast<long>(pp.m.chunks + 1) * D;
+    sp.arrivals = reinterpret_cast<uint32_t*>(pp.m.partials) + bh * sp.arrival_stride +
+                  static_cast<long>(pp.m.chunks) * D;
+  } else {
+    uint32_t* sync = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(pp.m.partials) +
+                                                 prep_partial_bytes(bh, pp.m.length, D));
+    sp.arrival_stride = 2;
+    sp.arrivals = sync;
+    sp.status = sync + prep_status_word(bh);
+  }
+  sp.kv_workgroups = 2 * bh * pp.m.chunks;
+  sp.xccs = dev.xccs;
+  sp.spin_limit = dev.spin_limit;
+  // a fill kernel, not hipMemsetAsync: safe to record in a captured graph
+  const int columns = bh * D;
+  float* value = kSage ? pp.m.value_scale : pp.q.center_value ? pp.m.value_mean : nullptr;
+  hipLaunchKernelGGL(prep_clear_kernel, dim3((columns + 255) / 256), dim3(256), 0, stream, sp.arrivals, sp.arrival_stride,
+                     bh, sp.status, pp.m.key_mean, value, columns);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  const long workgroups = static_cast<long>(sp.kv_workgroups) + pp.q.q_blocks_wg;
+  hipLaunchKernelGGL((prep_single_pass_kernel<kBf16, D, kSage>), dim3(static_cast<unsigned>(workgroups)), dim3(256), 0,
+                     stream, sp);
+  return hipGetLastError();
+}
+
+template <bool kBf16, int D, bool kSage>
+static hipError_t launch_prep_typed(const MeanParams& mp, const QuantParams& qp, const PrepDevice& dev, hipStream_t stream) {
+  const PrepParams pp{qp, mp};
+  const bool cascade16 = mp.block_rows == 16;  // every path but the three-pass one sums blocks of 16 rows
+  const bool forced = dev.spin_limit == 0;     // the single pass's fallback was asked for
+  const long kv_workgroups = 2L * mp.batch_heads * mp.chunks;
+  if (cascade16 && !forced && mp.chunks <= kShortChunks && (mp.chunks == 1 || kv_workgroups <= 2 * dev.cus)) {
+    hipLaunchKernelGGL((prep_short_kernel<kBf16, D, kSage>), dim3(static_cast<unsigned>(kv_workgroups + qp.q_blocks_wg)),
+                       dim3(256), 0, stream, pp);
+    return hipGetLastError();
+  }
+  const bool finish_in_waves = cascade16 && mp.chunks <= kWaveChunks;
+  const long kv_bytes = 4L * mp.batch_heads * mp.length * D;
+  const bool single_pass = cascade16 && mp.chunks <= kSinglePassChunks && single_pass_resident(mp.chunks, dev.cus, dev.xccs) &&
+                           aligned4(mp.partials) && aligned4(mp.key_mean) && aligned4(kSage ? mp.value_scale : mp.value_mean);
+  if (single_pass && (forced || !finish_in_waves || kv_bytes > two_pass_bytes(D)))
+    return launch_single_pass<kBf16, D, kSage>(pp, dev, stream);
+
   // one workgroup per (tensor, batch-head, chunk); LDS holds the chunk's L block sums of D columns
   const long workgroups = static_cast<long>(mp.tensors) * mp.batch_heads * mp.chunks;
   const size_t lds = static_cast<size_t>(mp.block_rows) * D * sizeof(float);
-  hipLaunchKernelGGL((mean_partial_kernel<kBf16, D>), dim3(static_cast<unsigned>(workgroups)), dim3(256), lds, stream,
-                     mp);
-  return hipGetLastError();
-}
-
-template <bool kBf16, int D>
-static hipError_t launch_prep_typed(const MeanParams& mp, const QuantParams& qp, const PrepDevice& dev,
-                                    hipStream_t stream) {
-  if (D == 128 && mp.block_rows == 16 && mp.chunks <= kSinglePassChunks && !mp.value_absmax &&
-      single_pass_resident(mp.chunks, dev.cus, dev.xccs)) {
-    SinglePassParams sp{};
-    sp.q = qp;
-    sp.m = mp;
-    const int words = static_cast<int>(prep_sync_words(mp.batch_heads));
-    uint32_t* sync = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(mp.partials) +
-                                                 prep_partial_bytes(mp.batch_heads, mp.length, D));
-    sp.arrivals = sync;
-    sp.status = sync + prep_status_word(mp.batch_heads);
-    sp.kv_workgroups = 2 * mp.batch_heads * mp.chunks;
-    sp.xccs = dev.xccs;
-    sp.spin_limit = dev.spin_limit;
-    // a fill kernel, not hipMemsetAsync: safe to record in a captured graph
-    const int means = mp.batch_heads * D;
-    const int threads = words > means ? words : means;
-    hipLaunchKernelGGL(prep_clear_kernel, dim3((threads + 255) / 256), dim3(256), 0, stream, sync, words, mp.key_mean,
-                       mp.value_mean, means, qp.center_value);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    const long workgroups = static_cast<long>(sp.kv_workgroups) + qp.q_blocks_wg;
-    hipLaunchKernelGGL((prep_single_pass_kernel<kBf16>), dim3(static_cast<unsigned>(workgroups)), dim3(256), 0, stream,
-                       sp);
+  hipLaunchKernelGGL((mean_partial_kernel<kBf16, D>), dim3(static_cast<unsigned>(workgroups)), dim3(256), lds, stream, mp);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  const dim3 blocks(static_cast<unsigned>(qp.q_blocks_wg + qp.k_blocks_wg + qp.v_blocks_wg));
+  if (finish_in_waves) {
+    hipLaunchKernelGGL((quantize_kernel<kBf16, D, kSage, true>), blocks, dim3(256), 0, stream, pp);
     return hipGetLastError();
   }
-  hipError_t err = launch_mean_partials<kBf16, D>(mp, stream);
-  if (err != hipSuccess) return err;
   const int fin_threads = 2 * mp.batch_heads * D;
   hipLaunchKernelGGL(mean_finalize_kernel, dim3((fin_threads + 63) / 64), dim3(64), 0, stream, mp, D);
   err = hipGetLastError();
   if (err != hipSuccess) return err;
-  const int blocks = qp.q_blocks_wg + qp.k_blocks_wg + qp.v_blocks_wg;
-  hipLaunchKernelGGL((quantize_kernel<kBf16, D>), dim3(blocks), dim3(256), 0, stream, qp);
+  hipLaunchKernelGGL((quantize_kernel<kBf16, D, kSage, false>), blocks, dim3(256), 0, stream, pp);
   return hipGetLastError();
 }
 
-template <bool kBf16, int D>
-static hipError_t launch_sage_prep_typed(const MeanParams& mp, const SageQuantParams& qp, hipStream_t stream) {
-  hipError_t err = launch_mean_partials<kBf16, D>(mp, stream);
-  if (err != hipSuccess) return err;
-  const int fin_threads = 2 * mp.batch_heads * D;
-  hipLaunchKernelGGL(mean_finalize_kernel, dim3((fin_threads + 63) / 64), dim3(64), 0, stream, mp, D);
-  err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  hipLaunchKernelGGL((sage_quantize_kernel<kBf16, D>), dim3(qp.k_blocks_wg + qp.v_blocks_wg), dim3(256), 0, stream,
-                     qp);
-  return hipGetLastError();
+template <bool kSage>
+static hipError_t launch_prep_operator(bool bf16, int head_dim, const MeanParams& mp, const QuantParams& qp,
+                                       const PrepDevice& dev, hipStream_t stream) {
+  if (bf16)
+    return head_dim == 128 ? launch_prep_typed<true, 128, kSage>(mp, qp, dev, stream)
+                           : launch_prep_typed<true, 64, kSage>(mp, qp, dev, stream);
+  return head_dim == 128 ? launch_prep_typed<false, 128, kSage>(mp, qp, dev, stream)
+                         : launch_prep_typed<false, 64, kSage>(mp, qp, dev, stream);
 }
 
-hipError_t launch_sage_prep(bool bf16, int head_dim, const MeanParams& mp, const SageQuantParams& qp,
+hipError_t launch_sage_prep(bool bf16, int head_dim, const MeanParams& mp, const QuantParams& qp, const PrepDevice& dev,
                             hipStream_t stream) {
-  if (bf16) {
-    return head_dim == 128 ? launch_sage_prep_typed<true, 128>(mp, qp, stream)
-                           : launch_sage_prep_typed<true, 64>(mp, qp, stream);
-  }
-  return head_dim == 128 ? launch_sage_prep_typed<false, 128>(mp, qp, stream)
-                         : launch_sage_prep_typed<false, 64>(mp, qp, stream);
+  return launch_prep_operator<true>(bf16, head_dim, mp, qp, dev, stream);
 }
 
 hipError_t launch_prep(bool bf16, int head_dim, const MeanParams& mp, const QuantParams& qp, const PrepDevice& dev,
                        hipStream_t stream) {
-  if (bf16) {
-    return head_dim == 128 ? launch_prep_typed<true, 128>(mp, qp, dev, stream)
-                           : launch_prep_typed<true, 64>(mp, qp, dev, stream);
-  }
-  return head_dim == 128 ? launch_prep_typed<false, 128>(mp, qp, dev, stream)
-                         : launch_prep_typed<false, 64>(mp, qp, dev, stream);
+  return launch_prep_operator<false>(bf16, head_dim, mp, qp, dev, stream);
 }
 
 }  // namespace piper
