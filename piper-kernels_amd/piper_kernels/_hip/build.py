@@ -2,8 +2,9 @@
 
 ``libpiper_mi355x.so`` is the operator's C ABI (``include/piper_mi355x.h``); ``libpiper_probe.so``
 holds the measurement probes (``include/piper_probe.h``), which only bench.py and the tests load.
-Both are plain C-ABI shared objects (no torch headers), built in-tree next to this file so they
-travel with the repository.  ``python -m piper_kernels._hip.build`` rebuilds them.
+Both are plain C-ABI shared objects (no torch headers).  ``libpiper_torch.so`` registers the custom
+ops' GPU kernels with torch over that C ABI (host code only).  All are built in-tree next to this file
+so they travel with the repository.  ``python -m piper_kernels._hip.build`` rebuilds them.
 """
 
 from __future__ import annotations
@@ -23,6 +24,8 @@ LIBRARY_PATH = Path(__file__).resolve().parent / "libpiper_mi355x.so"
 PROBE_LIBRARY_PATH = Path(__file__).resolve().parent / "libpiper_probe.so"
 SOURCES = ("abi.hip", "prep.hip", "attention.hip", "sage2pp.hip")
 PROBE_SOURCES = ("probe.hip",)
+TORCH_LIBRARY_PATH = Path(__file__).resolve().parent / "libpiper_torch.so"
+TORCH_SOURCE = "torch_op.cpp"
 OFFLOAD_ARCH = "gfx950"
 
 COMPILE_FLAGS = (
@@ -65,9 +68,28 @@ def _link(compiler: str, objects: list[Path], target: Path, verbose: bool) -> No
     os.replace(tmp, target)
 
 
+def _build_torch_library(verbose: bool) -> None:
+    """The torch kernels: one host source, compiled and linked against torch and the operator library."""
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(hipcc()).resolve().parents[1]
+    tmp = TORCH_LIBRARY_PATH.with_suffix(f".so.tmp{os.getpid()}")
+    _run(
+        ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+         "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+         f"-I{root / 'include'}", f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+         f"-I{rocm / 'include'}", "-I/opt/rocm/include", "-o", str(tmp), str(CSRC / TORCH_SOURCE),
+         f"-L{root / 'lib'}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+         f"-L{LIBRARY_PATH.parent}", "-lpiper_mi355x", "-Wl,-rpath,$ORIGIN"],
+        verbose,
+    )
+    os.replace(tmp, TORCH_LIBRARY_PATH)
+
+
 def build_library(verbose: bool = False) -> Path:
-    """Compile every HIP source for gfx950 and link both libraries; returns the operator
-    library's path (the probe library is ``PROBE_LIBRARY_PATH``)."""
+    """Compile every HIP source for gfx950, link both HIP libraries and build the torch kernels; returns
+    the operator library's path (the others: ``PROBE_LIBRARY_PATH``, ``TORCH_LIBRARY_PATH``)."""
     compiler = hipcc()
     BUILD_DIR.mkdir(parents=True, exist_ok=True)
     includes = [f"-I{INCLUDE}", f"-I{CSRC}"]
@@ -81,6 +103,7 @@ def build_library(verbose: bool = False) -> Path:
         list(pool.map(compile_one, sources))
     _link(compiler, [objects[s] for s in SOURCES], LIBRARY_PATH, verbose)
     _link(compiler, [objects[s] for s in PROBE_SOURCES], PROBE_LIBRARY_PATH, verbose)
+    _build_torch_library(verbose)
     return LIBRARY_PATH
 
 

@@ -1,5 +1,5 @@
-"""ctypes bindings of ``libpiper_mi355x.so`` (the operator's C ABI, ``include/piper_mi355x.h``)
-and of ``libpiper_probe.so`` (measurement probes, ``include/piper_probe.h``; loaded only by
+"""ctypes bindings of ``libpiper_mi355x.so`` (the operator's C ABI, ``include/piper_mi355x.h``),
+the loader of ``libpiper_torch.so`` (the custom ops' GPU kernels, ``csrc/torch_op.cpp``) and bindings of ``libpiper_probe.so`` (measurement probes, ``include/piper_probe.h``; loaded only by
 bench.py and the tests).
 
 The structures below mirror the header field for field.  torch is imported before the
@@ -16,7 +16,7 @@ from pathlib import Path
 
 import torch  # noqa: F401  (load torch's HIP runtime first; see module docstring)
 
-from .build import LIBRARY_PATH, PROBE_LIBRARY_PATH
+from .build import LIBRARY_PATH, PROBE_LIBRARY_PATH, TORCH_LIBRARY_PATH
 
 ABI_VERSION = 5
 QUERY_BLOCK = 32
@@ -326,13 +326,48 @@ class NativeLibrary:
 
 
 
+@ctypes.CFUNCTYPE(_i32, _i32, _i64, _i64, _i64, _i64, _i64, _i32)
+def _choose_plan(operator, batch, heads, query_length, key_length, head_dim, is_causal):
+    """The torch kernels' launch plan for a shape they have not seen (a negative number: none)."""
+    try:
+        from ..attention.piper_attention import _plan
+
+        select = _plan.select_sage_plan if operator else _plan.select_plan
+        return select(batch, heads, query_length, key_length, head_dim, bool(is_causal)).plan_id
+    except Exception:  # noqa: BLE001  (nothing may unwind through the C++ caller, which raises instead)
+        return -1
+
+
 _lock = threading.Lock()
 _library: NativeLibrary | None = None
+_torch_kernels: ctypes.CDLL | None = None
+
+
+def load_torch_kernels() -> None:
+    """Register the custom ops' GPU kernels with torch (once); raise :class:`LibraryUnavailableError`
+    if their library is absent."""
+    global _torch_kernels
+    with _lock:
+        if _torch_kernels is not None:
+            return
+        if not TORCH_LIBRARY_PATH.exists() or not LIBRARY_PATH.exists():
+            raise LibraryUnavailableError(
+                f"{TORCH_LIBRARY_PATH} is not built; run __graft_entry__.build() or python -m piper_kernels._hip.build"
+            )
+        try:
+            kernels = ctypes.CDLL(str(TORCH_LIBRARY_PATH))
+        except OSError as error:
+            raise LibraryUnavailableError(f"cannot open {TORCH_LIBRARY_PATH}: {error}") from error
+        kernels.piper_torch_set_plan_source.restype = None
+        kernels.piper_torch_set_plan_source(_choose_plan)
+        _torch_kernels = kernels
 
 
 def load_library(path: Path | None = None) -> NativeLibrary:
     """Open the in-tree library (once); raise :class:`LibraryUnavailableError` if absent."""
     global _library
+    if path is None and _library is not None:
+        return _library
     with _lock:
         if path is None and _library is not None:
             return _library

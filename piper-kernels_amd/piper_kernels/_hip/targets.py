@@ -59,4 +59,4 @@ class AcceleratorTarget:
     @property
     def supports_piper_mi355x(self) -> bool:
         """Whether the hand-written gfx950 (CDNA4, MI355X) kernels can run on this target."""
-        return self.is_amd_hip and self.is_architecture(MI355X_ARCHITECTURE)
+        return self.backend == "hip" and self.architecture == MI355X_ARCHITECTURE

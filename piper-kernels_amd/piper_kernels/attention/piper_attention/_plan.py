@@ -189,10 +189,14 @@ _PARTIAL_BYTES_PER_US = 4e6
 _MERGE_US = 2.2
 
 
+def _tile_us(head_dim: int) -> tuple[float, ...]:
+    return _TILE_US[64 if head_dim == 64 else 128]  # the library refuses any other head size
+
+
 def _split_us(tiles: int, rows: int, key_tiles: int, parts: int, head_dim: int) -> float:
     """Estimated time of a non-causal grid of `tiles` query tiles whose last, unfilled round of resident
     workgroups (`rows` query rows) is split into `parts` key ranges (csrc/kernels.h AttnParams)."""
-    steps = _TILE_US[head_dim]
+    steps = _tile_us(head_dim)
     slots = len(steps) * COMPUTE_UNITS
     whole, rest = divmod(tiles, slots)
     part_rounds, part_rest = divmod(rest * parts, slots)
@@ -215,7 +219,7 @@ def split_parts(batch: int, heads: int, query_length: int, key_length: int, head
     block_m = MI355XPlan(waves=4, three_per_cu=True).block_m
     tiles = batch * heads * (-(-query_length // block_m))
     key_tiles = -(-key_length // KEY_BLOCK)
-    rest = tiles % (len(_TILE_US[head_dim]) * COMPUTE_UNITS)
+    rest = tiles % (len(_tile_us(head_dim)) * COMPUTE_UNITS)
     if rest == 0:
         return 1
     rows = min(rest * block_m, batch * heads * query_length)

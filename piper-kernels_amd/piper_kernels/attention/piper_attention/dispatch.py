@@ -14,7 +14,7 @@ from __future__ import annotations
 
 import torch
 
-from ..._hip.library import load_library
+from ..._hip.library import load_library, load_torch_kernels
 from ..._hip.targets import AcceleratorTarget
 from .._validation import validate_attention_inputs
 from .hip import hip_piper_attention
@@ -60,4 +60,5 @@ def piper_attention(
         )
     if not torch.compiler.is_compiling():
         load_library()  # raises LibraryUnavailableError (a RuntimeError) if the library is missing
+        load_torch_kernels()
     return hip_piper_attention(query, key, value, converted_scale, is_causal)

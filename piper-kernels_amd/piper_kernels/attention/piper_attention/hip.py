@@ -306,7 +306,10 @@ def hip_piper_attention(
     is_causal: bool,
 ) -> torch.Tensor:
     """Piper Attention K/V prep + fused INT8 kernel (query quantised in its prologue) on MI355X
-    (schema of triton.py:984-999)."""
+    (schema of triton.py:984-999).  On the GPU this body runs only until ``csrc/torch_op.cpp`` has
+    registered the same call natively (in a compiled graph: its first call)."""
+    if query.is_cuda:
+        native.load_torch_kernels()
     return _run_piper_attention(query, key, value, scale, is_causal)
 
 

@@ -202,7 +202,10 @@ def hip_sage_attention_2pp(
     scale: float,
     is_causal: bool,
 ) -> torch.Tensor:
-    """SageAttention2++ K/V prep + fused INT8-QK / FP8-PV kernel on MI355X (schema of triton.py:1136-1145)."""
+    """SageAttention2++ K/V prep + fused INT8-QK / FP8-PV kernel on MI355X (schema of triton.py:1136-1145).
+    On the GPU this body runs only until ``csrc/torch_op.cpp`` has registered the same call natively."""
+    if query.is_cuda:
+        native.load_torch_kernels()
     return _run_sage_attention_2pp(query, key, value, scale, is_causal)
 
 

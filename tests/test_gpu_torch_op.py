@@ -1,0 +1,106 @@
+"""The native torch kernels (csrc/torch_op.cpp) against the Python path over the same C ABI, bit for bit:
+every option, inputs read in place and inputs that must be copied, a side stream whose inputs are freed
+at once, replays of a captured graph; errors stay Python exceptions; the plan source covers both
+operators."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from _parity import log
+from piper_kernels import piper_attention, sage_attention_2pp
+from piper_kernels._hip import library as native
+from piper_kernels.attention.piper_attention import _plan
+from piper_kernels.attention.piper_attention.hip import _run_piper_attention
+from piper_kernels.attention.sage_attention_2pp.hip import _run_sage_attention_2pp
+
+OPERATORS = {"piper": (piper_attention, _run_piper_attention), "sage": (sage_attention_2pp, _run_sage_attention_2pp)}
+
+
+def _inputs(b, h, sq, sk, d, dtype, device, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return tuple(torch.randn((b, h, s, d), generator=g).to(dtype).to(device) for s in (sq, sk, sk))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("operator", OPERATORS)
+@pytest.mark.parametrize("case", [
+    # (B, H, Sq, Sk, D, dtype, causal, layout): layouts read in place (bhsd, bshd) or copied (odd)
+    (1, 1, 1, 1, 64, torch.float16, False, "bhsd"),
+    (2, 3, 77, 77, 128, torch.bfloat16, True, "bshd"),
+    (1, 2, 300, 1000, 64, torch.bfloat16, False, "odd"),
+    (1, 8, 1024, 1024, 64, torch.float16, False, "bhsd"),  # key-range split: a workspace
+    (1, 24, 200, 3000, 128, torch.float16, False, "bshd"),
+], ids=str)
+def test_native_call_equals_the_python_path(case, operator, gfx950_device) -> None:
+    b, h, sq, sk, d, dtype, causal, layout = case
+    log(f"[case] torch op {operator} {case}")
+    q, k, v = _inputs(b, h, sq, sk, d, dtype, gfx950_device)
+    if layout == "bshd":
+        q, k, v = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (q, k, v))
+    elif layout == "odd":  # rows at odd multiples of two bytes
+        q, k, v = (torch.cat([x, x[..., :1]], -1)[..., :d] for x in (q, k, v))
+    public, python = OPERATORS[operator]
+    with torch.no_grad():
+        for scale in (None, 0.2):
+            got = public(q, k, v, scale=scale, is_causal=causal)
+            want = python(q, k, v, d**-0.5 if scale is None else scale, causal)
+            assert got.is_contiguous() and got.dtype is dtype and torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("operator", OPERATORS)
+def test_streams_and_graph_replays(operator, gfx950_device) -> None:
+    public, _ = OPERATORS[operator]
+    log(f"[case] torch op streams and graph {operator}")
+    sets = [_inputs(2, 4, 500, 500, 128, torch.float16, gfx950_device, seed) for seed in range(3)]
+    with torch.no_grad():
+        want = [public(*s, is_causal=True) for s in sets]
+        side = torch.cuda.Stream(gfx950_device)
+        side.wait_stream(torch.cuda.current_stream(gfx950_device))
+        got = []
+        for s in sets:
+            copies = tuple(x.clone() for x in s)
+            side.wait_stream(torch.cuda.current_stream(gfx950_device))
+            with torch.cuda.stream(side):
+                got.append(public(*copies, is_causal=True))
+            del copies  # freed while the side stream may still read them
+            torch.empty(1 << 20, device=gfx950_device).fill_(7.0)
+        torch.cuda.synchronize(gfx950_device)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+        static = tuple(x.clone() for x in sets[0])
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = public(*static, is_causal=True)
+        for i in (0, 1, 2, 0):
+            for x, y in zip(static, sets[i]):
+                x.copy_(y)
+            graph.replay()
+            torch.cuda.synchronize(gfx950_device)
+            assert torch.equal(out, want[i]), f"replay {i}"
+            assert torch.equal(public(*sets[i], is_causal=True), want[i])  # eager work between the replays
+
+
+@pytest.mark.gpu
+def test_errors_are_python_exceptions(gfx950_device) -> None:
+    native.load_torch_kernels()
+    op = torch.ops.piper_kernels.piper_attention
+    q = torch.zeros((1, 1, 8, 32), dtype=torch.float16, device=gfx950_device)
+    with pytest.raises(RuntimeError, match="head_dim must be 64 or 128"):
+        op(q, q, q, 0.125, False)
+    q = torch.zeros((1, 1, 8, 64), dtype=torch.float32, device=gfx950_device)
+    with pytest.raises(RuntimeError, match="float16 or bfloat16"):
+        op(q, q, q, 0.125, False)
+    q = q.half()
+    with pytest.raises(RuntimeError, match="scale must be finite and positive"):
+        op(q, q, q, 0.0, False)
+
+
+def test_plan_source_asks_the_package(monkeypatch) -> None:
+    ask = native._choose_plan
+    assert ask(0, 1, 8, 1024, 1024, 64, 0) == _plan.select_plan(1, 8, 1024, 1024, 64, False).plan_id
+    assert ask(1, 4, 32, 8192, 8192, 128, 1) == _plan.select_sage_plan(4, 32, 8192, 8192, 128, True).plan_id
+    monkeypatch.setattr(_plan, "select_plan", lambda *a: 1 / 0)
+    assert ask(0, 1, 8, 1024, 1024, 64, 0) < 0  # an error in Python is no plan
