@@ -206,9 +206,10 @@ typedef struct piper_prepare_args {
  * of the query tiles beyond whole rounds of resident workgroups are cut into `parts` ranges (2..8),
  * one workgroup each, which write their FP32 partial numerator, denominator and reference maximum to
  * the call's workspace; a merge kernel combines them (piper_attention_workspace_bytes gives the size).
- * For grids, or last rounds, too small to give every SIMD three waves.  The merge adds the parts in
- * another order than one sequential pass, so split plans agree with the others to rounding, not bit
- * for bit. */
+ * Two or four parts of a grid that then still fits the GPU at once are taken by the waves of one
+ * workgroup, whose sums meet in LDS (no partial sums in memory).  For grids, or last rounds, too small
+ * to give every SIMD three waves.  The merge adds the parts in another order than one sequential pass,
+ * so split plans agree with the others to rounding, not bit for bit. */
 #define PIPER_PLAN_KEY_PARTS(parts) (((parts) - 1) << 5)
 #define PIPER_PLAN_KEY_PARTS_OF(plan) ((((plan) >> 5) & 7) + 1)
 /* Work queues (Piper Attention, with PIPER_PLAN_THREE_WORKGROUPS, no key-range split): a

@@ -214,20 +214,28 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
     ap.query = to_input(*query);
   }
   // key-range split: part_tiles tiles per part, and no empty part; only the query tiles beyond whole
-  // rounds of resident workgroups are split
+  // rounds of resident workgroups are split.  Two or four parts of a grid whose workgroups then all fit
+  // the GPU at once are key streams instead.
   ap.key_parts = 1;
+  ap.key_streams = 1;
   if (key_parts > 1) {
     int cus = 0, xccs = 0;
     if (int st = device_topology(&cus, &xccs)) return st;
+    const int head_dim = static_cast<int>(s.head_dim);
     const int64_t tiles = static_cast<int64_t>(ap.query_tiles) * ap.batch_heads;
-    const int64_t slots = static_cast<int64_t>(piper::waves_per_simd(static_cast<int>(s.head_dim))) * std::max(cus, 1);
+    const int64_t slots = static_cast<int64_t>(piper::waves_per_simd(head_dim)) * std::max(cus, 1);
     ap.part_tiles = static_cast<int>(ceil_div(ap.nkb, key_parts));
     ap.key_parts = static_cast<int>(ceil_div(ap.nkb, ap.part_tiles));
     ap.whole_tiles = static_cast<int>(std::min<int64_t>(tiles / slots * slots, 0x7fffffff));
-    if (ap.whole_tiles == tiles) ap.key_parts = 1;
     ap.split_row0 = static_cast<long>(ap.whole_tiles / ap.query_tiles) * s.query_length +
                     static_cast<long>(ap.whole_tiles % ap.query_tiles) * block_m;
     ap.partials = static_cast<float*>(workspace);
+    if (ap.whole_tiles == tiles) ap.key_parts = 1;
+    if ((key_parts == 2 || key_parts == 4) && key_parts * tiles <= int64_t{piper::stream_workgroups(head_dim, key_parts)} * cus) {
+      ap.key_parts = 1;
+      ap.key_streams = key_parts;
+      ap.query_tiles = static_cast<int>(ceil_div(s.query_length, block_m / key_parts));
+    }
   }
   if (static_cast<int64_t>(ap.query_tiles) * ap.batch_heads * ap.key_parts > 0x7fffffff)
     return fail(PIPER_ERROR_UNSUPPORTED, "too many workgroups");

@@ -582,6 +582,180 @@ attention_w3_kernel(const AttnParams p) {
   w3_tile<D, kCausal, kOut, kPerThread, kCausal || kSplit, kSplit>(p, smem, tc, part, threadIdx.x & 63);
 }
 
+// Key streams: KS of a workgroup's four waves share 32 queries and take every KS-th key tile each, so a
+// grid too small to give every SIMD several waves gets KS times the waves, each with 1 / KS of the key
+// loop, and the sums meet in LDS at the end: no partial sums in memory, no merge kernel.  One iteration
+// stages KS consecutive tile records (double-buffered, as attention_w3_kernel); wave w handles query
+// group w % (4 / KS) and tile KS i + w / (4 / KS) of iteration i.  Per-block arithmetic is
+// block_update's; the waves' sums are aligned on their largest reference maximum as by
+// attention_merge_kernel, so results equal the sequential kernel's to rounding.  A lone wave of a SIMD
+// issues one VALU instruction per ~5.5 cycles and takes 1.2-1.5 us per key tile whatever the grid, which
+// is what bounds small grids: B1 H8 S1024 D64 12.9 + 4.2 us in four key parts and a merge, see
+// key_streams in kernels.h for the sizes that take this kernel and what they measured.
+template <int D, bool kCausal, int kOut, bool kPerThread, int KS>
+__global__ void __attribute__((amdgpu_flat_work_group_size(256, KS == 4 ? 512 : 256), amdgpu_waves_per_eu(KS == 4 ? 2 : stream_workgroups(D, KS), KS == 4 ? 2 : stream_workgroups(D, KS))))
+attention_streams_kernel(const AttnParams p) {
+  using L = TileLayout<D, 4>;
+  constexpr int kChunksD = D / 32;
+  constexpr int kGroups = 4 / KS;               // query groups of a workgroup
+  constexpr int kStage = KS * L::kStageBytes;
+  constexpr int kPieces = KS * L::kPieces;      // 1 KiB pieces of an iteration's records
+  constexpr int kRounds = (kPieces + 3) / 4;
+  constexpr int kShare = 4 * kChunksD / KS;     // four-feature groups that a wave writes at the end
+  __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
+  static_assert(4 * (D * 32 * 4 + 512) <= 2 * kStage, "every wave's sums fit the stages");
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5;
+  const int n = lane & 31;
+  const TileCoord tc = workgroup_tile<kCausal>(p);
+  const int bh = __builtin_amdgcn_readfirstlane(tc.bh);
+  const int qtile = __builtin_amdgcn_readfirstlane(tc.qtile);
+  const int group = wave % kGroups;
+  const int part = wave / kGroups;
+  const int q0 = qtile * (kGroups * 32) + group * 32;
+  const bool wave_live = q0 < p.query_length;
+
+  int tiles = p.nkb;
+  int wave_tiles = wave_live ? p.nkb : 0;
+  if constexpr (kCausal) {
+    tiles = (min(p.query_length, (qtile + 1) * kGroups * 32) - 1) / kKeyBlock + 1;
+    wave_tiles = wave_live ? (min(p.query_length, q0 + 32) - 1) / kKeyBlock + 1 : 0;
+  }
+  // the records of tiles [t, t + KS); tiles past the end repeat the last one (no iteration reads them)
+  const auto copy = [&](char* stage, int t) {
+    const uint32_t base = lds_address(stage);
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      const int piece = wave + 4 * r;
+      if (piece < kPieces) {
+        const int tile = min(t + piece / L::kPieces, tiles - 1);
+        const char* src = reinterpret_cast<const char*>(p.kv_tiles) +
+                          (static_cast<long>(bh) * p.nkb + tile) * L::kStageBytes + piece % L::kPieces * 1024;
+        copy_piece(src, lane * 16, base + piece * 1024);
+      }
+    }
+  };
+
+  v4i qf[kChunksD];
+  float cq = 0.0f;
+  v4i raw[D / 16];
+  const bool fused_live = p.fused_query && wave_live;
+  if (fused_live) issue_query_loads<D>(p, bh, q0, n, h, raw);
+  if (!p.fused_query && q0 < p.sq32) {
+    const int8_t* qrow = p.query_code + (static_cast<long>(bh) * p.sq32 + q0 + n) * D + 16 * h;
+#pragma unroll
+    for (int c = 0; c < kChunksD; ++c) qf[c] = *reinterpret_cast<const v4i*>(qrow + 32 * c);
+    cq = p.query_scale[(static_cast<long>(bh) * p.nqb + (q0 >> 5)) * kQueryScaleSlots + (kPerThread ? (n & 7) : 0)] *
+         p.score_multiplier;
+    // settled inside this branch, as in attention_kernel
+#pragma unroll
+    for (int c = 0; c < kChunksD; ++c) asm volatile("" ::"v"(qf[c]));
+    asm volatile("" ::"v"(cq));
+  } else {
+#pragma unroll
+    for (int c = 0; c < kChunksD; ++c) qf[c] = v4i{0, 0, 0, 0};
+  }
+  copy(smem, 0);
+  if (fused_live) {
+    // wait for the query loads only: this wave issued kRounds or kRounds - 1 copies after them
+    if (wave < kPieces - 4 * (kRounds - 1))
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRounds) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRounds - 1) : "memory");
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) asm volatile("" : "+v"(raw[i]));
+    cq = quantize_query_block<D, kPerThread>(p, q0, n, raw, qf) * p.score_multiplier;
+  }
+
+  float num[kChunksD][16];
+#pragma unroll
+  for (int j = 0; j < kChunksD; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) num[j][r] = 0.0f;
+  float den[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  float mref = -__builtin_inff();
+  float mlim = -__builtin_inff();
+  float kref = 0.0f;
+  const int krow = 16 * ((n >> 2) & 1) + 4 * (n >> 3) + (n & 3);
+  const uint32_t sel = code_selector();
+
+  const int steps = (tiles + KS - 1) / KS;
+  for (int i = 0; i < steps; ++i) {
+    stage_barrier<0>();  // this iteration's records landed, every read of the last one's is done
+    if (i + 1 < steps) copy(smem + ((i + 1) & 1) * kStage, KS * (i + 1));
+    const int t = KS * i + part;
+    if (t < wave_tiles) {
+      const char* stage = smem + (i & 1) * kStage + part * L::kStageBytes;
+      v16i sc[2];
+      block_scores<D, L>(stage, qf, h, krow, sc);
+      float ct[4];
+      if constexpr (kPerThread) {
+        const float4 ks = *reinterpret_cast<const float4*>(stage + D);
+        ct[0] = cq * ks.x;
+        ct[1] = cq * ks.y;
+        ct[2] = cq * ks.z;
+        ct[3] = cq * ks.w;
+      } else {
+        ct[0] = ct[1] = ct[2] = ct[3] = cq * *reinterpret_cast<const float*>(stage + D);
+      }
+      block_update<D, 4, kCausal>(stage, sc, ct, t, q0, n, h, sel, num, den, mref, mlim, kref);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const float den_total = cross_half_sum((den[0] + den[1]) + (den[2] + den[3]));
+  __syncthreads();  // every wave is done with the stages
+
+  // every wave's sums: [wave][four-feature group][lane] float4, then [wave][lane] float2 (den, mref)
+  float4* sums = reinterpret_cast<float4*>(smem);
+  float2* stats = reinterpret_cast<float2*>(smem + 4 * D * 32 * 4);
+#pragma unroll
+  for (int j = 0; j < kChunksD; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      sums[(wave * 4 * kChunksD + 4 * j + g) * 64 + lane] =
+          make_float4(num[j][4 * g + 0], num[j][4 * g + 1], num[j][4 * g + 2], num[j][4 * g + 3]);
+  stats[wave * 64 + lane] = make_float2(den_total, mref);
+  __syncthreads();
+  const int query = q0 + n;
+  if (!wave_live || query >= p.query_length) return;
+  float2 st[KS];
+  float top = -__builtin_inff();
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    st[k] = stats[(k * kGroups + group) * 64 + lane];
+    top = fmaxf(top, st[k].y);
+  }
+  float den_sum = 0.0f;
+  float weight[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    weight[k] = st[k].y == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(st[k].y - top);
+    den_sum = fmaf(st[k].x, weight[k], den_sum);
+  }
+  const float rden = (1.0f / 255.0f) / fmaxf(den_sum, 1e-30f);
+  const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
+#pragma unroll
+  for (int i = 0; i < kShare; ++i) {
+    const int four = part * kShare + i;  // this wave's share of the features: 4 j + g
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const float4 v = sums[((k * kGroups + group) * 4 * kChunksD + four) * 64 + lane];
+      acc.x = fmaf(v.x, weight[k], acc.x);
+      acc.y = fmaf(v.y, weight[k], acc.y);
+      acc.z = fmaf(v.z, weight[k], acc.z);
+      acc.w = fmaf(v.w, weight[k], acc.w);
+    }
+    const int d0 = 8 * four + 4 * h;  // 32 j + 8 g + 4 h
+    float4 m = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (!kCausal) m = *reinterpret_cast<const float4*>(p.value_mean + static_cast<long>(bh) * D + d0);
+    store4<kOut>(p.output, out_row + d0, fmaf(acc.x, rden, m.x), fmaf(acc.y, rden, m.y), fmaf(acc.z, rden, m.z),
+                 fmaf(acc.w, rden, m.w));
+  }
+}
+
 // The work-queue plan: a persistent grid (at most waves_per_simd(D) workgroups per CU) whose workgroups take
 // query tiles from one queue per XCC instead of waiting for the hardware to dispatch them.  The
 // hardware deals workgroups round-robin over the XCCs in id order, so a workgroup that cannot be
@@ -705,9 +879,25 @@ __global__ void __launch_bounds__(256) attention_merge_kernel(const AttnParams p
                fmaf(acc.w, rden, m.w));
 }
 
+template <int D, bool kCausal, bool kPerThread, int KS>
+static hipError_t launch_streams(int out_dtype, const AttnParams& ap, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(ap.query_tiles * ap.batch_heads));
+  const dim3 block(256);
+  switch (out_dtype) {
+    case 0: hipLaunchKernelGGL((attention_streams_kernel<D, kCausal, 0, kPerThread, KS>), grid, block, 0, stream, ap); break;
+    case 1: hipLaunchKernelGGL((attention_streams_kernel<D, kCausal, 1, kPerThread, KS>), grid, block, 0, stream, ap); break;
+    default: hipLaunchKernelGGL((attention_streams_kernel<D, kCausal, 2, kPerThread, KS>), grid, block, 0, stream, ap); break;
+  }
+  return hipGetLastError();
+}
+
 template <int D, bool kCausal, bool kPerThread>
 static hipError_t launch_w3(int out_dtype, const AttnParams& ap, hipStream_t stream) {
   const dim3 block(256);
+  if constexpr (!kCausal) {
+    if (ap.key_streams == 2) return launch_streams<D, kCausal, kPerThread, 2>(out_dtype, ap, stream);
+    if (ap.key_streams == 4) return launch_streams<D, kCausal, kPerThread, 4>(out_dtype, ap, stream);
+  }
   if (ap.queue_xccs > 0) {
     hipLaunchKernelGGL(queue_init_kernel, dim3(1), dim3(64), 0, stream, ap.queue, ap.queue_xccs,
                        ap.query_tiles * ap.batch_heads, ap.queue_workers);

@@ -67,6 +67,17 @@ constexpr int sage_tile_bytes(int head_dim) {
 // SageAttention2++ 210 -> 197 us.
 constexpr int waves_per_simd(int head_dim) { return head_dim == 64 ? 4 : 3; }
 
+// Workgroups of attention_streams_kernel resident per CU: two double-buffered sets of KS tile records each
+// (D = 128: 80 or 160 KiB of the CU's 160; D = 64: 44 or 88).  A key split of 2 or 4 parts takes that kernel
+// when its grid then fits the GPU at once; beyond, the workgroups would queue and the parts' partial sums
+// cost less than reading the records again for fewer queries.  Unsplit, parts, streams (us, 10-13 of them
+// the launching loop's floor): B1 H8 S1024 D64 22.4, 17.7, 13.9 (4); B1 H24 S1024 D64 22.7, 25.8, 18.4
+// (2); B1 H16 S1024 D128 30.2, 30.2, 20.4 (2); B1 H16 S2048 53.6, 52.5, 44.7 (2); B2 H12 Sq1000 Sk333 16.6,
+// 27.1, 15.6 (2); B1 H4 Sq512 Sk2048 52.4, 23.5, 24.6 (4).
+constexpr int stream_workgroups(int head_dim, int streams) {
+  return streams == 4 ? 1 : head_dim == 64 ? 3 : 2;
+}
+
 struct InputTensor {
   const void* data;  // 16-bit floats; the head_dim axis is contiguous
   long stride_batch;  // element strides
@@ -182,6 +193,8 @@ struct AttnParams {
   int whole_tiles;
   long split_row0;
   float* partials;
+  // Key streams (attention_streams_kernel): 2 or 4 waves of a workgroup share its queries; 1: none.
+  int key_streams;
   // Work-queue plan (three workgroups per CU, no key-range split): a persistent grid takes query
   // tiles from queue_xccs queues of consecutive logical ids, counters in `queue` (zero before the
   // launch).  queue_xccs = 0: the hardware dispatches one workgroup per query tile.

@@ -187,6 +187,11 @@ def heuristic_plan(batch: int, heads: int, query_length: int) -> MI355XPlan:
 _TILE_US = {128: (1.5, 1.75, 2.5), 64: (1.2, 1.4, 1.8, 2.3)}
 _PARTIAL_BYTES_PER_US = 4e6
 _MERGE_US = 2.2
+# Two or four parts of a grid that then still fits the GPU at once run as key streams of one workgroup
+# (csrc/kernels.h stream_workgroups): microseconds per step of `parts` key tiles when 1, 2, ... workgroups
+# share a CU, and the merge in LDS.
+_STREAM_US = {128: {2: (1.9, 2.4), 4: (2.5,)}, 64: {2: (1.5, 1.7, 2.2), 4: (1.5,)}}
+_STREAM_MERGE_US = 1.0
 
 
 def _tile_us(head_dim: int) -> tuple[float, ...]:
@@ -197,6 +202,9 @@ def _split_us(tiles: int, rows: int, key_tiles: int, parts: int, head_dim: int) 
     """Estimated time of a non-causal grid of `tiles` query tiles whose last, unfilled round of resident
     workgroups (`rows` query rows) is split into `parts` key ranges (csrc/kernels.h AttnParams)."""
     steps = _tile_us(head_dim)
+    streams = _STREAM_US[64 if head_dim == 64 else 128].get(parts)
+    if streams is not None and parts * tiles <= len(streams) * COMPUTE_UNITS:
+        return -(-key_tiles // parts) * streams[-(-parts * tiles // COMPUTE_UNITS) - 1] + _STREAM_MERGE_US
     slots = len(steps) * COMPUTE_UNITS
     whole, rest = divmod(tiles, slots)
     part_rounds, part_rest = divmod(rest * parts, slots)
@@ -214,8 +222,9 @@ def split_parts(batch: int, heads: int, query_length: int, key_length: int, head
     """Key parts for an untuned non-causal shape (1: no split): what ``_split_us`` finds fastest, if that
     gains 5% of the whole grid's time.  Small grids split to give every SIMD more waves, larger ones
     only the query tiles beyond whole rounds of resident workgroups.  Measured, unsplit against split: c1
-    (64 tiles of 16 key tiles) 22.4 -> 16.7 us in 4 parts; B1 H24 Sq256 Sk16384 (48 tiles of 256) 371 ->
-    74 us in 8 (105 in 4); B2 H12 Sq1000 Sk333 (192 tiles of 6) stays whole: 16.4 against 28.4 us in 2."""
+    (64 tiles of 16 key tiles) 22.4 -> 13.9 us in 4 streams (17.7 in 4 parts); B1 H16 S2048 D128 (256 tiles
+    of 32) 53.6 -> 44.7 in 2 streams; B1 H24 Sq256 Sk16384 (48 tiles of 256) 371 -> 74 us in 8 parts (105 in
+    4); B1 H28 S5000 (1120 tiles) 352 -> 331, the last round in 2 parts."""
     block_m = MI355XPlan(waves=4, three_per_cu=True).block_m
     tiles = batch * heads * (-(-query_length // block_m))
     key_tiles = -(-key_length // KEY_BLOCK)

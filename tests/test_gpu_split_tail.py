@@ -48,4 +48,7 @@ def test_the_rule_splits_only_partial_rounds_into_whole_key_tiles() -> None:
         assert 1 <= parts <= MAX_KEY_PARTS and (parts == 1 or 2 * parts <= -(-sk // 64))
     for d, tiles in ((128, 768), (128, 1536), (64, 1024)):  # whole rounds
         assert split_parts(1, 1, 128 * tiles, 4096, d) == 1
-    assert split_parts(1, 24, 256, 16384, 128) == 8 and split_parts(2, 12, 1000, 333, 128) == 1
+    assert split_parts(1, 24, 256, 16384, 128) == 8
+    # 192 query tiles still fit the GPU as two key streams each; 320 do not, and six key tiles are too few
+    # for partial sums
+    assert split_parts(2, 12, 1000, 333, 128) == 2 and split_parts(1, 40, 1000, 333, 128) == 1
