@@ -380,11 +380,21 @@ int piper_attention_workspace_bytes(const piper_shape* shape, int32_t plan, int6
 /* The same with the query quantised inside the kernel (see piper_attention_fused_args). */
 int piper_attention_forward_fused(const piper_attention_fused_args* args, void* stream);
 
+/* piper_attention_forward_fused, free to run a small causal grid as key streams: the waves of a workgroup
+ * share its query rows, each takes every second or fourth key tile, and their FP32 sums are added at
+ * the end.  Results equal piper_attention_forward_fused's to rounding, not bit for bit, and depend on
+ * the number of batch-heads (the grid) in that rounding.  What the custom op calls. */
+int piper_attention_forward_balanced(const piper_attention_fused_args* args, void* stream);
+
 /* SageAttention2++: buffer sizes, K/V prep (statistics, INT8 K, FP8 V^T tile records) and the
  * fused attention kernel (INT8 QK, FP8 PV on v_mfma_f32_32x32x64_f8f6f4, FP32 accumulation). */
 int piper_sage_prepared_layout(const piper_shape* shape, piper_sage_layout* layout);
 int piper_sage_prepare(const piper_sage_prepare_args* args, void* stream);
 int piper_sage_attention_forward(const piper_sage_attention_args* args, void* stream);
+
+/* The same, free to run a small grid as key streams (piper_attention_forward_balanced): every probability
+ * code is the other entry point's, the FP32 sums are added in another order. */
+int piper_sage_attention_forward_balanced(const piper_sage_attention_args* args, void* stream);
 
 /* Thread-local description of the last failure on this thread ("" if none). */
 const char* piper_last_error(void);

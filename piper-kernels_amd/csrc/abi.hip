@@ -134,7 +134,7 @@ piper::InputTensor to_input(const piper_tensor& t) {
 int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_causal, int32_t plan, int32_t flags,
                           const piper_shape& s, float scale, const piper_prepared& o, void* output,
                           const piper_tensor* query, int32_t query_dtype, void* workspace, int64_t workspace_bytes,
-                          void* stream) {
+                          bool balanced, void* stream) {
   if (abi_version != PIPER_ABI_VERSION)
     return fail(PIPER_ERROR_INVALID_ARGUMENT, "ABI version mismatch: caller %d, library %d", abi_version,
                 PIPER_ABI_VERSION);
@@ -236,6 +236,12 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
       ap.key_streams = key_parts;
       ap.query_tiles = static_cast<int>(ceil_div(s.query_length, block_m / key_parts));
     }
+  }
+  if (balanced && is_causal && waves == 3 && !work_queue) {
+    int cus = 0, xccs = 0;
+    if (int st = device_topology(&cus, &xccs)) return st;
+    ap.key_streams = piper::small_grid_streams(false, true, static_cast<long>(ap.query_tiles) * ap.batch_heads, ap.nkb, cus);
+    ap.query_tiles = static_cast<int>(ceil_div(s.query_length, block_m / ap.key_streams));
   }
   if (static_cast<int64_t>(ap.query_tiles) * ap.batch_heads * ap.key_parts > 0x7fffffff)
     return fail(PIPER_ERROR_UNSUPPORTED, "too many workgroups");
@@ -420,7 +426,7 @@ int piper_prepare_status(const piper_shape* shape, const void* workspace, uint32
 int piper_attention_forward(const piper_attention_args* a, void* stream) {
   if (a == nullptr) return fail(PIPER_ERROR_INVALID_ARGUMENT, "args is NULL");
   return launch_attention_call(a->abi_version, a->output_dtype, a->is_causal, a->plan, a->flags, a->shape,
-                               a->scale, a->prepared, a->output, nullptr, 0, a->workspace, a->workspace_bytes, stream);
+                               a->scale, a->prepared, a->output, nullptr, 0, a->workspace, a->workspace_bytes, false, stream);
 }
 
 int piper_attention_workspace_bytes(const piper_shape* shape, int32_t plan, int64_t* bytes) {
@@ -435,12 +441,16 @@ int piper_attention_workspace_bytes(const piper_shape* shape, int32_t plan, int6
   return PIPER_OK;
 }
 
-int piper_attention_forward_fused(const piper_attention_fused_args* a, void* stream) {
+static int fused_call(const piper_attention_fused_args* a, bool balanced, void* stream) {
   if (a == nullptr) return fail(PIPER_ERROR_INVALID_ARGUMENT, "args is NULL");
   return launch_attention_call(a->abi_version, a->output_dtype, a->is_causal, a->plan, a->flags, a->shape,
                                a->scale, a->prepared, a->output, &a->query, a->dtype, a->workspace,
-                               a->workspace_bytes, stream);
+                               a->workspace_bytes, balanced, stream);
 }
+
+int piper_attention_forward_fused(const piper_attention_fused_args* a, void* stream) { return fused_call(a, false, stream); }
+
+int piper_attention_forward_balanced(const piper_attention_fused_args* a, void* stream) { return fused_call(a, true, stream); }
 
 int piper_sage_prepared_layout(const piper_shape* shape, piper_sage_layout* layout) {
   if (int st = check_shape(shape)) return st;
@@ -526,7 +536,7 @@ int piper_sage_prepare(const piper_sage_prepare_args* a, void* stream) {
   return PIPER_OK;
 }
 
-int piper_sage_attention_forward(const piper_sage_attention_args* a, void* stream) {
+static int sage_attention_call(const piper_sage_attention_args* a, bool balanced, void* stream) {
   if (a == nullptr) return fail(PIPER_ERROR_INVALID_ARGUMENT, "args is NULL");
   if (a->abi_version != PIPER_ABI_VERSION)
     return fail(PIPER_ERROR_INVALID_ARGUMENT, "ABI version mismatch: caller %d, library %d", a->abi_version,
@@ -575,6 +585,14 @@ int piper_sage_attention_forward(const piper_sage_attention_args* a, void* strea
                     piper::order_across_heads(sp.batch_heads, sp.nkb, piper::sage_tile_bytes(static_cast<int>(s.head_dim)));
   sp.per_thread = (a->flags & PIPER_ATTENTION_QK_PER_THREAD) ? 1 : 0;
   sp.fp16_partials = (a->flags & PIPER_SAGE_FP16_PARTIALS) ? 1 : 0;
+  sp.key_streams = 1;
+  if (balanced && waves == 3 && !sp.fp16_partials) {
+    int cus = 0, xccs = 0;
+    if (int st = device_topology(&cus, &xccs)) return st;
+    sp.key_streams = piper::small_grid_streams(true, a->is_causal != 0, static_cast<long>(sp.query_tiles) * sp.batch_heads,
+                                               sp.nkb, cus);
+    sp.query_tiles = static_cast<int>(ceil_div(s.query_length, 128 / sp.key_streams));
+  }
   if (static_cast<int64_t>(sp.query_tiles) * sp.batch_heads > 0x7fffffff)
     return fail(PIPER_ERROR_UNSUPPORTED, "too many workgroups");
 
@@ -583,6 +601,14 @@ int piper_sage_attention_forward(const piper_sage_attention_args* a, void* strea
   if (err != hipSuccess) return fail(PIPER_ERROR_HIP, "attention launch failed: %s", hipGetErrorString(err));
   g_last_error[0] = '\0';
   return PIPER_OK;
+}
+
+int piper_sage_attention_forward(const piper_sage_attention_args* a, void* stream) {
+  return sage_attention_call(a, false, stream);
+}
+
+int piper_sage_attention_forward_balanced(const piper_sage_attention_args* a, void* stream) {
+  return sage_attention_call(a, true, stream);
 }
 
 }  // extern "C"

@@ -599,8 +599,7 @@ attention_streams_kernel(const AttnParams p) {
   constexpr int kChunksD = D / 32;
   constexpr int kGroups = 4 / KS;               // query groups of a workgroup
   constexpr int kStage = KS * L::kStageBytes;
-  constexpr int kPieces = KS * L::kPieces;      // 1 KiB pieces of an iteration's records
-  constexpr int kRounds = (kPieces + 3) / 4;
+  constexpr int kRounds = stream_rounds<L, KS>();
   constexpr int kShare = 4 * kChunksD / KS;     // four-feature groups that a wave writes at the end
   __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
   static_assert(4 * (D * 32 * 4 + 512) <= 2 * kStage, "every wave's sums fit the stages");
@@ -623,21 +622,6 @@ attention_streams_kernel(const AttnParams p) {
     tiles = (min(p.query_length, (qtile + 1) * kGroups * 32) - 1) / kKeyBlock + 1;
     wave_tiles = wave_live ? (min(p.query_length, q0 + 32) - 1) / kKeyBlock + 1 : 0;
   }
-  // the records of tiles [t, t + KS); tiles past the end repeat the last one (no iteration reads them)
-  const auto copy = [&](char* stage, int t) {
-    const uint32_t base = lds_address(stage);
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      const int piece = wave + 4 * r;
-      if (piece < kPieces) {
-        const int tile = min(t + piece / L::kPieces, tiles - 1);
-        const char* src = reinterpret_cast<const char*>(p.kv_tiles) +
-                          (static_cast<long>(bh) * p.nkb + tile) * L::kStageBytes + piece % L::kPieces * 1024;
-        copy_piece(src, lane * 16, base + piece * 1024);
-      }
-    }
-  };
-
   v4i qf[kChunksD];
   float cq = 0.0f;
   v4i raw[D / 16];
@@ -657,10 +641,10 @@ attention_streams_kernel(const AttnParams p) {
 #pragma unroll
     for (int c = 0; c < kChunksD; ++c) qf[c] = v4i{0, 0, 0, 0};
   }
-  copy(smem, 0);
+  copy_tiles<L, KS>(p, smem, bh, 0, tiles, wave, lane);
   if (fused_live) {
     // wait for the query loads only: this wave issued kRounds or kRounds - 1 copies after them
-    if (wave < kPieces - 4 * (kRounds - 1))
+    if (wave < stream_full_waves<L, KS>())
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRounds) : "memory");
     else
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRounds - 1) : "memory");
@@ -684,7 +668,7 @@ attention_streams_kernel(const AttnParams p) {
   const int steps = (tiles + KS - 1) / KS;
   for (int i = 0; i < steps; ++i) {
     stage_barrier<0>();  // this iteration's records landed, every read of the last one's is done
-    if (i + 1 < steps) copy(smem + ((i + 1) & 1) * kStage, KS * (i + 1));
+    if (i + 1 < steps) copy_tiles<L, KS>(p, smem + ((i + 1) & 1) * kStage, bh, KS * (i + 1), tiles, wave, lane);
     const int t = KS * i + part;
     if (t < wave_tiles) {
       const char* stage = smem + (i & 1) * kStage + part * L::kStageBytes;
@@ -894,10 +878,8 @@ static hipError_t launch_streams(int out_dtype, const AttnParams& ap, hipStream_
 template <int D, bool kCausal, bool kPerThread>
 static hipError_t launch_w3(int out_dtype, const AttnParams& ap, hipStream_t stream) {
   const dim3 block(256);
-  if constexpr (!kCausal) {
-    if (ap.key_streams == 2) return launch_streams<D, kCausal, kPerThread, 2>(out_dtype, ap, stream);
-    if (ap.key_streams == 4) return launch_streams<D, kCausal, kPerThread, 4>(out_dtype, ap, stream);
-  }
+  if (ap.key_streams == 2) return launch_streams<D, kCausal, kPerThread, 2>(out_dtype, ap, stream);
+  if (ap.key_streams == 4) return launch_streams<D, kCausal, kPerThread, 4>(out_dtype, ap, stream);
   if (ap.queue_xccs > 0) {
     hipLaunchKernelGGL(queue_init_kernel, dim3(1), dim3(64), 0, stream, ap.queue, ap.queue_xccs,
                        ap.query_tiles * ap.batch_heads, ap.queue_workers);

@@ -78,6 +78,24 @@ constexpr int stream_workgroups(int head_dim, int streams) {
   return streams == 4 ? 1 : head_dim == 64 ? 3 : 2;
 }
 
+// Key streams of a grid whose plan does not choose them (causal Piper Attention, SageAttention2++), from its
+// 128-row query tiles and 64-key tiles: four where that gives at most one workgroup per CU, two where that
+// does, and two for causal grids of up to two (SageAttention2++ one) workgroups of 128 rows per CU, whose
+// longest tile sets the time, if the keys are long enough to pay for the shorter query tiles' prologues.
+// SageAttention2++'s iterations exchange their maxima, and beyond 4096 keys a row's rounding should not
+// depend on the batch: no streams there.  Measured, none against the choice (us, 10-13 of them the launching
+// loop's floor): Piper Attention causal B1 H8 S1024 D64 21.9, 11.3 (4); B2 H16 S1531 D128 42.4, 34.5 (2); B1
+// H12 S4096 98.8, 67.9 (2); B1 H8 S8192 198, 162 (2); on the other side of the line B1 H24 S4096 (768
+// tiles) 114, two streams 129, and B4 H32 S512 (512 tiles of 8) 21.5, 26.3.  SageAttention2++ B1 H8 S1024
+// D64 18.2, 11.1 (4); B1 H16 S1024 D128 24.3, 19.7 (2); causal B1 H16 S2048 43.1, 34.3 (2); not taken: B1 H16
+// S2048 42.9, 45.1, causal B2 H16 S1531 36.8, 38.8.
+inline int small_grid_streams(bool sage, bool causal, long tiles, int key_tiles, int cus) {
+  if (key_tiles < 4 || (sage && key_tiles > 64)) return 1;
+  if (4 * tiles <= cus) return 4;
+  if (2 * tiles <= cus) return 2;
+  return causal && key_tiles >= 16 && tiles <= (sage ? 1L : 2L) * cus ? 2 : 1;
+}
+
 struct InputTensor {
   const void* data;  // 16-bit floats; the head_dim axis is contiguous
   long stride_batch;  // element strides
@@ -234,6 +252,7 @@ struct SageParams {
   int xcd_remap;
   int across_heads;
   int per_thread;  // Q/K scales per thread group (the tile's four K slots, per-row-group Q scales)
+  int key_streams;  // sage_streams_kernel: 2 or 4 waves of a workgroup share its queries; 1: none
   int fp16_partials;  // round each block's FP8 product to FP16 (the reference's arithmetic)
 };
 

@@ -45,18 +45,16 @@ struct SageLayout : StagePieces<sage_tile_bytes(D), NW> {  // the tile record is
 };
 
 // Online softmax and PV of one 64-key block (block index t, staged at `stage`) for one wave,
-// in two parts.  Head: raw scores, masks, block maximum and the frame move (rescale of the
-// accumulators when the running maximum grows; exact, otherwise the weight is 1).  Tail:
+// in three parts.  Scores: raw scores, masks and the block maximum.  Frame: the accumulators move to the
+// frame `next` (rescaled when the running maximum grows; exact, otherwise the weight is 1).  Tail:
 // probabilities, denominator share, FP8 codes and the PV MFMAs.  ct[g] = query scale * key scale
 // * softmax scale * log2 e for the keys of K thread group g (keys k with (k % 8) / 2 == g; all
 // four equal for per-block K scales); register 4q + i holds key 16h + 4q + i (or 32 + ...), so
 // it belongs to group 2 (q % 2) + i / 2.  mrun is the running maximum (log2 units, per query),
 // den this lane half's share of the denominator; x carries the raw scores from head to tail.
-template <int D, bool kCausal, bool kPerThread>
-__device__ __forceinline__ void sage_block_head(const v16i (&s)[2], const float (&ct)[4], int t, int q0, int n,
-                                                int h, int key_length, float (&x)[32], v16f (&acc)[D / 32],
-                                                float& den, float& mrun) {
-  constexpr int kChunksD = D / 32;
+template <bool kCausal, bool kPerThread>
+__device__ __forceinline__ float sage_block_raw(const v16i (&s)[2], const float (&ct)[4], int t, int q0, int n, int h,
+                                                int key_length, float (&x)[32]) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     x[r] = unbias_score(s[0][r]);
@@ -87,7 +85,6 @@ __device__ __forceinline__ void sage_block_head(const v16i (&s)[2], const float 
   }
   // ct > 0, so the maximum commutes with the scaling: max(RN(x ct)) = RN(max(x) ct) -- per K
   // thread group when the groups have their own scales
-  float block_max;
   if constexpr (kPerThread) {
     float gmax[4];
 #pragma unroll
@@ -96,12 +93,15 @@ __device__ __forceinline__ void sage_block_head(const v16i (&s)[2], const float 
       gmax[g] = cross_half_max(fmaxf(fmaxf(fmaxf(x[r], x[r + 1]), fmaxf(x[r + 8], x[r + 9])),
                                      fmaxf(fmaxf(x[16 + r], x[17 + r]), fmaxf(x[24 + r], x[25 + r]))));
     }
-    block_max = fmaxf(fmaxf(gmax[0] * ct[0], gmax[1] * ct[1]), fmaxf(gmax[2] * ct[2], gmax[3] * ct[3])) -
-                kLog2Of448;
+    return fmaxf(fmaxf(gmax[0] * ct[0], gmax[1] * ct[1]), fmaxf(gmax[2] * ct[2], gmax[3] * ct[3])) - kLog2Of448;
   } else {
-    block_max = cross_half_max(max32(x)) * ct[0] - kLog2Of448;
+    return cross_half_max(max32(x)) * ct[0] - kLog2Of448;
   }
-  const float next = fmaxf(mrun, block_max);
+}
+
+template <int D>
+__device__ __forceinline__ void sage_frame(float next, v16f (&acc)[D / 32], float& den, float& mrun) {
+  constexpr int kChunksD = D / 32;
   const bool grow = next > mrun;
   if (__builtin_amdgcn_ballot_w64(grow) != 0) {
     const float w = grow ? __builtin_amdgcn_exp2f(mrun - next) : 1.0f;  // exp2(-inf) = 0 at the start
@@ -112,6 +112,14 @@ __device__ __forceinline__ void sage_block_head(const v16i (&s)[2], const float 
     den *= w;
     mrun = next;
   }
+}
+
+template <int D, bool kCausal, bool kPerThread>
+__device__ __forceinline__ void sage_block_head(const v16i (&s)[2], const float (&ct)[4], int t, int q0, int n,
+                                                int h, int key_length, float (&x)[32], v16f (&acc)[D / 32],
+                                                float& den, float& mrun) {
+  const float block_max = sage_block_raw<kCausal, kPerThread>(s, ct, t, q0, n, h, key_length, x);
+  sage_frame<D>(fmaxf(mrun, block_max), acc, den, mrun);
 }
 
 template <int D, int NW, bool kFp16Partials>
@@ -390,10 +398,176 @@ sage_attention_w3_kernel(const SageParams p) {
   }
 }
 
+// Key streams, as Piper Attention's attention_streams_kernel: KS waves of a workgroup share 32 queries and
+// take every KS-th key tile each.  FP8 probabilities round relative to the running maximum, so the waves
+// exchange their block maxima in every iteration (one more barrier) and each tile gets the frame that the
+// sequential kernel gives it, max over the tiles up to it: every probability code is the sequential
+// kernel's, and only the FP32 sums are added in another order.
+template <int D, bool kCausal, int kOut, bool kPerThread, int KS>
+__global__ void __attribute__((amdgpu_flat_work_group_size(256, KS == 4 ? 512 : 256), amdgpu_waves_per_eu(KS == 4 ? 2 : stream_workgroups(D, KS), KS == 4 ? 2 : stream_workgroups(D, KS))))
+sage_streams_kernel(const SageParams p) {
+  using L = SageLayout<D, 4>;
+  constexpr int kChunksD = D / 32;
+  constexpr int kGroups = 4 / KS;
+  constexpr int kStage = KS * L::kStageBytes;
+  constexpr int kRounds = stream_rounds<L, KS>();
+  constexpr int kShare = 4 * kChunksD / KS;  // four-feature groups that a wave writes at the end
+  __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
+  __shared__ float maxima[4][32];  // [wave][query]: the iteration's block maxima
+  static_assert(4 * (D * 32 * 4 + 512) <= 2 * kStage, "every wave's sums fit the stages");
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5;
+  const int n = lane & 31;
+  const TileCoord tc = workgroup_tile<kCausal>(p);
+  const int bh = __builtin_amdgcn_readfirstlane(tc.bh);
+  const int qtile = __builtin_amdgcn_readfirstlane(tc.qtile);
+  const int group = wave % kGroups;
+  const int part = wave / kGroups;
+  const int q0 = qtile * (kGroups * 32) + group * 32;
+  const bool wave_live = q0 < p.query_length;
+
+  int tiles = p.nkb;
+  int wave_tiles = wave_live ? p.nkb : 0;
+  if constexpr (kCausal) {
+    tiles = (min(p.query_length, (qtile + 1) * kGroups * 32) - 1) / kKeyBlock + 1;
+    wave_tiles = wave_live ? (min(p.query_length, q0 + 32) - 1) / kKeyBlock + 1 : 0;
+  }
+
+  v4i raw[D / 16];
+  if (wave_live) issue_query_loads<D>(p, bh, q0, n, h, raw);
+  copy_tiles<L, KS>(p, smem, bh, 0, tiles, wave, lane);
+  v4i qf[kChunksD];
+  float cq = 0.0f;
+  if (wave_live) {
+    // wait for the query loads only: this wave issued kRounds or kRounds - 1 copies after them
+    if (wave < stream_full_waves<L, KS>())
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRounds) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRounds - 1) : "memory");
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) asm volatile("" : "+v"(raw[i]));
+    cq = quantize_query_block<D, kPerThread>(p, q0, n, raw, qf) * (p.scale_log2e * kScoreUnit);
+  } else {
+#pragma unroll
+    for (int c = 0; c < kChunksD; ++c) qf[c] = v4i{0, 0, 0, 0};
+  }
+
+  v16f acc[kChunksD];
+#pragma unroll
+  for (int j = 0; j < kChunksD; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+  float den = 0.0f;
+  float mrun = -__builtin_inff();  // the frame of this wave's sums
+  float seen = -__builtin_inff();  // the running maximum over every tile of the iterations before
+  const int krow = 16 * ((n >> 2) & 1) + 4 * (n >> 3) + (n & 3);
+
+  const int steps = (tiles + KS - 1) / KS;
+  for (int i = 0; i < steps; ++i) {
+    stage_barrier<0>();  // this iteration's records landed, every read of the last one's (and of maxima) is done
+    if (i + 1 < steps) copy_tiles<L, KS>(p, smem + ((i + 1) & 1) * kStage, bh, KS * (i + 1), tiles, wave, lane);
+    const int t = KS * i + part;
+    const char* stage = smem + (i & 1) * kStage + part * L::kStageBytes;
+    float ct[4];
+    float x[32];
+    float block_max = -__builtin_inff();
+    if (t < wave_tiles) {
+      v16i sc[2];
+      block_scores<D, L>(stage, qf, h, krow, sc);
+      if constexpr (kPerThread) {
+        const float4 ks = *reinterpret_cast<const float4*>(stage + D);
+        ct[0] = cq * ks.x;
+        ct[1] = cq * ks.y;
+        ct[2] = cq * ks.z;
+        ct[3] = cq * ks.w;
+      } else {
+        ct[0] = ct[1] = ct[2] = ct[3] = cq * *reinterpret_cast<const float*>(stage + D);
+      }
+      block_max = sage_block_raw<kCausal, kPerThread>(sc, ct, t, q0, n, h, p.key_length, x);
+    }
+    if (h == 0) maxima[wave][n] = block_max;  // both lane halves hold it
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float frame = seen;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const float m = maxima[k * kGroups + group][n];
+      seen = fmaxf(seen, m);
+      if (k <= part) frame = seen;
+    }
+    if (t < wave_tiles) {
+      sage_frame<D>(frame, acc, den, mrun);
+      sage_block_tail<D, 4, false>(stage, x, ct, n, h, acc, den, mrun);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const float den_total = cross_half_sum(den);
+  __syncthreads();  // every wave is done with the stages
+
+  // every wave's sums: [wave][four-feature group][lane] float4, then [wave][lane] float2 (den, frame)
+  float4* sums = reinterpret_cast<float4*>(smem);
+  float2* stats = reinterpret_cast<float2*>(smem + 4 * D * 32 * 4);
+#pragma unroll
+  for (int j = 0; j < kChunksD; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      sums[(wave * 4 * kChunksD + 4 * j + g) * 64 + lane] =
+          make_float4(acc[j][4 * g + 0], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]);
+  stats[wave * 64 + lane] = make_float2(den_total, mrun);
+  __syncthreads();
+  const int query = q0 + n;
+  if (!wave_live || query >= p.query_length) return;
+  float total = 0.0f;
+  float weight[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    const float2 st = stats[(k * kGroups + group) * 64 + lane];
+    weight[k] = st.y == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(st.y - seen);
+    total = fmaf(st.x, weight[k], total);
+  }
+  const float rden = 1.0f / fmaxf(total, 1e-30f);
+  const float* vscale = p.value_scale + static_cast<long>(bh) * D;
+  const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
+#pragma unroll
+  for (int i = 0; i < kShare; ++i) {
+    const int four = part * kShare + i;  // this wave's share of the features: 4 j + g
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const float4 v = sums[((k * kGroups + group) * 4 * kChunksD + four) * 64 + lane];
+      sum.x = fmaf(v.x, weight[k], sum.x);
+      sum.y = fmaf(v.y, weight[k], sum.y);
+      sum.z = fmaf(v.z, weight[k], sum.z);
+      sum.w = fmaf(v.w, weight[k], sum.w);
+    }
+    const int d0 = 8 * four + 4 * h;  // 32 j + 8 g + 4 h
+    const float4 vs = *reinterpret_cast<const float4*>(vscale + d0);
+    store4<kOut>(p.output, out_row + d0, (sum.x * vs.x) * rden, (sum.y * vs.y) * rden, (sum.z * vs.z) * rden,
+                 (sum.w * vs.w) * rden);
+  }
+}
+
+template <int D, bool kCausal, bool kPerThread, int KS>
+static hipError_t sage_launch_streams(int out_dtype, const SageParams& sp, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(sp.query_tiles * sp.batch_heads));
+  const dim3 block(256);
+  switch (out_dtype) {
+    case 0: hipLaunchKernelGGL((sage_streams_kernel<D, kCausal, 0, kPerThread, KS>), grid, block, 0, stream, sp); break;
+    case 1: hipLaunchKernelGGL((sage_streams_kernel<D, kCausal, 1, kPerThread, KS>), grid, block, 0, stream, sp); break;
+    default: hipLaunchKernelGGL((sage_streams_kernel<D, kCausal, 2, kPerThread, KS>), grid, block, 0, stream, sp); break;
+  }
+  return hipGetLastError();
+}
+
 template <int D, int NW, bool kCausal, bool kPerThread, bool kFp16Partials>
 static hipError_t sage_launch_out(int out_dtype, const SageParams& sp, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(sp.query_tiles * sp.batch_heads));
   if constexpr (NW == 3) {  // three 4-wave workgroups per CU
+    if constexpr (!kFp16Partials) {
+      if (sp.key_streams == 2) return sage_launch_streams<D, kCausal, kPerThread, 2>(out_dtype, sp, stream);
+      if (sp.key_streams == 4) return sage_launch_streams<D, kCausal, kPerThread, 4>(out_dtype, sp, stream);
+    }
     const dim3 block(256);
     switch (out_dtype) {
       case 0:

@@ -132,6 +132,30 @@ __device__ __forceinline__ void copy_block(const Params& p, char* stage, int bh,
   }
 }
 
+// The records of tiles [t, t + KS) into one stage of KS records (the key-stream kernels' iterations; four
+// waves); tiles past `tiles` repeat the last one, which no iteration reads: every wave issues the same
+// number of copies whatever the tile (stream_rounds, one fewer from wave stream_full_waves on).
+template <class L, int KS>
+constexpr int stream_rounds() { return (KS * L::kPieces + 3) / 4; }
+template <class L, int KS>
+constexpr int stream_full_waves() { return KS * L::kPieces - 4 * (stream_rounds<L, KS>() - 1); }
+
+template <class L, int KS, class Params>
+__device__ __forceinline__ void copy_tiles(const Params& p, char* stage, int bh, int t, int tiles, int wave, int lane) {
+  static_assert(L::kWaves == 4, "four waves");
+  const uint32_t base = lds_address(stage);
+#pragma unroll
+  for (int r = 0; r < stream_rounds<L, KS>(); ++r) {
+    const int piece = wave + 4 * r;  // wave-uniform: scalar arithmetic and a scalar branch
+    if (piece < KS * L::kPieces) {
+      const int tile = min(t + piece / L::kPieces, tiles - 1);
+      const char* src = reinterpret_cast<const char*>(p.kv_tiles) +
+                        (static_cast<long>(bh) * p.nkb + tile) * L::kStageBytes + piece % L::kPieces * 1024;
+      copy_piece(src, lane * 16, base + piece * 1024);
+    }
+  }
+}
+
 // Workgroup barrier that lets this wave's newest kInFlight direct loads stay in flight.
 // (__syncthreads would drain every outstanding load.)  LDS reads are waited for as well, so
 // a stage is never overwritten under a pending read.

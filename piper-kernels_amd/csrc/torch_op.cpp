@@ -166,7 +166,7 @@ at::Tensor piper_attention(const at::Tensor& query, const at::Tensor& key, const
   a.output = call.output.mutable_data_ptr();
   a.workspace = attention_bytes > 0 ? base + attention : nullptr;
   a.workspace_bytes = attention_bytes;
-  check(piper_attention_forward_fused(&a, call.handle), "piper_attention_forward_fused");
+  check(piper_attention_forward_balanced(&a, call.handle), "piper_attention_forward_balanced");
   call.keep_inputs();
   return call.output;
 }
@@ -214,7 +214,7 @@ at::Tensor sage_attention_2pp(const at::Tensor& query, const at::Tensor& key, co
   a.query = tensor_arg(call.query);
   a.prepared = p.prepared;
   a.output = call.output.mutable_data_ptr();
-  check(piper_sage_attention_forward(&a, call.handle), "piper_sage_attention_forward");
+  check(piper_sage_attention_forward_balanced(&a, call.handle), "piper_sage_attention_forward_balanced");
   call.keep_inputs();
   return call.output;
 }

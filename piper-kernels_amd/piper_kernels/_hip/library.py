@@ -36,10 +36,12 @@ EXPORTED_SYMBOLS = (
     "piper_prepare_status",
     "piper_attention_forward",
     "piper_attention_forward_fused",
+    "piper_attention_forward_balanced",
     "piper_attention_workspace_bytes",
     "piper_sage_prepared_layout",
     "piper_sage_prepare",
     "piper_sage_attention_forward",
+    "piper_sage_attention_forward_balanced",
     "piper_last_error",
 )
 
@@ -244,6 +246,8 @@ class NativeLibrary:
         lib.piper_attention_forward.restype = ctypes.c_int
         lib.piper_attention_forward_fused.argtypes = [ctypes.POINTER(PiperAttentionFusedArgs), _ptr]
         lib.piper_attention_forward_fused.restype = ctypes.c_int
+        lib.piper_attention_forward_balanced.argtypes = [ctypes.POINTER(PiperAttentionFusedArgs), _ptr]
+        lib.piper_attention_forward_balanced.restype = ctypes.c_int
         lib.piper_attention_workspace_bytes.argtypes = [ctypes.POINTER(PiperShape), _i32, ctypes.POINTER(_i64)]
         lib.piper_attention_workspace_bytes.restype = ctypes.c_int
         lib.piper_sage_prepared_layout.argtypes = [ctypes.POINTER(PiperShape), ctypes.POINTER(PiperSageLayout)]
@@ -252,6 +256,8 @@ class NativeLibrary:
         lib.piper_sage_prepare.restype = ctypes.c_int
         lib.piper_sage_attention_forward.argtypes = [ctypes.POINTER(PiperSageAttentionArgs), _ptr]
         lib.piper_sage_attention_forward.restype = ctypes.c_int
+        lib.piper_sage_attention_forward_balanced.argtypes = [ctypes.POINTER(PiperSageAttentionArgs), _ptr]
+        lib.piper_sage_attention_forward_balanced.restype = ctypes.c_int
         version = lib.piper_abi_version()
         if version != ABI_VERSION:
             raise LibraryUnavailableError(
@@ -309,6 +315,11 @@ class NativeLibrary:
             self._lib.piper_attention_forward_fused(ctypes.byref(args), _ptr(stream)), "piper_attention_forward_fused"
         )
 
+    def attention_forward_balanced(self, args: PiperAttentionFusedArgs, stream: int) -> None:
+        """attention_forward_fused, free to run a small causal grid as key streams (equal to rounding)."""
+        self._check(self._lib.piper_attention_forward_balanced(ctypes.byref(args), _ptr(stream)),
+                    "piper_attention_forward_balanced")
+
     def sage_prepared_layout(self, shape: PiperShape) -> PiperSageLayout:
         layout = PiperSageLayout()
         self._check(
@@ -323,6 +334,12 @@ class NativeLibrary:
         self._check(
             self._lib.piper_sage_attention_forward(ctypes.byref(args), _ptr(stream)), "piper_sage_attention_forward"
         )
+
+    def sage_attention_forward_balanced(self, args: PiperSageAttentionArgs, stream: int) -> None:
+        """sage_attention_forward, free to run a small grid as key streams (equal to rounding)."""
+        self._check(self._lib.piper_sage_attention_forward_balanced(ctypes.byref(args), _ptr(stream)),
+                    "piper_sage_attention_forward_balanced")
+
 
 
 

@@ -1,7 +1,8 @@
 """Key streams (csrc/attention.hip attention_streams_kernel): two and four parts of small grids, at the
 edges -- fewer key tiles than streams, key tiles that do not divide, query rows past the end in one of a
 workgroup's groups, one row -- against the unsplit kernel and the oracle; the two-step and the fused
-entry points bit for bit alike."""
+entry points bit for bit alike.  The balanced entry points, which choose streams themselves (causal Piper
+Attention, SageAttention2++), against the others."""
 
 from __future__ import annotations
 
@@ -10,6 +11,7 @@ import torch
 
 from _parity import assert_attention_close, gpu_attention, gpu_prepare, log, oracle_attention
 from oracle import piper_oracle as oracle
+from piper_kernels._hip import library as native
 from piper_kernels.attention.piper_attention._plan import MI355XPlan
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +46,53 @@ def test_streams_match_the_unsplit_kernel_and_the_oracle(shape, d, parts, granul
     assert (split - whole).abs().max().item() <= 1e-5 * max(1.0, whole.abs().max().item())
     expected, bound = oracle_attention(oracle.prepare(q, k, v, False, granularity), d**-0.5, False)
     assert_attention_close(split.cpu().numpy(), expected, f"{parts} streams", flip_bound=bound)
+
+
+class _Balanced:
+    """The library with its attention entry points replaced by the balanced ones."""
+
+    def __init__(self, lib):
+        self._lib = lib
+
+    def __getattr__(self, name):
+        return getattr(self._lib, {"attention_forward_fused": "attention_forward_balanced",
+                                   "sage_attention_forward": "sage_attention_forward_balanced"}.get(name, name))
+
+
+BALANCED = [
+    # (operator, B, H, Sq, Sk, causal): four streams, two streams, a grid past the rule's lines
+    ("piper", 1, 3, 500, 500, True),
+    ("piper", 1, 12, 1031, 1031, True),
+    ("piper", 2, 30, 1031, 1031, True),
+    ("sage", 1, 3, 500, 500, True),
+    ("sage", 1, 12, 1031, 1031, True),
+    ("sage", 1, 5, 97, 300, False),
+    ("sage", 1, 40, 257, 700, False),
+    ("sage", 2, 40, 257, 700, False),
+]
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("case", BALANCED, ids=str)
+def test_balanced_entry_points_equal_the_others_to_rounding(case, d, gfx950_device, monkeypatch) -> None:
+    from piper_kernels.attention.piper_attention.hip import _launch_piper_attention, _prepare_piper_attention
+    from piper_kernels.attention.sage_attention_2pp.hip import _launch_sage_attention_2pp, _prepare_sage_attention_2pp
+
+    operator, b, h, sq, sk, causal = case
+    log(f"[case] balanced {case} D={d}")
+    g = torch.Generator().manual_seed(sq + h)
+    q = torch.randn((b, h, sq, d), generator=g).to(torch.bfloat16).to(gfx950_device)
+    k, v = (torch.randn((b, h, sk, d), generator=g).to(torch.bfloat16).to(gfx950_device) for _ in range(2))
+    lib = native.load_library()
+    outs = []
+    for handle in (lib, _Balanced(lib)):
+        monkeypatch.setattr(native, "load_library", lambda *a, handle=handle: handle)
+        out = torch.empty((b, h, sq, d), device=gfx950_device)
+        if operator == "piper":
+            prepared = _prepare_piper_attention(q, k, v, d**-0.5, causal, quantize_query=False)
+            outs.append(_launch_piper_attention(prepared, output=out))
+        else:
+            outs.append(_launch_sage_attention_2pp(_prepare_sage_attention_2pp(q, k, v, d**-0.5, causal), output=out))
+    # every probability code is the same (an FP8 code off by one step would show as 1e-3); the FP32 sums
+    # enter in another order: a few ulps of a value of the outputs' size
+    assert (outs[0] - outs[1]).abs().max().item() <= 2e-6 * max(1.0, outs[0].abs().max().item())

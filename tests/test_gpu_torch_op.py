@@ -1,5 +1,4 @@
-"""The native torch kernels (csrc/torch_op.cpp) against the Python path over the same C ABI, bit for bit:
-every option, inputs read in place and inputs that must be copied, a side stream whose inputs are freed
+"""The native torch kernels (csrc/torch_op.cpp) against the Python path over the same C ABI: every option, inputs read in place and inputs that must be copied, a side stream whose inputs are freed
 at once, replays of a captured graph; errors stay Python exceptions; the plan source covers both
 operators."""
 
@@ -32,6 +31,7 @@ def _inputs(b, h, sq, sk, d, dtype, device, seed=0):
     (1, 2, 300, 1000, 64, torch.bfloat16, False, "odd"),
     (1, 8, 1024, 1024, 64, torch.float16, False, "bhsd"),  # key-range split: a workspace
     (1, 24, 200, 3000, 128, torch.float16, False, "bshd"),
+    (1, 5, 1100, 1100, 128, torch.bfloat16, True, "bshd"),  # causal key streams
 ], ids=str)
 def test_native_call_equals_the_python_path(case, operator, gfx950_device) -> None:
     b, h, sq, sk, d, dtype, causal, layout = case
@@ -46,7 +46,11 @@ def test_native_call_equals_the_python_path(case, operator, gfx950_device) -> No
         for scale in (None, 0.2):
             got = public(q, k, v, scale=scale, is_causal=causal)
             want = python(q, k, v, d**-0.5 if scale is None else scale, causal)
-            assert got.is_contiguous() and got.dtype is dtype and torch.equal(got, want)
+            assert got.is_contiguous() and got.dtype is dtype
+            # the op may run key streams, whose FP32 sums differ by rounding (1e-5 as for the split plans)
+            # and can round to the neighbouring 16-bit value
+            step = 2.0 ** (-10 if dtype is torch.float16 else -7)
+            torch.testing.assert_close(got.float(), want.float(), rtol=step, atol=1e-5)
 
 
 @pytest.mark.gpu
