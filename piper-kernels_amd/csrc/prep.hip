@@ -254,6 +254,32 @@ __device__ __forceinline__ void wave_statistics(const MeanParams& p, int tensor,
 // tile (a workgroup of 4 waves holds units of one kind only).  No LDS: V tiles are written
 // transposed straight from registers.
 // ---------------------------------------------------------------------------------------
+// A 16-byte load of rows that the prep reads for the last time: kept out of the caches' replacement order, so
+// that it neither evicts the tile records written meanwhile nor waits for lines it will not reuse.  Single
+// pass: B2 H24 S16384 D128 229 -> 169 us, B1 H24 S16384 92 -> 84, SageAttention2++ B4 H32 S8192 263 -> 239.
+__device__ __forceinline__ uint4 load_once(const uint16_t* p) {
+  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+  const v4u v = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// The padding of a tile record's K rows (row 0's holds the scales) and V^T rows, written as zeros by the
+// wave that writes the rows: with it every cache line of the record is written whole.  A line with a hole
+// reaches memory as a partial write, which the memory side completes by reading the line first: the single
+// pass at B4 H32 S8192 D128 (345 MB of records) 264 -> 185 us causal, SageAttention2++ 239 -> 203; B1 H24
+// S16384, whose records fit the last-level cache, 84 -> 86.
+template <int D>
+__device__ __forceinline__ void pad_key_rows(int8_t* tile, int lane) {
+  if (lane != 0) *reinterpret_cast<uint4*>(tile + lane * kv_k_stride(D) + D) = make_uint4(0, 0, 0, 0);
+}
+
+template <int D>
+__device__ __forceinline__ void pad_value_rows(uint8_t* rows, int lane) {
+#pragma unroll
+  for (int r = 0; r < D; r += kWave)
+    *reinterpret_cast<uint4*>(rows + (r + lane) * kv_v_stride() + kKeyBlock) = make_uint4(0, 0, 0, 0);
+}
+
 // Q or K block of kRows rows.  Per block (the reference's "per_warp", sage/reference.py:61-77):
 // one scale over kRows x D values.  Per thread group (its "per_thread", sage/reference.py:23-58):
 // a 32-row Q block has 8 scales, row r in group r % 8 (rows {t, t+8, t+16, t+24}); a 64-row K
@@ -283,7 +309,7 @@ __device__ __forceinline__ void quantize_block(const InputTensor& in, int b, int
 #pragma unroll
   for (int it = 0; it < kIters; ++it) {
     const int row = row0 + it * kRowsPerIter + sub;
-    raw[it] = !kGuard || row < length ? *reinterpret_cast<const uint4*>(base + static_cast<long>(row) * in.stride_seq)
+    raw[it] = !kGuard || row < length ? load_once(base + static_cast<long>(row) * in.stride_seq)
                                       : make_uint4(0, 0, 0, 0);
   }
 #pragma unroll
@@ -336,6 +362,7 @@ __device__ __forceinline__ void quantize_block(const InputTensor& in, int b, int
     uint2 packed = make_uint2(pack_low_bytes(c[0], c[1], c[2], c[3]), pack_low_bytes(c[4], c[5], c[6], c[7]));
     *reinterpret_cast<uint2*>(codes + static_cast<long>(it * kRowsPerIter + sub) * kStride + group * 8) = packed;
   }
+  if constexpr (kStride != D) pad_key_rows<D>(codes, lane);
   // key tiles also carry their scales in the padding of K row 0 (bytes [D, D + 4 * kSlots))
   float* tile_scales = kStride != D ? reinterpret_cast<float*>(codes + D) : nullptr;
   if (!per_thread || kSlots == 1) {
@@ -404,7 +431,7 @@ __device__ __forceinline__ void load_unit_rows(const InputTensor& in, int b, int
 #pragma unroll
   for (int j = 0; j < kKeys; ++j) {
     const int row = kb * kKeyBlock + key0 + j;
-    raw[j] = !kGuard || row < length ? *reinterpret_cast<const uint4*>(base + static_cast<long>(row) * in.stride_seq)
+    raw[j] = !kGuard || row < length ? load_once(base + static_cast<long>(row) * in.stride_seq)
                                      : make_uint4(0, 0, 0, 0);
   }
 }
@@ -465,6 +492,7 @@ __device__ __forceinline__ void quantize_value_rows(const QuantParams& p, int un
     else
       *reinterpret_cast<uint2*>(dst) = make_uint2(packed[i][0], packed[i][1]);
   }
+  pad_value_rows<D>(tile + kv_v_offset(D), lane);
   // per-key metadata, one key per lane: lane (group, sub) with group < kKeys owns key key0 + group
   float* meta = reinterpret_cast<float*>(tile + kv_log_offset(D));
   if (group < kKeys) {
@@ -561,6 +589,7 @@ __device__ __forceinline__ void quantize_channel_rows(const QuantParams& p, int 
     else
       *reinterpret_cast<uint2*>(dst) = make_uint2(packed[i][0], packed[i][1]);
   }
+  pad_value_rows<D>(tile + sage_v_offset(D), lane);
 }
 
 // A V tile's codes from its rows and the statistic of the lane's eight columns: the means that centre
@@ -738,6 +767,7 @@ __device__ __forceinline__ void quantize_key_rows(uint4 (&raw)[kKeyBlock / (kWav
     *reinterpret_cast<uint2*>(tile + (kKeys * sub + j) * kStride + 8 * group) =
         make_uint2(pack_low_bytes(c[0], c[1], c[2], c[3]), pack_low_bytes(c[4], c[5], c[6], c[7]));
   }
+  pad_key_rows<D>(tile, lane);
   if (lane == 0) {
     const float4 s4 = make_float4(scale[0], scale[1], scale[2], scale[3]);
     *reinterpret_cast<float4*>(scale_out) = s4;
