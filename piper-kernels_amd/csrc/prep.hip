@@ -254,15 +254,6 @@ __device__ __forceinline__ void wave_statistics(const MeanParams& p, int tensor,
 // tile (a workgroup of 4 waves holds units of one kind only).  No LDS: V tiles are written
 // transposed straight from registers.
 // ---------------------------------------------------------------------------------------
-// A 16-byte load of rows that the prep reads for the last time: kept out of the caches' replacement order, so
-// that it neither evicts the tile records written meanwhile nor waits for lines it will not reuse.  Single
-// pass: B2 H24 S16384 D128 229 -> 169 us, B1 H24 S16384 92 -> 84, SageAttention2++ B4 H32 S8192 263 -> 239.
-__device__ __forceinline__ uint4 load_once(const uint16_t* p) {
-  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-  const v4u v = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p));
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-
 // The padding of a tile record's K rows (row 0's holds the scales) and V^T rows, written as zeros by the
 // wave that writes the rows: with it every cache line of the record is written whole.  A line with a hole
 // reaches memory as a partial write, which the memory side completes by reading the line first: the single
@@ -309,7 +300,7 @@ __device__ __forceinline__ void quantize_block(const InputTensor& in, int b, int
 #pragma unroll
   for (int it = 0; it < kIters; ++it) {
     const int row = row0 + it * kRowsPerIter + sub;
-    raw[it] = !kGuard || row < length ? load_once(base + static_cast<long>(row) * in.stride_seq)
+    raw[it] = !kGuard || row < length ? *reinterpret_cast<const uint4*>(base + static_cast<long>(row) * in.stride_seq)
                                       : make_uint4(0, 0, 0, 0);
   }
 #pragma unroll
@@ -416,10 +407,21 @@ __device__ __forceinline__ uint32_t insert_byte(uint32_t packed, uint32_t word) 
   return __builtin_amdgcn_perm(word, packed, kSel);
 }
 
+// A 16-byte load of rows that are read once: kept out of the caches' replacement order, so that it neither
+// evicts the tile records written meanwhile nor waits for lines it will not reuse.  The single pass loads
+// this way: B2 H24 S16384 D128 229 -> 169 us, B1 H24 S16384 92 -> 84, SageAttention2++ B4 H32 S8192 263 ->
+// 239.  The two-pass quantisation does not, whose rows are in the last-level cache (B2 H16 S1531 causal 13
+// us, 17 with these loads).
+__device__ __forceinline__ uint4 load_once(const uint16_t* p) {
+  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+  const v4u v = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // Rows [16 sub, +16) of a 64-row K block or V tile (8 rows at D = 64), columns [8 group, +8):
 // lane (group, sub)'s share of the unit, every load in flight before any arithmetic.  Rows past
 // the end read as zero.
-template <int D, bool kGuard>
+template <int D, bool kGuard, bool kOnce = false>
 __device__ __forceinline__ void load_unit_rows(const InputTensor& in, int b, int h, int kb, int length, int lane,
                                                uint4 (&raw)[kKeyBlock / (kWave / (D / 8))]) {
   constexpr int kGroups = D / 8;
@@ -431,8 +433,9 @@ __device__ __forceinline__ void load_unit_rows(const InputTensor& in, int b, int
 #pragma unroll
   for (int j = 0; j < kKeys; ++j) {
     const int row = kb * kKeyBlock + key0 + j;
-    raw[j] = !kGuard || row < length ? load_once(base + static_cast<long>(row) * in.stride_seq)
-                                     : make_uint4(0, 0, 0, 0);
+    const uint16_t* src = base + static_cast<long>(row) * in.stride_seq;
+    if (kGuard && row >= length) raw[j] = make_uint4(0, 0, 0, 0);
+    else raw[j] = kOnce ? load_once(src) : *reinterpret_cast<const uint4*>(src);
   }
 }
 
@@ -961,7 +964,7 @@ __device__ __forceinline__ void single_pass_chunk(const SinglePassParams& p, Sin
 
   uint4 raw[kKeys];
   if (full_unit) {
-    load_unit_rows<D, false>(in, b, h, kb, length, lane, raw);
+    load_unit_rows<D, false, true>(in, b, h, kb, length, lane, raw);
   } else {
 #pragma unroll
     for (int j = 0; j < kKeys; ++j) raw[j] = make_uint4(0, 0, 0, 0);
