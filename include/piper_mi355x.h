@@ -336,13 +336,15 @@ int piper_prepared_layout(const piper_shape* shape, piper_layout* layout);
  * with PIPER_PREPARE_SKIP_QUERY only K and V.  key_mean must be 4-byte aligned, the workspace
  * and the other prepared buffers 16-byte aligned.
  *
- * Launches, at D = 128 with Sk <= 32768 when one XCC of the device holds a tensor's 256-row
- * chunks at once (4 * CUs / XCCs >= ceil(Sk / 256); every MI355X partition mode): a fill kernel
- * (sync words cleared, means marked pending) and the single pass, which reads K and V once: each
+ * Launches: one for short sequences in small grids (each workgroup sums the whole sequence itself); two
+ * for mid-length ones (FP32 mean partials in torch's CPU order, then quantisation whose waves finish the
+ * means); up to Sk = 32768 otherwise, when one XCC of the device holds a tensor's 256-row chunks at once
+ * (4 * CUs / XCCs >= ceil(Sk / 256); every MI355X partition mode), a fill kernel (arrival counters and
+ * status word cleared, means marked pending) and the single pass, which reads K and V once: each
  * chunk publishes its partial sums, the last chunk of a batch-head tensor finalises the mean,
  * the others wait for it (bounded: a chunk whose wait ends computes the mean itself from K/V in
  * HBM, same bits, and is counted in the status word), then every chunk quantises its rows.
- * Otherwise: FP32 mean partials (torch's CPU order), mean finalisation, one quantisation kernel.
+ * Beyond: mean partials, mean finalisation, quantisation.  Every route gives the same bits.
  * Work on other streams or in other processes that holds the GPU's workgroup slots can delay a
  * tensor's last chunk: the results stay exact, the prep gets slower (piper_prepare_status). */
 int piper_prepare(const piper_prepare_args* args, void* stream);
@@ -350,7 +352,7 @@ int piper_prepare(const piper_prepare_args* args, void* stream);
 /* The status word of the last prep that used `workspace` (NULL: the static scratch of
  * piper_prepare_static on the current device) for `shape`: the number of single-pass chunks
  * whose bounded wait for their tensor's mean ended, so that they computed it themselves (0 for
- * the three-kernel path).  Diagnostic: copies the word to *count and synchronises `stream`. */
+ * the other routes).  Diagnostic: copies the word to *count and synchronises `stream`. */
 int piper_prepare_status(const piper_shape* shape, const void* workspace, uint32_t* count, void* stream);
 
 /* piper_prepare without a caller workspace.  No counterpart in the reference: for callers that

@@ -113,7 +113,7 @@ int device_topology(int* cus, int* xccs) {
     int c = 0, x = 0;
     err = hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, device);
     if (err != hipSuccess) return fail(PIPER_ERROR_HIP, "compute-unit count query failed: %s", hipGetErrorString(err));
-    // no XCC count (an older runtime): 0, which keeps the prep on its three-kernel path
+    // no XCC count (an older runtime): 0, which keeps the prep off the single pass
     if (hipDeviceGetAttribute(&x, hipDeviceAttributeNumberOfXccs, device) != hipSuccess || x < 0) x = 0;
     (void)hipGetLastError();
     g_topology[device][0] = c;
