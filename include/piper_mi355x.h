@@ -374,9 +374,11 @@ int piper_prepare_static(const piper_prepare_args* args, void* stream);
 /* Fused INT8-QK / UINT8-P x INT8-V online-softmax attention on `stream`. */
 int piper_attention_forward(const piper_attention_args* args, void* stream);
 
-/* Workspace bytes the attention entry points need for `plan`: parts * B * H * Sq * (D + 2) * 4 for
- * a key-range split, 256 for the work-queue plan (its counters; the library zeroes them on the
- * stream before each call), 0 otherwise. */
+/* Workspace bytes the attention entry points need for `plan` on the current device: parts * rows *
+ * (D + 2) * 4 for a key-range split, `rows` the query rows of the tiles that are split (those beyond
+ * whole rounds of resident workgroups; none where the parts are taken by the waves of a workgroup), at
+ * most parts * B * H * Sq * (D + 2) * 4, which is the answer without a device; 256 for the work-queue
+ * plan (its counters; the library zeroes them on the stream before each call), 0 otherwise. */
 int piper_attention_workspace_bytes(const piper_shape* shape, int32_t plan, int64_t* bytes);
 
 /* The same with the query quantised inside the kernel (see piper_attention_fused_args). */

@@ -124,6 +124,22 @@ int device_topology(int* cus, int* xccs) {
   return PIPER_OK;
 }
 
+// The key-range split of a call on the current device; without one, every row counted as split, which
+// bounds the workspace on any device.
+piper::KeySplit split_of(const piper_shape& s, int parts) {
+  const long batch_heads = s.batch * s.heads;
+  const int key_tiles = static_cast<int>(ceil_div(s.key_length, PIPER_KEY_BLOCK));
+  const int head_dim = static_cast<int>(s.head_dim);
+  int cus = 0, xccs = 0;
+  if (parts > 1 && device_topology(&cus, &xccs) != PIPER_OK) {
+    (void)hipGetLastError();
+    piper::KeySplit whole{parts, 1, key_tiles, 0, 0, 0};
+    whole.bytes = parts * batch_heads * s.query_length * (head_dim + 2) * 4;
+    return whole;
+  }
+  return piper::key_split(batch_heads, s.query_length, key_tiles, head_dim, parts, cus);
+}
+
 piper::InputTensor to_input(const piper_tensor& t) {
   return piper::InputTensor{t.data, static_cast<long>(t.stride_batch), static_cast<long>(t.stride_head),
                             static_cast<long>(t.stride_seq)};
@@ -157,9 +173,9 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
   }
   if (work_queue && !(plan & PIPER_PLAN_THREE_WORKGROUPS))
     return fail(PIPER_ERROR_UNSUPPORTED, "the work-queue plan needs PIPER_PLAN_THREE_WORKGROUPS");
-  if (key_parts > 1 || work_queue) {
-    int64_t need = 0;
-    if (int st = piper_attention_workspace_bytes(&s, plan, &need)) return st;
+  const piper::KeySplit split = split_of(s, key_parts);
+  const int64_t need = work_queue ? piper::kQueueBytes : split.bytes;
+  if (need > 0) {
     if (workspace == nullptr || workspace_bytes < need)
       return fail(PIPER_ERROR_INVALID_ARGUMENT, "the %s needs a workspace of %lld bytes, got %lld",
                   work_queue ? "work-queue plan" : "key-range split", (long long)need, (long long)workspace_bytes);
@@ -213,30 +229,19 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
     ap.query_bf16 = query_dtype == PIPER_BFLOAT16 ? 1 : 0;
     ap.query = to_input(*query);
   }
-  // key-range split: part_tiles tiles per part, and no empty part; only the query tiles beyond whole
-  // rounds of resident workgroups are split.  Two or four parts of a grid whose workgroups then all fit
-  // the GPU at once are key streams instead.
-  ap.key_parts = 1;
-  ap.key_streams = 1;
   if (key_parts > 1) {
     int cus = 0, xccs = 0;
-    if (int st = device_topology(&cus, &xccs)) return st;
-    const int head_dim = static_cast<int>(s.head_dim);
-    const int64_t tiles = static_cast<int64_t>(ap.query_tiles) * ap.batch_heads;
-    const int64_t slots = static_cast<int64_t>(piper::waves_per_simd(head_dim)) * std::max(cus, 1);
-    ap.part_tiles = static_cast<int>(ceil_div(ap.nkb, key_parts));
-    ap.key_parts = static_cast<int>(ceil_div(ap.nkb, ap.part_tiles));
-    ap.whole_tiles = static_cast<int>(std::min<int64_t>(tiles / slots * slots, 0x7fffffff));
-    ap.split_row0 = static_cast<long>(ap.whole_tiles / ap.query_tiles) * s.query_length +
-                    static_cast<long>(ap.whole_tiles % ap.query_tiles) * block_m;
-    ap.partials = static_cast<float*>(workspace);
-    if (ap.whole_tiles == tiles) ap.key_parts = 1;
-    if ((key_parts == 2 || key_parts == 4) && key_parts * tiles <= int64_t{piper::stream_workgroups(head_dim, key_parts)} * cus) {
-      ap.key_parts = 1;
-      ap.key_streams = key_parts;
-      ap.query_tiles = static_cast<int>(ceil_div(s.query_length, block_m / key_parts));
-    }
+    if (int st = device_topology(&cus, &xccs)) return st;  // split_of's bound is no launch geometry
   }
+  ap.key_parts = split.parts;
+  ap.key_streams = split.streams;
+  if (split.parts > 1) {
+    ap.part_tiles = split.part_tiles;
+    ap.whole_tiles = static_cast<int>(std::min(split.whole_tiles, 0x7fffffffL));
+    ap.split_row0 = split.row0;
+    ap.partials = static_cast<float*>(workspace);
+  }
+  if (split.streams > 1) ap.query_tiles = static_cast<int>(ceil_div(s.query_length, block_m / split.streams));
   if (balanced && is_causal && waves == 3 && !work_queue) {
     int cus = 0, xccs = 0;
     if (int st = device_topology(&cus, &xccs)) return st;
@@ -433,10 +438,7 @@ int piper_attention_workspace_bytes(const piper_shape* shape, int32_t plan, int6
   if (int st = check_shape(shape)) return st;
   if (bytes == nullptr) return fail(PIPER_ERROR_INVALID_ARGUMENT, "bytes is NULL");
   if (plan < 0 || plan > PIPER_PLAN_MASK) return fail(PIPER_ERROR_UNSUPPORTED, "unknown plan %d", plan);
-  *bytes = (plan & PIPER_PLAN_WORK_QUEUE)
-               ? piper::kQueueBytes
-               : piper::attention_partial_bytes(shape->batch * shape->heads, shape->query_length,
-                                                static_cast<int>(shape->head_dim), PIPER_PLAN_KEY_PARTS_OF(plan));
+  *bytes = (plan & PIPER_PLAN_WORK_QUEUE) ? piper::kQueueBytes : split_of(*shape, PIPER_PLAN_KEY_PARTS_OF(plan)).bytes;
   g_last_error[0] = '\0';
   return PIPER_OK;
 }

@@ -226,9 +226,36 @@ __host__ __device__ inline long split_rows(const AttnParams& p) {
   return static_cast<long>(p.batch_heads) * p.query_length - p.split_row0;
 }
 
-// The workspace bytes of a key-range split (0 without one).
-inline long attention_partial_bytes(long batch_heads, long query_length, int head_dim, int key_parts) {
-  return key_parts > 1 ? static_cast<long>(key_parts) * batch_heads * query_length * (head_dim + 2) * 4 : 0;
+// How a plan of `parts` key parts runs a grid on a device of `cus` compute units: only the query tiles
+// beyond whole rounds of resident workgroups are split, no part is empty, and two or four parts of a grid
+// whose workgroups then all fit the GPU at once are key streams, which need no partial sums.  The launch
+// and the workspace's size both come from here.
+struct KeySplit {
+  int parts;         // key ranges of a split query tile (1: nothing is split)
+  int streams;       // key streams (1: none)
+  int part_tiles;    // key tiles per range
+  long whole_tiles;  // query tiles that run unsplit, before the split ones
+  long row0;         // the first output row (of batch_heads * query_length) of the split tiles
+  long bytes;        // workspace: the split rows' partial sums, D numerators and two floats per part
+};
+
+inline KeySplit key_split(long batch_heads, long query_length, int key_tiles, int head_dim, int parts, int cus) {
+  constexpr int kRows = 128;  // query rows of a workgroup
+  KeySplit k{1, 1, key_tiles, 0, 0, 0};
+  if (parts <= 1) return k;
+  const long per_head = (query_length + kRows - 1) / kRows;
+  const long tiles = per_head * batch_heads;
+  const long slots = static_cast<long>(waves_per_simd(head_dim)) * (cus > 1 ? cus : 1);
+  k.part_tiles = (key_tiles + parts - 1) / parts;
+  k.whole_tiles = tiles / slots * slots;
+  k.row0 = k.whole_tiles / per_head * query_length + k.whole_tiles % per_head * kRows;
+  if ((parts == 2 || parts == 4) && parts * tiles <= static_cast<long>(stream_workgroups(head_dim, parts)) * cus) {
+    k.streams = parts;
+  } else if (k.whole_tiles < tiles) {
+    k.parts = (key_tiles + k.part_tiles - 1) / k.part_tiles;
+    if (k.parts > 1) k.bytes = k.parts * (batch_heads * query_length - k.row0) * (head_dim + 2) * 4;
+  }
+  return k;
 }
 
 // The work-queue plan's counters: one per XCC, at most kQueueCounters.

@@ -228,7 +228,8 @@ def _launch_piper_attention(
     # the work-queue plan: its counters
     workspace = None
     if prepared.plan.key_parts > 1 or prepared.plan.work_queue:
-        size = lib.attention_workspace_bytes(_native_shape(batch, heads, sq, sk, d), prepared.plan.plan_id)
+        with torch.cuda.device(device):  # the size depends on the device's compute units
+            size = lib.attention_workspace_bytes(_native_shape(batch, heads, sq, sk, d), prepared.plan.plan_id)
         workspace = torch.empty(size, dtype=torch.uint8, device=device)
     ws_ptr, ws_bytes = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel())
     if prepared.fused_query:

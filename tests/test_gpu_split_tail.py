@@ -52,3 +52,42 @@ def test_the_rule_splits_only_partial_rounds_into_whole_key_tiles() -> None:
     # 192 query tiles still fit the GPU as two key streams each; 320 do not, and six key tiles are too few
     # for partial sums
     assert split_parts(2, 12, 1000, 333, 128) == 2 and split_parts(1, 40, 1000, 333, 128) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_the_split_stays_inside_the_workspace_it_asks_for(case, gfx950_device, monkeypatch) -> None:
+    """The bytes piper_attention_workspace_bytes reports on this device: the split rows' partial sums only;
+    nothing behind them is written, and one byte less is refused."""
+    from piper_kernels._hip import library as native
+
+    h, tiles, last, sk, d, parts = case
+    sq = (tiles - 1) * 128 + last
+    log(f"[case] split workspace {case}")
+    plan = MI355XPlan(waves=4, three_per_cu=True, key_parts=parts)
+    lib = native.load_library()
+    size = lib.attention_workspace_bytes(native.PiperShape(1, h, sq, sk, d), plan.plan_id)
+    slots = torch.cuda.get_device_properties(gfx950_device).multi_processor_count * (4 if d == 64 else 3)
+    first = h * tiles // slots * slots
+    rows = h * sq - (first // tiles * sq + first % tiles * 128)
+    key_tiles = -(-sk // 64)
+    assert size == -(-key_tiles // -(-key_tiles // parts)) * rows * (d + 2) * 4
+    g = torch.Generator().manual_seed(sq)
+    q = torch.randn((1, h, sq, d), generator=g).to(torch.float16)
+    k, v = (torch.randn((1, h, sk, d), generator=g).to(torch.float16) for _ in range(2))
+    prepared = gpu_prepare(q, k, v, d**-0.5, False, gfx950_device, quantize_query=False, plan=plan)
+    guarded = torch.full((size + 4096,), 0x5A, dtype=torch.uint8, device=gfx950_device)
+    out = torch.empty((1, h, sq, d), device=gfx950_device)
+    args = native.PiperAttentionFusedArgs(
+        abi_version=native.ABI_VERSION, dtype=native.FLOAT16, output_dtype=native.FLOAT32, is_causal=0, plan=plan.plan_id,
+        scale=d**-0.5, flags=0, reserved=0, shape=native.PiperShape(1, h, sq, sk, d),
+        query=native.PiperTensor(prepared.query.data_ptr(), *prepared.query.stride()[:3]), prepared=prepared.native_prepared(),
+        output=out.data_ptr(), workspace=guarded.data_ptr(), workspace_bytes=size - 1)
+    stream = torch.cuda.current_stream(gfx950_device).cuda_stream
+    with pytest.raises(RuntimeError, match="needs a workspace"):
+        lib.attention_forward_fused(args, stream)
+    args.workspace_bytes = size
+    lib.attention_forward_fused(args, stream)
+    torch.cuda.synchronize(gfx950_device)
+    assert bool((guarded[size:] == 0x5A).all())
+    assert torch.equal(out, gpu_attention(prepared, torch.float32))
