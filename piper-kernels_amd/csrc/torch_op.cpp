@@ -13,8 +13,11 @@
 
 #include <array>
 #include <atomic>
+#include <exception>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <string>
 
 #include "piper_mi355x.h"
 
@@ -221,14 +224,26 @@ at::Tensor sage_attention_2pp(const at::Tensor& query, const at::Tensor& key, co
 
 }  // namespace
 
-// Sets the function that chooses launch plans and forgets the plans chosen so far.
-extern "C" __attribute__((visibility("default"))) void piper_torch_set_plan_source(PlanSource source) {
-  g_plan_source.store(source);
-  std::lock_guard<std::mutex> lock(g_plans_mutex);
-  g_plans.clear();
-}
-
-TORCH_LIBRARY_IMPL(piper_kernels, CUDA, m) {
-  m.impl("piper_attention", &piper_attention);
-  m.impl("sage_attention_2pp", &sage_attention_2pp);
+// Sets the function that chooses launch plans, forgets the plans chosen so far and registers the kernels with
+// torch (once; only here, so that no thread's call finds kernels without a plan source).  Returns NULL, or
+// what went wrong.
+extern "C" __attribute__((visibility("default"))) const char* piper_torch_set_plan_source(PlanSource source) {
+  static thread_local std::string error;
+  try {
+    std::lock_guard<std::mutex> lock(g_plans_mutex);
+    g_plan_source.store(source);
+    g_plans.clear();
+    static torch::Library* kernels = nullptr;  // registered until the process ends
+    if (kernels == nullptr) {
+      auto library = std::make_unique<torch::Library>(torch::Library::IMPL, "piper_kernels", c10::DispatchKey::CUDA,
+                                                      __FILE__, __LINE__);
+      library->impl("piper_attention", &piper_attention);
+      library->impl("sage_attention_2pp", &sage_attention_2pp);
+      kernels = library.release();
+    }
+  } catch (const std::exception& e) {
+    error = e.what();
+    return error.c_str();
+  }
+  return nullptr;
 }

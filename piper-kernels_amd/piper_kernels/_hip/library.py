@@ -375,8 +375,10 @@ def load_torch_kernels() -> None:
             kernels = ctypes.CDLL(str(TORCH_LIBRARY_PATH))
         except OSError as error:
             raise LibraryUnavailableError(f"cannot open {TORCH_LIBRARY_PATH}: {error}") from error
-        kernels.piper_torch_set_plan_source.restype = None
-        kernels.piper_torch_set_plan_source(_choose_plan)
+        kernels.piper_torch_set_plan_source.restype = ctypes.c_char_p
+        error = kernels.piper_torch_set_plan_source(_choose_plan)  # registers the kernels
+        if error is not None:
+            raise LibraryUnavailableError(f"{TORCH_LIBRARY_PATH}: {error.decode('utf-8', 'replace')}")
         _torch_kernels = kernels
 
 

@@ -4,12 +4,16 @@ operators."""
 
 from __future__ import annotations
 
+import subprocess
+import sys
+
 import pytest
 import torch
 
 from _parity import log
 from piper_kernels import piper_attention, sage_attention_2pp
 from piper_kernels._hip import library as native
+from piper_kernels._hip.build import PACKAGE_ROOT
 from piper_kernels.attention.piper_attention import _plan
 from piper_kernels.attention.piper_attention.hip import _run_piper_attention
 from piper_kernels.attention.sage_attention_2pp.hip import _run_sage_attention_2pp
@@ -108,3 +112,23 @@ def test_plan_source_asks_the_package(monkeypatch) -> None:
     assert ask(1, 4, 32, 8192, 8192, 128, 1) == _plan.select_sage_plan(4, 32, 8192, 8192, 128, True).plan_id
     monkeypatch.setattr(_plan, "select_plan", lambda *a: 1 / 0)
     assert ask(0, 1, 8, 1024, 1024, 64, 0) < 0  # an error in Python is no plan
+
+
+def test_kernels_are_registered_together_with_their_plan_source() -> None:
+    """Opening the library registers nothing: a call of another thread between that and the plan source's
+    setting would find kernels that cannot choose a plan."""
+    program = """
+import ctypes, sys
+sys.path.insert(0, sys.argv[1])
+import torch, piper_kernels
+from piper_kernels._hip import library
+from piper_kernels._hip.build import TORCH_LIBRARY_PATH
+ops = ["piper_kernels::piper_attention", "piper_kernels::sage_attention_2pp"]
+has = lambda: [torch._C._dispatch_has_kernel_for_dispatch_key(op, "CUDA") for op in ops]
+kernels = ctypes.CDLL(str(TORCH_LIBRARY_PATH))
+assert has() == [False, False], has()
+library.load_torch_kernels()
+assert has() == [True, True], has()
+library.load_torch_kernels()
+"""
+    subprocess.run([sys.executable, "-c", program, str(PACKAGE_ROOT)], check=True, timeout=120)
