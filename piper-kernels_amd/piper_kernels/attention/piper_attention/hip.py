@@ -307,10 +307,12 @@ def hip_piper_attention(
     is_causal: bool,
 ) -> torch.Tensor:
     """Piper Attention K/V prep + fused INT8 kernel (query quantised in its prologue) on MI355X
-    (schema of triton.py:984-999).  On the GPU this body runs only until ``csrc/torch_op.cpp`` has
-    registered the same call natively (in a compiled graph: its first call)."""
+    (schema of triton.py:984-999).  On the GPU this body runs only where a process's first call
+    comes from a compiled graph or the op itself: it registers ``csrc/torch_op.cpp`` and goes there, as every
+    later call does."""
     if query.is_cuda:
         native.load_torch_kernels()
+        return torch.ops.piper_kernels.piper_attention(query, key, value, scale, is_causal)
     return _run_piper_attention(query, key, value, scale, is_causal)
 
 

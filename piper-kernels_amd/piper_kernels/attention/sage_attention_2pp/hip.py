@@ -203,9 +203,11 @@ def hip_sage_attention_2pp(
     is_causal: bool,
 ) -> torch.Tensor:
     """SageAttention2++ K/V prep + fused INT8-QK / FP8-PV kernel on MI355X (schema of triton.py:1136-1145).
-    On the GPU this body runs only until ``csrc/torch_op.cpp`` has registered the same call natively."""
+    On the GPU this body runs only where a process's first call comes from a compiled graph or the op itself:
+    it registers ``csrc/torch_op.cpp`` and goes there, as every later call does."""
     if query.is_cuda:
         native.load_torch_kernels()
+        return torch.ops.piper_kernels.sage_attention_2pp(query, key, value, scale, is_causal)
     return _run_sage_attention_2pp(query, key, value, scale, is_causal)
 
 

@@ -132,3 +132,33 @@ assert has() == [True, True], has()
 library.load_torch_kernels()
 """
     subprocess.run([sys.executable, "-c", program, str(PACKAGE_ROOT)], check=True, timeout=120)
+
+
+@pytest.mark.gpu
+def test_first_call_of_a_process_equals_the_next(gfx950_device) -> None:
+    """A compiled graph, or the op itself, can be a process's first use; its bits are those of every later call
+    (shapes that run key streams, whose sums have an order of their own)."""
+    log("[case] first call of a process")
+    program = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import torch
+from piper_kernels import piper_attention
+g = torch.Generator().manual_seed(3)
+q, k, v = (torch.randn((1, 3, 1000, 128), generator=g).to(torch.float16).cuda() for _ in range(3))
+compiled = torch.compile(lambda q, k, v: piper_attention(q, k, v, is_causal=True), fullgraph=True, backend="eager")
+with torch.no_grad():
+    first = compiled(q, k, v)
+    assert torch.equal(first, compiled(q, k, v)) and torch.equal(first, piper_attention(q, k, v, is_causal=True))
+"""
+    direct = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import torch, piper_kernels
+op = torch.ops.piper_kernels.sage_attention_2pp
+g = torch.Generator().manual_seed(4)
+q, k, v = (torch.randn((1, 3, 1000, 128), generator=g).to(torch.float16).cuda() for _ in range(3))
+assert torch.equal(op(q, k, v, 0.1, False), op(q, k, v, 0.1, False))
+"""
+    for text in (program, direct):
+        subprocess.run([sys.executable, "-c", text, str(PACKAGE_ROOT)], check=True, timeout=100)
