@@ -30,6 +30,7 @@ enum Operator : int32_t { kPiper = 0, kSage = 1 };
 using PlanSource = int32_t (*)(int32_t op, int64_t batch, int64_t heads, int64_t query_length, int64_t key_length,
                                int64_t head_dim, int32_t is_causal);
 std::atomic<PlanSource> g_plan_source{nullptr};
+thread_local std::string g_plan_error;  // why the source of this thread's call found no plan
 
 using PlanKey = std::array<int64_t, 7>;
 std::mutex g_plans_mutex;
@@ -45,9 +46,10 @@ int32_t plan_for(Operator op, const piper_shape& s, bool causal) {
   }
   const PlanSource source = g_plan_source.load();
   TORCH_CHECK(source != nullptr, "piper_kernels: no launch-plan source is set");
+  g_plan_error.clear();
   // without the lock: the source takes Python's
   const int32_t plan = source(op, s.batch, s.heads, s.query_length, s.key_length, s.head_dim, causal);
-  TORCH_CHECK(plan >= 0, "piper_kernels: no launch plan for this shape");
+  TORCH_CHECK(plan >= 0, "piper_kernels: no launch plan for this shape: ", g_plan_error);
   std::lock_guard<std::mutex> lock(g_plans_mutex);
   if (g_plans.size() >= kMaxPlans) g_plans.clear();
   g_plans.emplace(key, plan);
@@ -223,6 +225,14 @@ at::Tensor sage_attention_2pp(const at::Tensor& query, const at::Tensor& key, co
 }
 
 }  // namespace
+
+// What went wrong in the plan source: its text joins the error that the call raises.
+extern "C" __attribute__((visibility("default"))) void piper_torch_plan_error(const char* text) {
+  try {
+    g_plan_error = text != nullptr ? text : "";
+  } catch (const std::exception&) {  // out of memory: the call's error goes without the text
+  }
+}
 
 // Sets the function that chooses launch plans, forgets the plans chosen so far and registers the kernels with
 // torch (once; only here, so that no thread's call finds kernels without a plan source).  Returns NULL, or

@@ -345,13 +345,17 @@ class NativeLibrary:
 
 @ctypes.CFUNCTYPE(_i32, _i32, _i64, _i64, _i64, _i64, _i64, _i32)
 def _choose_plan(operator, batch, heads, query_length, key_length, head_dim, is_causal):
-    """The torch kernels' launch plan for a shape they have not seen (a negative number: none)."""
+    """The torch kernels' launch plan for a shape they have not seen (a negative number: none, and the error's
+    text goes to the call that asked)."""
     try:
         from ..attention.piper_attention import _plan
 
         select = _plan.select_sage_plan if operator else _plan.select_plan
         return select(batch, heads, query_length, key_length, head_dim, bool(is_causal)).plan_id
-    except Exception:  # noqa: BLE001  (nothing may unwind through the C++ caller, which raises instead)
+    except BaseException as error:  # noqa: BLE001  (nothing may unwind through the C++ caller, which raises instead;
+        # an interrupt that left here would count as plan 0)
+        if _torch_kernels is not None:
+            _torch_kernels.piper_torch_plan_error(f"{type(error).__name__}: {error}".encode("utf-8", "replace"))
         return -1
 
 
@@ -364,6 +368,8 @@ def load_torch_kernels() -> None:
     """Register the custom ops' GPU kernels with torch (once); raise :class:`LibraryUnavailableError`
     if their library is absent."""
     global _torch_kernels
+    if _torch_kernels is not None:
+        return
     with _lock:
         if _torch_kernels is not None:
             return
@@ -376,6 +382,8 @@ def load_torch_kernels() -> None:
         except OSError as error:
             raise LibraryUnavailableError(f"cannot open {TORCH_LIBRARY_PATH}: {error}") from error
         kernels.piper_torch_set_plan_source.restype = ctypes.c_char_p
+        kernels.piper_torch_plan_error.restype = None
+        kernels.piper_torch_plan_error.argtypes = [ctypes.c_char_p]
         error = kernels.piper_torch_set_plan_source(_choose_plan)  # registers the kernels
         if error is not None:
             raise LibraryUnavailableError(f"{TORCH_LIBRARY_PATH}: {error.decode('utf-8', 'replace')}")

@@ -113,6 +113,26 @@ def test_plan_source_asks_the_package(monkeypatch) -> None:
     monkeypatch.setattr(_plan, "select_plan", lambda *a: 1 / 0)
     assert ask(0, 1, 8, 1024, 1024, 64, 0) < 0  # an error in Python is no plan
 
+    def interrupted(*_):
+        raise KeyboardInterrupt
+
+    monkeypatch.setattr(_plan, "select_plan", interrupted)
+    assert ask(0, 1, 8, 1024, 1024, 64, 0) < 0  # and neither is an interrupt
+
+
+@pytest.mark.gpu
+def test_a_failed_plan_names_its_cause(gfx950_device, monkeypatch) -> None:
+    def broken(*_):
+        raise ValueError("this table has no such entry")
+
+    q, k, v = _inputs(1, 1, 37, 41, 64, torch.float16, gfx950_device)  # a shape no other test plans
+    monkeypatch.setattr(_plan, "select_plan", broken)
+    with torch.no_grad(), pytest.raises(RuntimeError, match="ValueError: this table has no such entry"):
+        piper_attention(q, k, v)
+    monkeypatch.undo()
+    with torch.no_grad():
+        assert torch.isfinite(piper_attention(q, k, v)).all()
+
 
 def test_kernels_are_registered_together_with_their_plan_source() -> None:
     """Opening the library registers nothing: a call of another thread between that and the plan source's
