@@ -66,16 +66,19 @@ int32_t dtype_code(const at::Tensor& t) {
   return t.scalar_type() == at::kBFloat16 ? PIPER_BFLOAT16 : PIPER_FLOAT16;
 }
 
-// Any [B, H, S, D] view whose rows are 16-byte aligned is read in place; anything else is copied.
+// Any [B, H, S, D] view whose rows are 16-byte aligned is read in place (the strides of axes of size 1 do
+// not count); anything else is copied.  A copy, not contiguous(): that keeps a contiguous view as it is, also
+// one that starts between two 16-byte boundaries.
 at::Tensor native_input(const at::Tensor& t) {
   TORCH_CHECK(t.dim() == 4, "piper_kernels: tensors must have shape [batch, heads, sequence, head_dim]");
-  const bool in_place = (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0 && t.stride(0) % 8 == 0 &&
-                        t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0;
-  return in_place ? t : t.contiguous();
+  bool in_place = (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0 && t.stride(3) == 1;
+  for (int64_t axis = 0; axis < 3; ++axis) in_place = in_place && (t.size(axis) == 1 || t.stride(axis) % 8 == 0);
+  return in_place ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
 piper_tensor tensor_arg(const at::Tensor& t) {
-  return piper_tensor{t.const_data_ptr(), t.stride(0), t.stride(1), t.stride(2)};
+  const auto stride = [&](int64_t axis) { return t.size(axis) == 1 ? 0 : t.stride(axis); };
+  return piper_tensor{t.const_data_ptr(), stride(0), stride(1), stride(2)};
 }
 
 // One allocation handed out in 256-byte steps.

@@ -94,12 +94,13 @@ class PreparedPiperAttention:
 
 
 def _native_input(tensor: torch.Tensor) -> tuple[torch.Tensor, native.PiperTensor]:
-    """Keep any [B,H,S,D] view whose rows are 16-byte aligned; copy anything else."""
-    strides = tensor.stride()[:3]
-    if tensor.data_ptr() % 16 != 0 or any(s % 8 != 0 for s in strides):
-        tensor = tensor.contiguous()
-        strides = tensor.stride()[:3]
-    return tensor, native.PiperTensor(tensor.data_ptr(), *strides)
+    """Keep any [B,H,S,D] view whose rows are 16-byte aligned (the strides of axes of size 1 do not count);
+    copy anything else, a contiguous view that starts between two 16-byte boundaries too."""
+    axes = list(zip(tensor.shape, tensor.stride()))[:3]
+    if tensor.data_ptr() % 16 != 0 or any(n > 1 and s % 8 != 0 for n, s in axes):
+        tensor = tensor.clone(memory_format=torch.contiguous_format)
+        axes = list(zip(tensor.shape, tensor.stride()))[:3]
+    return tensor, native.PiperTensor(tensor.data_ptr(), *(s if n > 1 else 0 for n, s in axes))
 
 
 def _native_shape(batch: int, heads: int, sq: int, sk: int, d: int) -> native.PiperShape:
@@ -244,7 +245,7 @@ def _launch_piper_attention(
             flags=flags,
             reserved=0,
             shape=_native_shape(batch, heads, sq, sk, d),
-            query=native.PiperTensor(query.data_ptr(), *query.stride()[:3]),
+            query=_native_input(query)[1],
             prepared=prepared.native_prepared(),
             output=out.data_ptr(),
             workspace=ws_ptr,

@@ -61,12 +61,13 @@ class PreparedSageAttention2pp:
 
 
 def _native_input(tensor: torch.Tensor) -> tuple[torch.Tensor, native.PiperTensor]:
-    """Keep any [B,H,S,D] view whose rows are 16-byte aligned; copy anything else."""
-    strides = tensor.stride()[:3]
-    if tensor.data_ptr() % 16 != 0 or any(s % 8 != 0 for s in strides):
-        tensor = tensor.contiguous()
-        strides = tensor.stride()[:3]
-    return tensor, native.PiperTensor(tensor.data_ptr(), *strides)
+    """Keep any [B,H,S,D] view whose rows are 16-byte aligned (the strides of axes of size 1 do not count);
+    copy anything else, a contiguous view that starts between two 16-byte boundaries too."""
+    axes = list(zip(tensor.shape, tensor.stride()))[:3]
+    if tensor.data_ptr() % 16 != 0 or any(n > 1 and s % 8 != 0 for n, s in axes):
+        tensor = tensor.clone(memory_format=torch.contiguous_format)
+        axes = list(zip(tensor.shape, tensor.stride()))[:3]
+    return tensor, native.PiperTensor(tensor.data_ptr(), *(s if n > 1 else 0 for n, s in axes))
 
 
 def _prepare_sage_attention_2pp(
@@ -167,7 +168,7 @@ def _launch_sage_attention_2pp(
         | (native.SAGE_FP16_PARTIALS if accumulate == "reference" else 0),
         reserved=0,
         shape=native.PiperShape(batch, heads, sq, sk, d),
-        query=native.PiperTensor(query.data_ptr(), *query.stride()[:3]),
+        query=_native_input(query)[1],
         prepared=prepared.native_prepared(),
         output=out.data_ptr(),
     )

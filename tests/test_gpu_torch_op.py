@@ -4,6 +4,7 @@ operators."""
 
 from __future__ import annotations
 
+import importlib
 import subprocess
 import sys
 
@@ -182,3 +183,37 @@ assert torch.equal(op(q, k, v, 0.1, False), op(q, k, v, 0.1, False))
 """
     for text in (program, direct):
         subprocess.run([sys.executable, "-c", text, str(PACKAGE_ROOT)], check=True, timeout=100)
+
+
+def _between_boundaries(x):
+    """The same values in a contiguous view that starts two bytes after a 16-byte boundary."""
+    return torch.cat([x.reshape(-1)[:1], x.reshape(-1)])[1:].view(x.shape)
+
+
+def _odd_strides(x):
+    """[1, 1, 1, D] values whose size-1 axes carry odd strides."""
+    return torch.as_strided(x, x.shape, (7, 5, 3, 1))
+
+
+@pytest.mark.parametrize("path", ["piper_attention", "sage_attention_2pp"])
+def test_python_inputs_are_aligned_or_copied(path) -> None:
+    module = importlib.import_module(f"piper_kernels.attention.{path}.hip")
+    x = torch.randn(2, 3, 8, 64).half()
+    got, arg = module._native_input(_between_boundaries(x))
+    assert torch.equal(got, x) and arg.data == got.data_ptr() and arg.data % 16 == 0
+    one = torch.randn(1, 1, 1, 64).half()
+    got, arg = module._native_input(_odd_strides(one))
+    assert got.data_ptr() == one.data_ptr() and (arg.stride_batch, arg.stride_head, arg.stride_seq) == (0, 0, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("operator", OPERATORS)
+def test_contiguous_views_off_the_alignment_run(operator, gfx950_device) -> None:
+    log(f"[case] torch op {operator} contiguous views between 16-byte boundaries, odd strides of size-1 axes")
+    public, python = OPERATORS[operator]
+    for view, shape in ((_between_boundaries, (2, 3, 77, 77)), (_odd_strides, (1, 1, 1, 1))):
+        inputs = _inputs(*shape, 64, torch.float16, gfx950_device)
+        with torch.no_grad():
+            want = public(*inputs)
+            assert torch.equal(public(*map(view, inputs)), want)
+            assert torch.equal(python(*map(view, inputs), 64**-0.5, False), python(*inputs, 64**-0.5, False))
