@@ -70,7 +70,6 @@ int32_t dtype_code(const at::Tensor& t) {
 // not count); anything else is copied.  A copy, not contiguous(): that keeps a contiguous view as it is, also
 // one that starts between two 16-byte boundaries.
 at::Tensor native_input(const at::Tensor& t) {
-  TORCH_CHECK(t.dim() == 4, "piper_kernels: tensors must have shape [batch, heads, sequence, head_dim]");
   bool in_place = (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0 && t.stride(3) == 1;
   for (int64_t axis = 0; axis < 3; ++axis) in_place = in_place && (t.size(axis) == 1 || t.stride(axis) % 8 == 0);
   return in_place ? t : t.clone(at::MemoryFormat::Contiguous);
@@ -91,6 +90,21 @@ struct Arena {
   }
 };
 
+// The kernels read key and value by the query's shape, type and device: what the public functions refuse is
+// refused here too, where a program can call the op itself.  Returns the device.
+c10::Device checked_device(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
+  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4,
+              "piper_kernels: tensors must have shape [batch, heads, sequence, head_dim]");
+  TORCH_CHECK(k.device() == q.device() && v.device() == q.device(),
+              "piper_kernels: query, key and value must share a device");
+  TORCH_CHECK(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type(),
+              "piper_kernels: query, key and value must share a dtype");
+  TORCH_CHECK(k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(1) == q.size(1) && k.size(3) == q.size(3),
+              "piper_kernels: batch, heads and head_dim must agree and key and value lengths match, got ", q.sizes(), ", ",
+              k.sizes(), " and ", v.sizes());
+  return q.device();
+}
+
 // What both operators' calls share: inputs, shape, output, stream.
 struct Call {
   c10::OptionalDeviceGuard guard;
@@ -101,7 +115,7 @@ struct Call {
   void* handle;
 
   Call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v)
-      : guard(q.device()),
+      : guard(checked_device(q, k, v)),
         query(native_input(q)),
         key(native_input(k)),
         value(native_input(v)),

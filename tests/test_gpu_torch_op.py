@@ -1,6 +1,6 @@
-"""The native torch kernels (csrc/torch_op.cpp) against the Python path over the same C ABI: every option, inputs read in place and inputs that must be copied, a side stream whose inputs are freed
-at once, replays of a captured graph; errors stay Python exceptions; the plan source covers both
-operators."""
+"""The native torch kernels (csrc/torch_op.cpp) against the Python path over the same C ABI: every option,
+inputs read in place and inputs that must be copied, a side stream whose inputs are freed at once,
+replays of a captured graph; errors stay Python exceptions; the plan source covers both operators."""
 
 from __future__ import annotations
 
@@ -105,6 +105,24 @@ def test_errors_are_python_exceptions(gfx950_device) -> None:
     q = q.half()
     with pytest.raises(RuntimeError, match="scale must be finite and positive"):
         op(q, q, q, 0.0, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("operator", ["piper_attention", "sage_attention_2pp"])
+def test_the_op_refuses_tensors_that_do_not_belong_together(operator, gfx950_device) -> None:
+    """The kernels read key and value by the query's shape and type; nothing is launched here."""
+    native.load_torch_kernels()
+    op = getattr(torch.ops.piper_kernels, operator)
+    q = torch.zeros((1, 2, 8, 64), dtype=torch.float16, device=gfx950_device)
+    for key, value, text in [
+        (q, q[:, :, :7], "key and value lengths match"),
+        (q[:, :1], q[:, :1], "heads and head_dim must agree"),
+        (q.bfloat16(), q.bfloat16(), "share a dtype"),
+        (q.cpu(), q.cpu(), "share a device"),
+        (q[0], q[0], "must have shape"),
+    ]:
+        with pytest.raises(RuntimeError, match=text):
+            op(q, key, value, 0.125, False)
 
 
 def test_plan_source_asks_the_package(monkeypatch) -> None:
