@@ -169,9 +169,10 @@ typedef struct piper_layout {
                                       for piper_attention_forward_fused, which quantises Q itself */
 #define PIPER_PREPARE_QK_PER_THREAD 2 /* Q and K scales per thread group (the reference's
                                          "per_thread"); default: one per block ("per_warp") */
-#define PIPER_PREPARE_SELF_MEAN 4 /* diagnostic, for tests: every single-pass chunk that would wait
-                                     for its tensor's mean computes it itself at once (the bounded
-                                     wait's fallback; same bits, slower) */
+#define PIPER_PREPARE_SELF_MEAN 4 /* diagnostic, for tests (both operators' preps): every single-pass
+                                     chunk that would wait for its tensor's mean (SageAttention2++'s V:
+                                     its channel scales) computes it itself at once (the bounded wait's
+                                     fallback; same bits, slower) */
 
 typedef struct piper_prepare_args {
   int32_t abi_version; /* PIPER_ABI_VERSION */
@@ -295,7 +296,8 @@ typedef struct piper_sage_layout {
 typedef struct piper_sage_prepare_args {
   int32_t abi_version; /* PIPER_ABI_VERSION */
   int32_t dtype;       /* PIPER_FLOAT16 or PIPER_BFLOAT16: dtype of key and value */
-  int32_t flags;       /* 0 or PIPER_PREPARE_QK_PER_THREAD (K scales per thread group) */
+  int32_t flags;       /* OR of PIPER_PREPARE_QK_PER_THREAD (K scales per thread group) and
+                          PIPER_PREPARE_SELF_MEAN */
   int32_t reserved;    /* 0 */
   piper_shape shape;   /* query_length is not used by the prep */
   piper_tensor key;
@@ -391,7 +393,10 @@ int piper_attention_forward_fused(const piper_attention_fused_args* args, void* 
 int piper_attention_forward_balanced(const piper_attention_fused_args* args, void* stream);
 
 /* SageAttention2++: buffer sizes, K/V prep (statistics, INT8 K, FP8 V^T tile records) and the
- * fused attention kernel (INT8 QK, FP8 PV on v_mfma_f32_32x32x64_f8f6f4, FP32 accumulation). */
+ * fused attention kernel (INT8 QK, FP8 PV on v_mfma_f32_32x32x64_f8f6f4, FP32 accumulation).
+ * The prep takes piper_prepare's routes, the waiting single pass among them: a chunk whose bounded wait
+ * for its tensor's statistic ends computes it itself, same bits, but this prep's workspace has no status
+ * word, so such a chunk is not counted. */
 int piper_sage_prepared_layout(const piper_shape* shape, piper_sage_layout* layout);
 int piper_sage_prepare(const piper_sage_prepare_args* args, void* stream);
 int piper_sage_attention_forward(const piper_sage_attention_args* args, void* stream);

@@ -478,7 +478,8 @@ int piper_sage_prepare(const piper_sage_prepare_args* a, void* stream) {
   if (a->dtype != PIPER_FLOAT16 && a->dtype != PIPER_BFLOAT16)
     return fail(PIPER_ERROR_UNSUPPORTED, "input dtype must be float16 or bfloat16");
   if (int st = check_shape(&a->shape)) return st;
-  if ((a->flags & ~PIPER_PREPARE_QK_PER_THREAD) != 0) return fail(PIPER_ERROR_UNSUPPORTED, "unknown flags %d", a->flags);
+  if ((a->flags & ~(PIPER_PREPARE_QK_PER_THREAD | PIPER_PREPARE_SELF_MEAN)) != 0)
+    return fail(PIPER_ERROR_UNSUPPORTED, "unknown flags %d", a->flags);
   if (int st = check_input("key", a->key)) return st;
   if (int st = check_input("value", a->value)) return st;
   const piper_sage_prepared& o = a->prepared;
@@ -528,7 +529,7 @@ int piper_sage_prepare(const piper_sage_prepare_args* a, void* stream) {
 
   piper::PrepDevice dev{};
   if (int st = device_topology(&dev.cus, &dev.xccs)) return st;
-  dev.spin_limit = piper::kPrepSpinLimit;
+  dev.spin_limit = (a->flags & PIPER_PREPARE_SELF_MEAN) ? 0 : piper::kPrepSpinLimit;
 
   const hipError_t err =
       piper::launch_sage_prep(a->dtype == PIPER_BFLOAT16, static_cast<int>(s.head_dim), mp, qp, dev,

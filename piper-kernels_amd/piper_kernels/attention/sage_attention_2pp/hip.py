@@ -80,11 +80,13 @@ def _prepare_sage_attention_2pp(
     plan: MI355XPlan | None = None,
     workspace: torch.Tensor | None = None,
     qk_granularity: str = "per_thread",
+    prep_flags: int = 0,
 ) -> PreparedSageAttention2pp:
     """K/V statistics, INT8 K and FP8 V on the GPU (one HIP prep pipeline); allocate the output.
 
     ``qk_granularity``: ``"per_thread"`` (the default of the reference's portable path,
     ``sage_attention_2pp/reference.py:35``) or ``"per_warp"`` (its grouped SM12x Triton path).
+    ``prep_flags`` adds ``native.PREPARE_SELF_MEAN`` (diagnostic: the single pass's fallback; same outputs).
     """
     if qk_granularity not in ("per_warp", "per_thread"):
         raise ValueError(f"unknown Q/K quantization granularity: {qk_granularity}")
@@ -122,7 +124,8 @@ def _prepare_sage_attention_2pp(
     args = native.PiperSagePrepareArgs(
         abi_version=native.ABI_VERSION,
         dtype=_DTYPE_CODES[key.dtype],
-        flags=native.PREPARE_QK_PER_THREAD if qk_granularity == "per_thread" else 0,
+        flags=(native.PREPARE_QK_PER_THREAD if qk_granularity == "per_thread" else 0)
+        | (prep_flags & native.PREPARE_SELF_MEAN),
         shape=shape,
         key=k_arg,
         value=v_arg,

@@ -1,7 +1,7 @@
 """The prep's routes (csrc/prep.hip launch_prep_typed) agree bit for bit: a batch-head's codes, scales
 and statistics do not depend on how many other batch-heads the call has, while the route does (short,
-two-pass, single pass).  Lengths at the edges of 16-row blocks, 64-row units and 256-row chunks against
-the oracle, on strided inputs."""
+two-pass, single pass).  Lengths at the edges of 16-row blocks, 64-row units and 256-row chunks, and just
+beyond the single pass's longest (the statistics' own kernel), against the oracle, on strided inputs."""
 
 from __future__ import annotations
 
@@ -61,8 +61,17 @@ def test_routes_agree_bit_for_bit(route, operator, causal, gfx950_device) -> Non
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("s", [1, 15, 16, 17, 64, 255, 256, 257, 1023, 1024, 1025, 1300])
 def test_edge_lengths_match_the_oracle(s, d, gfx950_device) -> None:
-    log(f"[case] prep edge length {s} D={d}")
-    q, k, v = _inputs(1, 2, s, d, 7 * s + d)
+    _check_against_the_oracle(s, d, 2, gfx950_device)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_past_the_single_pass_matches_the_oracle(d, gfx950_device) -> None:
+    _check_against_the_oracle(32768 + 257, d, 1, gfx950_device)
+
+
+def _check_against_the_oracle(s, d, heads, gfx950_device) -> None:
+    log(f"[case] prep length {s} D={d}")
+    q, k, v = _inputs(1, heads, s, d, 7 * s + d)
     for causal in (False, True):
         prepared = gpu_prepare(q, k, v, d**-0.5, causal, gfx950_device, qk_granularity="per_thread")
         assert_prep_bit_exact(prepared_numpy(prepared), oracle.prepare(q, k, v, causal, "per_thread"), prepared.shape, causal)

@@ -1,7 +1,7 @@
 """piper_prepare_static (no caller workspace: the prep's workspace lives in the library's static
 per-GPU scratch) against piper_prepare, through the C ABI on MI355X: every prepared byte the
 header specifies and the attention output equal, on calls in a row, each smaller than the one
-before (non-causal single pass, the three-kernel path at D = 64, causal single pass); and a call
+before (non-causal single pass, causal single pass, two-pass at D = 64, short); and a call
 on preallocated buffers makes no allocation at all."""
 
 from __future__ import annotations
@@ -15,9 +15,11 @@ from _parity import gpu_attention, log, prepared_numpy
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # (B, H, Sq, Sk, D, dtype, causal): the second is smaller and reuses the scratch the first filled
-    (1, 4, 4096, 4096, 128, torch.float16, False),
-    (1, 2, 300, 193, 64, torch.bfloat16, False),
+    # (B, H, Sq, Sk, D, dtype, causal): each is smaller and reuses the scratch that the first filled; more
+    # than 32 chunks of 256 keys take the single pass, up to 4 in a small grid the short prep
+    (1, 4, 700, 9000, 128, torch.float16, False),
+    (1, 2, 8300, 8300, 128, torch.bfloat16, True),
+    (1, 2, 300, 2100, 64, torch.bfloat16, False),
     (1, 2, 192, 192, 128, torch.bfloat16, True),
 ]
 
