@@ -387,9 +387,9 @@ int piper_attention_workspace_bytes(const piper_shape* shape, int32_t plan, int6
 int piper_attention_forward_fused(const piper_attention_fused_args* args, void* stream);
 
 /* piper_attention_forward_fused, free to run a small causal grid as key streams: the waves of a workgroup
- * share its query rows, each takes every second or fourth key tile, and their FP32 sums are added at
- * the end.  Results equal piper_attention_forward_fused's to rounding, not bit for bit, and depend on
- * the number of batch-heads (the grid) in that rounding.  What the custom op calls. */
+ * share its query rows, each computes the probability codes of every second or fourth key tile and adds all
+ * tiles, in order, to its share of the features.  Bit for bit piper_attention_forward_fused's results, faster
+ * on small causal grids.  What the custom op calls. */
 int piper_attention_forward_balanced(const piper_attention_fused_args* args, void* stream);
 
 /* SageAttention2++: buffer sizes, K/V prep (statistics, INT8 K, FP8 V^T tile records) and the
@@ -401,8 +401,7 @@ int piper_sage_prepared_layout(const piper_shape* shape, piper_sage_layout* layo
 int piper_sage_prepare(const piper_sage_prepare_args* args, void* stream);
 int piper_sage_attention_forward(const piper_sage_attention_args* args, void* stream);
 
-/* The same, free to run a small grid as key streams (piper_attention_forward_balanced): every probability
- * code is the other entry point's, the FP32 sums are added in another order. */
+/* The same, free to run a small grid as key streams (piper_attention_forward_balanced), bit for bit. */
 int piper_sage_attention_forward_balanced(const piper_sage_attention_args* args, void* stream);
 
 /* Thread-local description of the last failure on this thread ("" if none). */

@@ -245,7 +245,8 @@ int launch_attention_call(int32_t abi_version, int32_t output_dtype, int32_t is_
   if (balanced && is_causal && waves == 3 && !work_queue) {
     int cus = 0, xccs = 0;
     if (int st = device_topology(&cus, &xccs)) return st;
-    ap.key_streams = piper::small_grid_streams(false, true, static_cast<long>(ap.query_tiles) * ap.batch_heads, ap.nkb, cus);
+    ap.key_streams = piper::small_grid_streams(false, true, static_cast<int>(s.head_dim),
+                                               static_cast<long>(ap.query_tiles) * ap.batch_heads, ap.nkb, cus);
     ap.query_tiles = static_cast<int>(ceil_div(s.query_length, block_m / ap.key_streams));
   }
   if (static_cast<int64_t>(ap.query_tiles) * ap.batch_heads * ap.key_parts > 0x7fffffff)
@@ -592,8 +593,8 @@ static int sage_attention_call(const piper_sage_attention_args* a, bool balanced
   if (balanced && waves == 3 && !sp.fp16_partials) {
     int cus = 0, xccs = 0;
     if (int st = device_topology(&cus, &xccs)) return st;
-    sp.key_streams = piper::small_grid_streams(true, a->is_causal != 0, static_cast<long>(sp.query_tiles) * sp.batch_heads,
-                                               sp.nkb, cus);
+    sp.key_streams = piper::small_grid_streams(true, a->is_causal != 0, static_cast<int>(s.head_dim),
+                                               static_cast<long>(sp.query_tiles) * sp.batch_heads, sp.nkb, cus);
     sp.query_tiles = static_cast<int>(ceil_div(s.query_length, 128 / sp.key_streams));
   }
   if (static_cast<int64_t>(sp.query_tiles) * sp.batch_heads > 0x7fffffff)

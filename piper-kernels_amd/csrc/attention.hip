@@ -43,15 +43,26 @@ struct TileLayout : StagePieces<kv_tile_bytes(D), NW> {  // the tile record is t
   static constexpr int kCorrOffset = kv_corr_offset(D);  // D ints: biased 128 * colsum
 };
 
+// What a wave of the key-stream kernel hands on of its block: the UINT8 codes, the four partial sums of
+// e / (255 vs) per lane, and the block maximum.
+struct BlockCodes {
+  uint32_t pw[8];
+  float ps[4];
+  float mx;
+};
+
 // Online softmax and PV of one 64-key block (block index t, staged at `stage`) for one wave.
 // ct[g]: the score multiplier q_scale * k_scale * softmax_scale * log2(e) of key thread group g
 // (keys k with (k % 8) / 2 == g; all four equal for per-block K scales).  Output register r of
 // lane half h holds key 16h + r (and 32 + 16h + r), so register 4q + i belongs to group
 // 2 (q % 2) + i / 2.
-template <int D, int NW, bool kCausal>
+// kCodes: the scores and codes only, into `codes`; num, den and the frame are left alone (fold_block adds the
+// block to them, with the same arithmetic).
+template <int D, int NW, bool kCausal, bool kCodes = false>
 __device__ __forceinline__ void block_update(const char* stage, const v16i (&s)[2], const float (&ct)[4], int t,
                                              int q0, int n, int h, uint32_t sel, float (&num)[D / 32][16],
-                                             float (&den)[4], float& mref, float& mlim, float& kref) {
+                                             float (&den)[4], float& mref, float& mlim, float& kref,
+                                             BlockCodes* codes = nullptr) {
   using L = TileLayout<D, NW>;
   constexpr int kChunksD = D / 32;
 
@@ -90,8 +101,8 @@ __device__ __forceinline__ void block_update(const char* stage, const v16i (&s)[
 
   // ---- lazy rescale of num/den when the block maximum outgrows the reference by 2^8 ----
   // (kept beside mref: mlim = mref + 2^8 and kref = 255 * 2^-mref)
-  const bool grow = mx > mlim;
-  if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+  const bool grow = !kCodes && mx > mlim;
+  if (!kCodes && __builtin_amdgcn_ballot_w64(grow) != 0) {
     const float alpha = grow ? __builtin_amdgcn_exp2f(mref - mx) : 1.0f;
     if (grow) {
       mref = mx;
@@ -175,6 +186,14 @@ __device__ __forceinline__ void block_update(const char* stage, const v16i (&s)[
       pw[4 + q] = pack_codes(f0, f1, f2, f3);
     }
     dw = beta;
+  }
+  if constexpr (kCodes) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) codes->pw[q] = pw[q];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) codes->ps[q] = ps[q];
+    codes->mx = mx;
+    return;
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) den[q] = fmaf(ps[q], dw, den[q]);
@@ -582,26 +601,152 @@ attention_w3_kernel(const AttnParams p) {
   w3_tile<D, kCausal, kOut, kPerThread, kCausal || kSplit, kSplit>(p, smem, tc, part, threadIdx.x & 63);
 }
 
-// Key streams: KS of a workgroup's four waves share 32 queries and take every KS-th key tile each, so a
-// grid too small to give every SIMD several waves gets KS times the waves, each with 1 / KS of the key
-// loop, and the sums meet in LDS at the end: no partial sums in memory, no merge kernel.  One iteration
-// stages KS consecutive tile records (double-buffered, as attention_w3_kernel); wave w handles query
-// group w % (4 / KS) and tile KS i + w / (4 / KS) of iteration i.  Per-block arithmetic is
-// block_update's; the waves' sums are aligned on their largest reference maximum as by
-// attention_merge_kernel, so results equal the sequential kernel's to rounding.  A lone wave of a SIMD
-// issues one VALU instruction per ~5.5 cycles and takes 1.2-1.5 us per key tile whatever the grid, which
-// is what bounds small grids: B1 H8 S1024 D64 12.9 + 4.2 us in four key parts and a merge, see
-// key_streams in kernels.h for the sizes that take this kernel and what they measured.
+// Where a key-stream wave leaves its block for the others: codes (two 16-byte pieces per lane), block maxima
+// and the denominator's partial sums, in the tile's K rows, which every wave that reads them has read by then.  The K
+// rows of a D = 64 tile are too small for two query groups' partial sums, which then lie apart.
+template <int D, int KS>
+struct StreamExchange {
+  static constexpr int kGroups = 4 / KS;
+  static constexpr int kMaxima = 2048;
+  static constexpr bool kApart = D == 64 && KS == 2;
+  static constexpr int kSums = kMaxima + 256;
+  static constexpr int kSlot = kv_v_offset(D) / kGroups;
+  static constexpr int kApartBytes = kApart ? 4 * 1024 : 0;
+  static_assert((kApart ? kSums : kSums + 1024) <= kSlot && kSlot % 16 == 0, "a wave's block fits its share of the K rows");
+};
+
+// The numerator and denominator of one query group over tiles [t, t + KS) of an iteration, in tile order and
+// with block_update's arithmetic, for the features of StreamShare: the same bits as one wave that runs
+// the tiles one after another.  The MFMA chains in flight: two chunks of a tile, or every tile of one chunk.
+template <int D, int KS>
+__device__ __forceinline__ void fold_blocks(const char* stages, const char* sums, int t, int wave_tiles, int group, int part,
+                                            int lane, float (&num)[StreamShare<D, KS>::kChunks][StreamShare<D, KS>::kRegs],
+                                            float (&den)[4], float& mref, float& mlim, float& kref) {
+  using L = TileLayout<D, 4>;
+  using S = StreamShare<D, KS>;
+  using X = StreamExchange<D, KS>;
+  constexpr int kTiles = S::kChunks == 2 ? 1 : KS;  // tiles in flight
+  constexpr int kChains = kTiles * S::kChunks;
+  const int h = lane >> 5;
+  const int chunk = S::chunk(part);
+  const int half = S::half(part);
+  const int vrow = (32 * chunk + ((lane & 31) ^ (16 * half))) * L::kVStride + 16 * h;
+#pragma unroll
+  for (int k0 = 0; k0 < KS; k0 += kTiles) {
+    if (t + k0 >= wave_tiles) break;
+    v16i acc[kChains];
+    v4i a0[kChains], a1[kChains], p0[kTiles], p1[kTiles];
+    float mx[kTiles];
+    float4 ps[kTiles];
+#pragma unroll
+    for (int u = 0; u < kChains; ++u) {
+      const int c = u % S::kChunks;
+      const char* stage = stages + (k0 + u / S::kChunks) * L::kStageBytes;
+      if (c == 0) {
+        // a tile past the end: what its slot holds is read and not used
+        const int i = u / S::kChunks;
+        const char* slot = stage + group * X::kSlot;
+        p0[i] = *reinterpret_cast<const v4i*>(slot + 16 * lane);
+        p1[i] = *reinterpret_cast<const v4i*>(slot + 1024 + 16 * lane);
+        mx[i] = *reinterpret_cast<const float*>(slot + X::kMaxima + 4 * lane);
+        const char* from = X::kApart ? sums + ((k0 + i) * X::kGroups + group) * 1024 : slot + X::kSums;
+        ps[i] = *reinterpret_cast<const float4*>(from + 16 * lane);
+      }
+      const v4i* corr4 = reinterpret_cast<const v4i*>(stage + L::kCorrOffset) + 8 * (chunk + c) + 4 * half + h;
+      if constexpr (S::kRegs < 16) asm("" : "=v"(acc[u]));  // registers 8 to 15 are no one's features
+#pragma unroll
+      for (int g = 0; 4 * g < S::kRegs; ++g) {
+        const v4i c4 = corr4[2 * g];
+        acc[u][4 * g + 0] = c4[0];
+        acc[u][4 * g + 1] = c4[1];
+        acc[u][4 * g + 2] = c4[2];
+        acc[u][4 * g + 3] = c4[3];
+      }
+      const char* v = stage + L::kKBytes + vrow + 32 * c * L::kVStride;
+      a0[u] = *reinterpret_cast<const v4i*>(v);
+      a1[u] = *reinterpret_cast<const v4i*>(v + 32);
+    }
+    // four tiles: every load issued before the first wait (the scheduler otherwise waits tile by tile)
+    if constexpr (kTiles == 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kChains; ++u)
+      acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0[u], p0[u / S::kChunks], acc[u], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < kChains; ++u)
+      acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1[u], p1[u / S::kChunks], acc[u], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < kTiles; ++u) {
+      if (t + k0 + u >= wave_tiles) break;
+      const bool grow = mx[u] > mlim;
+      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+        const float alpha = grow ? __builtin_amdgcn_exp2f(mref - mx[u]) : 1.0f;
+        if (grow) {
+          mref = mx[u];
+          mlim = mx[u] + kLazyRescale;
+          kref = __builtin_amdgcn_exp2f(kLog2Of255 - mx[u]);
+        }
+#pragma unroll
+        for (int c = 0; c < S::kChunks; ++c)
+#pragma unroll
+          for (int r = 0; r < S::kRegs; ++r) num[c][r] *= alpha;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) den[q] *= alpha;
+      }
+      float weight = __builtin_amdgcn_exp2f(mx[u] - mref);
+      float dw = kref;
+      if (__builtin_amdgcn_ballot_w64(!(fabsf(mx[u]) <= kDirectRange)) != 0) {
+        if (mx[u] == -__builtin_inff()) weight = 0.0f;
+        dw = weight;
+      }
+      den[0] = fmaf(ps[u].x, dw, den[0]);
+      den[1] = fmaf(ps[u].y, dw, den[1]);
+      den[2] = fmaf(ps[u].z, dw, den[2]);
+      den[3] = fmaf(ps[u].w, dw, den[3]);
+#pragma unroll
+      for (int c = 0; c < S::kChunks; ++c)
+#pragma unroll
+        for (int r = 0; r < S::kRegs; ++r) num[c][r] = fmaf(unbias(acc[u * S::kChunks + c][r]), weight, num[c][r]);
+    }
+  }
+}
+
+// Key streams: KS of a workgroup's four waves share 32 queries, so a grid too small to give every SIMD
+// several waves gets KS times the waves, each with 1 / KS of the work, and no partial sums in memory.  One
+// iteration stages KS consecutive tile records (double-buffered, as attention_w3_kernel); wave w handles
+// query group w % (4 / KS) and tile KS i + w / (4 / KS) of iteration i.  A lone wave of a SIMD issues one
+// VALU instruction per ~5.5 cycles and takes 1.2-1.5 us per key tile whatever the grid, which is what bounds
+// small grids; stream_workgroups and small_grid_streams in kernels.h have the sizes that take this kernel
+// and what they measured.
+//
+// Causal (kOrdered): a wave computes its tile's scores and probability codes, most of a tile's instructions,
+// and hands the codes on through the tile's K rows, dead by then; each wave then adds all KS tiles, in order, to
+// its own 1 / KS of the features (fold_blocks).  The sums grow in the same order as in one wave that takes
+// the tiles one by one, so the output equals the other kernels' bit for bit: how many batch-heads a causal
+// call has chooses its kernel, not a row's bits.
+// Non-causal, where the plan's key parts choose the streams: each wave keeps the sums of its own tiles, and
+// they are aligned on their largest reference maximum at the end, as by attention_merge_kernel, so results equal
+// the sequential kernel's to rounding.  That saves the exchange: us at B1 H8 S1024 D64 (four streams)
+// 10.2 against 12.1 in order, B1 H16 S2048 D128 (two) 43.0 against 47.2; causal, for which only the order
+// leaves a row's bits alone, B2 H16 S1531 D128 36.3 (two; 34.7 merged at the end, 42 without streams), B1 H12
+// S4096 72.1 (64.1; 98), B1 H8 S1024 D64 11.6 (four; 10.2; 22).
+//
+// The work-group size attribute counts 512 threads for four streams, where LDS leaves one workgroup per
+// CU: that makes two waves per SIMD a possible target, for which the compiler keeps to 256 registers without
+// accumulation registers; no launch has more than 256 threads.
 template <int D, bool kCausal, int kOut, bool kPerThread, int KS>
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, KS == 4 ? 512 : 256), amdgpu_waves_per_eu(KS == 4 ? 2 : stream_workgroups(D, KS), KS == 4 ? 2 : stream_workgroups(D, KS))))
 attention_streams_kernel(const AttnParams p) {
   using L = TileLayout<D, 4>;
+  using S = StreamShare<D, KS>;
+  using X = StreamExchange<D, KS>;
+  constexpr bool kOrdered = kCausal;
   constexpr int kChunksD = D / 32;
+  constexpr int kChunks = kOrdered ? S::kChunks : kChunksD;  // this wave's share of the numerator
+  constexpr int kRegs = kOrdered ? S::kRegs : 16;
   constexpr int kGroups = 4 / KS;               // query groups of a workgroup
   constexpr int kStage = KS * L::kStageBytes;
   constexpr int kRounds = stream_rounds<L, KS>();
-  constexpr int kShare = 4 * kChunksD / KS;     // four-feature groups that a wave writes at the end
-  __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
+  __shared__ __attribute__((aligned(16))) char smem[2 * kStage + (kOrdered ? X::kApartBytes : 0)];
   static_assert(4 * (D * 32 * 4 + 512) <= 2 * kStage, "every wave's sums fit the stages");
 
   const int lane = threadIdx.x & 63;
@@ -653,11 +798,11 @@ attention_streams_kernel(const AttnParams p) {
     cq = quantize_query_block<D, kPerThread>(p, q0, n, raw, qf) * p.score_multiplier;
   }
 
-  float num[kChunksD][16];
+  float num[kChunks][kRegs];
 #pragma unroll
-  for (int j = 0; j < kChunksD; ++j)
+  for (int c = 0; c < kChunks; ++c)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) num[j][r] = 0.0f;
+    for (int r = 0; r < kRegs; ++r) num[c][r] = 0.0f;
   float den[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   float mref = -__builtin_inff();
   float mlim = -__builtin_inff();
@@ -670,11 +815,12 @@ attention_streams_kernel(const AttnParams p) {
     stage_barrier<0>();  // this iteration's records landed, every read of the last one's is done
     if (i + 1 < steps) copy_tiles<L, KS>(p, smem + ((i + 1) & 1) * kStage, bh, KS * (i + 1), tiles, wave, lane);
     const int t = KS * i + part;
+    char* stages = smem + (i & 1) * kStage;
+    char* stage = stages + part * L::kStageBytes;
+    v16i sc[2];
+    float ct[4];
     if (t < wave_tiles) {
-      const char* stage = smem + (i & 1) * kStage + part * L::kStageBytes;
-      v16i sc[2];
       block_scores<D, L>(stage, qf, h, krow, sc);
-      float ct[4];
       if constexpr (kPerThread) {
         const float4 ks = *reinterpret_cast<const float4*>(stage + D);
         ct[0] = cq * ks.x;
@@ -684,59 +830,95 @@ attention_streams_kernel(const AttnParams p) {
       } else {
         ct[0] = ct[1] = ct[2] = ct[3] = cq * *reinterpret_cast<const float*>(stage + D);
       }
+    }
+    if constexpr (kOrdered) {
+      if constexpr (kGroups > 1) stream_barrier();  // every wave has read the K rows (else only this one does)
+      if (t < wave_tiles) {
+        BlockCodes codes;
+        float no_num[kChunksD][16], no_den[4], no_frame[3];  // not touched
+        block_update<D, 4, kCausal, true>(stage, sc, ct, t, q0, n, h, sel, no_num, no_den, no_frame[0], no_frame[1],
+                                          no_frame[2], &codes);
+        char* slot = stage + group * X::kSlot;
+        *reinterpret_cast<uint4*>(slot + 16 * lane) = make_uint4(codes.pw[0], codes.pw[1], codes.pw[2], codes.pw[3]);
+        *reinterpret_cast<uint4*>(slot + 1024 + 16 * lane) = make_uint4(codes.pw[4], codes.pw[5], codes.pw[6], codes.pw[7]);
+        *reinterpret_cast<float*>(slot + X::kMaxima + 4 * lane) = codes.mx;
+        char* to = X::kApart ? smem + 2 * kStage + wave * 1024 : slot + X::kSums;
+        *reinterpret_cast<float4*>(to + 16 * lane) = make_float4(codes.ps[0], codes.ps[1], codes.ps[2], codes.ps[3]);
+      }
+      stream_barrier();  // every wave's block is there
+      fold_blocks<D, KS>(stages, smem + 2 * kStage, KS * i, wave_tiles, group, part, lane, num, den, mref, mlim, kref);
+    } else if (t < wave_tiles) {
       block_update<D, 4, kCausal>(stage, sc, ct, t, q0, n, h, sel, num, den, mref, mlim, kref);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const float den_total = cross_half_sum((den[0] + den[1]) + (den[2] + den[3]));
-  __syncthreads();  // every wave is done with the stages
 
-  // every wave's sums: [wave][four-feature group][lane] float4, then [wave][lane] float2 (den, mref)
-  float4* sums = reinterpret_cast<float4*>(smem);
-  float2* stats = reinterpret_cast<float2*>(smem + 4 * D * 32 * 4);
+  const float den_total = cross_half_sum((den[0] + den[1]) + (den[2] + den[3]));
+  if constexpr (kOrdered) {
+    const int query = q0 + n;
+    if (!wave_live || query >= p.query_length) return;
+    const float rden = (1.0f / 255.0f) / fmaxf(den_total, 1e-30f);  // the numerator holds 255 x the reference's
+    const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
 #pragma unroll
-  for (int j = 0; j < kChunksD; ++j)
+    for (int c = 0; c < S::kChunks; ++c) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      sums[(wave * 4 * kChunksD + 4 * j + g) * 64 + lane] =
-          make_float4(num[j][4 * g + 0], num[j][4 * g + 1], num[j][4 * g + 2], num[j][4 * g + 3]);
-  stats[wave * 64 + lane] = make_float2(den_total, mref);
-  __syncthreads();
-  const int query = q0 + n;
-  if (!wave_live || query >= p.query_length) return;
-  float2 st[KS];
-  float top = -__builtin_inff();
+      for (int g = 0; 4 * g < S::kRegs; ++g) {
+        const int d0 = 32 * (S::chunk(part) + c) + 16 * S::half(part) + 8 * g + 4 * h;
+        // the sequential kernel's epilogue, whose causal mean is zero
+        store4<kOut>(p.output, out_row + d0, fmaf(num[c][4 * g + 0], rden, 0.0f), fmaf(num[c][4 * g + 1], rden, 0.0f),
+                     fmaf(num[c][4 * g + 2], rden, 0.0f), fmaf(num[c][4 * g + 3], rden, 0.0f));
+      }
+    }
+  } else {
+    constexpr int kShare = 4 * kChunksD / KS;  // four-feature groups that a wave writes
+    __syncthreads();                           // every wave is done with the stages
+
+    // every wave's sums: [wave][four-feature group][lane] float4, then [wave][lane] float2 (den, mref)
+    float4* sums = reinterpret_cast<float4*>(smem);
+    float2* stats = reinterpret_cast<float2*>(smem + 4 * D * 32 * 4);
 #pragma unroll
-  for (int k = 0; k < KS; ++k) {
-    st[k] = stats[(k * kGroups + group) * 64 + lane];
-    top = fmaxf(top, st[k].y);
-  }
-  float den_sum = 0.0f;
-  float weight[KS];
+    for (int j = 0; j < kChunksD; ++j)
 #pragma unroll
-  for (int k = 0; k < KS; ++k) {
-    weight[k] = st[k].y == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(st[k].y - top);
-    den_sum = fmaf(st[k].x, weight[k], den_sum);
-  }
-  const float rden = (1.0f / 255.0f) / fmaxf(den_sum, 1e-30f);
-  const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
-#pragma unroll
-  for (int i = 0; i < kShare; ++i) {
-    const int four = part * kShare + i;  // this wave's share of the features: 4 j + g
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int g = 0; g < 4; ++g)
+        sums[(wave * 4 * kChunksD + 4 * j + g) * 64 + lane] =
+            make_float4(num[j][4 * g + 0], num[j][4 * g + 1], num[j][4 * g + 2], num[j][4 * g + 3]);
+    stats[wave * 64 + lane] = make_float2(den_total, mref);
+    __syncthreads();
+    const int query = q0 + n;
+    if (!wave_live || query >= p.query_length) return;
+    float2 st[KS];
+    float top = -__builtin_inff();
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
-      const float4 v = sums[((k * kGroups + group) * 4 * kChunksD + four) * 64 + lane];
-      acc.x = fmaf(v.x, weight[k], acc.x);
-      acc.y = fmaf(v.y, weight[k], acc.y);
-      acc.z = fmaf(v.z, weight[k], acc.z);
-      acc.w = fmaf(v.w, weight[k], acc.w);
+      st[k] = stats[(k * kGroups + group) * 64 + lane];
+      top = fmaxf(top, st[k].y);
     }
-    const int d0 = 8 * four + 4 * h;  // 32 j + 8 g + 4 h
-    float4 m = make_float4(0.f, 0.f, 0.f, 0.f);
-    if constexpr (!kCausal) m = *reinterpret_cast<const float4*>(p.value_mean + static_cast<long>(bh) * D + d0);
-    store4<kOut>(p.output, out_row + d0, fmaf(acc.x, rden, m.x), fmaf(acc.y, rden, m.y), fmaf(acc.z, rden, m.z),
-                 fmaf(acc.w, rden, m.w));
+    float den_sum = 0.0f;
+    float weight[KS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      weight[k] = st[k].y == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(st[k].y - top);
+      den_sum = fmaf(st[k].x, weight[k], den_sum);
+    }
+    const float rden = (1.0f / 255.0f) / fmaxf(den_sum, 1e-30f);
+    const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
+#pragma unroll
+    for (int i = 0; i < kShare; ++i) {
+      const int four = part * kShare + i;  // this wave's share of the features: 4 j + g
+      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        const float4 v = sums[((k * kGroups + group) * 4 * kChunksD + four) * 64 + lane];
+        acc.x = fmaf(v.x, weight[k], acc.x);
+        acc.y = fmaf(v.y, weight[k], acc.y);
+        acc.z = fmaf(v.z, weight[k], acc.z);
+        acc.w = fmaf(v.w, weight[k], acc.w);
+      }
+      const int d0 = 8 * four + 4 * h;  // 32 j + 8 g + 4 h
+      const float4 m = *reinterpret_cast<const float4*>(p.value_mean + static_cast<long>(bh) * D + d0);
+      store4<kOut>(p.output, out_row + d0, fmaf(acc.x, rden, m.x), fmaf(acc.y, rden, m.y), fmaf(acc.z, rden, m.z),
+                   fmaf(acc.w, rden, m.w));
+    }
   }
 }
 

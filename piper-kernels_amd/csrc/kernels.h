@@ -78,22 +78,26 @@ constexpr int stream_workgroups(int head_dim, int streams) {
   return streams == 4 ? 1 : head_dim == 64 ? 3 : 2;
 }
 
-// Key streams of a grid whose plan does not choose them (causal Piper Attention, SageAttention2++), from its
-// 128-row query tiles and 64-key tiles: four where that gives at most one workgroup per CU, two where that
-// does, and two for causal grids of up to two (SageAttention2++ one) workgroups of 128 rows per CU, whose
-// longest tile sets the time, if the keys are long enough to pay for the shorter query tiles' prologues.
-// SageAttention2++'s iterations exchange their maxima, and beyond 4096 keys a row's rounding should not
-// depend on the batch: no streams there.  Measured, none against the choice (us, 10-13 of them the launching
-// loop's floor): Piper Attention causal B1 H8 S1024 D64 21.9, 11.3 (4); B2 H16 S1531 D128 42.4, 34.5 (2); B1
-// H12 S4096 98.8, 67.9 (2); B1 H8 S8192 198, 162 (2); on the other side of the line B1 H24 S4096 (768
-// tiles) 114, two streams 129, and B4 H32 S512 (512 tiles of 8) 21.5, 26.3.  SageAttention2++ B1 H8 S1024
-// D64 18.2, 11.1 (4); B1 H16 S1024 D128 24.3, 19.7 (2); causal B1 H16 S2048 43.1, 34.3 (2); not taken: B1 H16
-// S2048 42.9, 45.1, causal B2 H16 S1531 36.8, 38.8.
-inline int small_grid_streams(bool sage, bool causal, long tiles, int key_tiles, int cus) {
+// Key streams of a grid whose plan does not choose them (causal Piper Attention, SageAttention2++; both give the
+// sequential kernels' bits), from its 128-row query tiles and 64-key tiles: four where that gives at most one
+// workgroup per CU, two where that does, and two for causal grids of up to `quarters` quarters of a
+// workgroup of 128 rows per CU, whose longest tile sets the time, if the keys are long enough to pay for the
+// shorter query tiles' prologues.
+// Measured, none against the choice (us without the host): Piper Attention causal B1 H8 S1024 D64 22, 11.6
+// (4); B1 H9 S1024 D128 27.5, 21.1 (2); B2 H16 S1531 D128 42, 36.5 (2); B1 H12 S4096 98, 72 (2); B1 H8 S8192
+// 198, 177 (2); B1 H2 S32768 734, 668 (2).  At the line, D = 128: S1024 (16 key tiles) 384 query tiles 30.8,
+// 29.7, not taken 448 31.4, 33.7; S1536 432 tiles 41.9, 40.5, not 504 42.1, 46.8; S2048 448 tiles 53.1, 50.3,
+// not 512 54.0, 55.8; S3072 not 504 75.7, 76.9; S4096 512 tiles 98.9, 95.4, not 768 114, 129.  D = 64: 512 tiles
+// of S1024 23.1, 23.3, of S2048 40.7, 33.9.  SageAttention2++ B1 H8 S1024 D64 18.2, 11.9 (4); B1 H16 S1024 D128
+// 24.3, 21.0 (2); causal B1 H16 S2048 43.1, 36.6 (2); B1 H32 S1024 D128 26.0, 22.5 (2); not taken: B1 H16 S2048
+// 42.9, 45.1, causal B2 H16 S1531 36.8, 38.8.
+inline int small_grid_streams(bool sage, bool causal, int head_dim, long tiles, int key_tiles, int cus) {
   if (key_tiles < 4 || (sage && key_tiles > 64)) return 1;
   if (4 * tiles <= cus) return 4;
   if (2 * tiles <= cus) return 2;
-  return causal && key_tiles >= 16 && tiles <= (sage ? 1L : 2L) * cus ? 2 : 1;
+  if (!causal || key_tiles < 16) return 1;
+  const int quarters = sage ? 4 : head_dim == 64 || key_tiles >= 64 ? 8 : key_tiles >= 24 ? 7 : 6;
+  return 4 * tiles <= static_cast<long>(quarters) * cus ? 2 : 1;
 }
 
 struct InputTensor {

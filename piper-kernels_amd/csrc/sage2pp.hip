@@ -99,9 +99,8 @@ __device__ __forceinline__ float sage_block_raw(const v16i (&s)[2], const float 
   }
 }
 
-template <int D>
-__device__ __forceinline__ void sage_frame(float next, v16f (&acc)[D / 32], float& den, float& mrun) {
-  constexpr int kChunksD = D / 32;
+template <int kChunksD>
+__device__ __forceinline__ void sage_frame(float next, v16f (&acc)[kChunksD], float& den, float& mrun) {
   const bool grow = next > mrun;
   if (__builtin_amdgcn_ballot_w64(grow) != 0) {
     const float w = grow ? __builtin_amdgcn_exp2f(mrun - next) : 1.0f;  // exp2(-inf) = 0 at the start
@@ -119,12 +118,21 @@ __device__ __forceinline__ void sage_block_head(const v16i (&s)[2], const float 
                                                 int h, int key_length, float (&x)[32], v16f (&acc)[D / 32],
                                                 float& den, float& mrun) {
   const float block_max = sage_block_raw<kCausal, kPerThread>(s, ct, t, q0, n, h, key_length, x);
-  sage_frame<D>(fmaxf(mrun, block_max), acc, den, mrun);
+  sage_frame(fmaxf(mrun, block_max), acc, den, mrun);
 }
 
-template <int D, int NW, bool kFp16Partials>
+// What a wave of the key-stream kernel hands on of its block: the FP8 codes and this lane half's share of
+// the denominator.
+struct SageCodes {
+  uint32_t pw[8];
+  float den;
+};
+
+// kCodes: the codes and the denominator share only, into `codes` (sage_fold_blocks adds them).
+template <int D, int NW, bool kFp16Partials, bool kCodes = false>
 __device__ __forceinline__ void sage_block_tail(const char* stage, const float (&x)[32], const float (&ct)[4], int n,
-                                                int h, v16f (&acc)[D / 32], float& den, float mrun) {
+                                                int h, v16f (&acc)[D / 32], float& den, float mrun,
+                                                SageCodes* codes = nullptr) {
   using L = SageLayout<D, NW>;
   constexpr int kChunksD = D / 32;
   // ---- p = exp2(s ct - m') in [0, 448], the denominator share and the FP8 codes ----
@@ -142,6 +150,12 @@ __device__ __forceinline__ void sage_block_tail(const char* stage, const float (
     ps[2] += e2;
     ps[3] += e3;
     pw[q] = pack_fp8(e0, e1, e2, e3);
+  }
+  if constexpr (kCodes) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) codes->pw[q] = pw[q];
+    codes->den = (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    return;
   }
   den += (ps[0] + ps[1]) + (ps[2] + ps[3]);
   const v8i p = {static_cast<int>(pw[0]), static_cast<int>(pw[1]), static_cast<int>(pw[2]), static_cast<int>(pw[3]),
@@ -398,23 +412,67 @@ sage_attention_w3_kernel(const SageParams p) {
   }
 }
 
-// Key streams, as Piper Attention's attention_streams_kernel: KS waves of a workgroup share 32 queries and
-// take every KS-th key tile each.  FP8 probabilities round relative to the running maximum, so the waves
-// exchange their block maxima in every iteration (one more barrier) and each tile gets the frame that the
-// sequential kernel gives it, max over the tiles up to it: every probability code is the sequential
-// kernel's, and only the FP32 sums are added in another order.
+// Where a key-stream wave leaves its block for the others: codes (two 16-byte pieces per lane) and the
+// denominator's share, in the tile's K rows, which every wave has read by then.
+template <int D, int KS>
+struct SageExchange {
+  static constexpr int kGroups = 4 / KS;
+  static constexpr int kDen = 2048;
+  static constexpr int kSlot = sage_v_offset(D) / kGroups;
+  static_assert(kDen + 256 <= kSlot && kSlot % 16 == 0, "a wave's block fits its share of the K rows");
+};
+
+// The sums of one query group over tiles [t, t + KS) of an iteration, in tile order and with the arithmetic of
+// sage_frame and sage_block_tail, for the wave's share of the features (StreamShare): the same bits as one
+// wave that runs the tiles one after another.  frames[k]: the running maximum up to tile t + k.
+template <int D, int KS>
+__device__ __forceinline__ void sage_fold_blocks(const char* stages, const float (&frames)[KS], int t, int wave_tiles, int group,
+                                                 int part, int lane, v16f (&acc)[StreamShare<D, KS>::kChunks], float& den,
+                                                 float& mrun) {
+  using L = SageLayout<D, 4>;
+  using S = StreamShare<D, KS>;
+  const int chunk = S::chunk(part);
+  const int vrow = (32 * chunk + ((lane & 31) ^ (16 * S::half(part)))) * L::kVStride + 16 * (lane >> 5);
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    if (t + k >= wave_tiles) break;
+    const char* stage = stages + k * L::kStageBytes;
+    const char* slot = stage + group * SageExchange<D, KS>::kSlot;
+    const v4i p0 = *reinterpret_cast<const v4i*>(slot + 16 * lane);
+    const v4i p1 = *reinterpret_cast<const v4i*>(slot + 1024 + 16 * lane);
+    const float share = *reinterpret_cast<const float*>(slot + SageExchange<D, KS>::kDen + 4 * lane);
+    const v8i p = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
+    sage_frame(frames[k], acc, den, mrun);
+    den += share;
+#pragma unroll
+    for (int c = 0; c < S::kChunks; ++c) {
+      const char* v = stage + L::kVOffset + vrow + 32 * c * L::kVStride;
+      const v4i a0 = *reinterpret_cast<const v4i*>(v);
+      const v4i a1 = *reinterpret_cast<const v4i*>(v + 32);
+      const v8i a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+      acc[c] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, p, acc[c], 0, 0, 0, 0, 0, 0);
+    }
+  }
+}
+
+// Key streams, as Piper Attention's attention_streams_kernel (one tile's scores and codes per wave, then each
+// wave all tiles for its share of the features).  FP8 probabilities round relative to the running maximum, so
+// the waves first exchange their block maxima and each tile gets the frame that the sequential kernel
+// gives it, the maximum over the tiles up to it.  Bit-identical to the other kernels, so a row's bits do not
+// depend on how many batch-heads the call has.  us without streams, with sums merged at the end instead (whose
+// FP32 additions came in another order), and so: B1 H8 S1024 D64 18.2, 10.6, 11.9; B1 H16 S1024 D128 24.3,
+// 19.8, 21.0; causal B1 H16 S2048 43.1, 33.7, 36.6; B1 H4 S4096 D64 59, 41.4, 47.4.
 template <int D, bool kCausal, int kOut, bool kPerThread, int KS>
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, KS == 4 ? 512 : 256), amdgpu_waves_per_eu(KS == 4 ? 2 : stream_workgroups(D, KS), KS == 4 ? 2 : stream_workgroups(D, KS))))
 sage_streams_kernel(const SageParams p) {
   using L = SageLayout<D, 4>;
+  using S = StreamShare<D, KS>;
   constexpr int kChunksD = D / 32;
   constexpr int kGroups = 4 / KS;
   constexpr int kStage = KS * L::kStageBytes;
   constexpr int kRounds = stream_rounds<L, KS>();
-  constexpr int kShare = 4 * kChunksD / KS;  // four-feature groups that a wave writes at the end
   __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
   __shared__ float maxima[4][32];  // [wave][query]: the iteration's block maxima
-  static_assert(4 * (D * 32 * 4 + 512) <= 2 * kStage, "every wave's sums fit the stages");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -454,11 +512,11 @@ sage_streams_kernel(const SageParams p) {
     for (int c = 0; c < kChunksD; ++c) qf[c] = v4i{0, 0, 0, 0};
   }
 
-  v16f acc[kChunksD];
+  v16f acc[S::kChunks];
 #pragma unroll
-  for (int j = 0; j < kChunksD; ++j)
+  for (int c = 0; c < S::kChunks; ++c)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[c][r] = 0.0f;
   float den = 0.0f;
   float mrun = -__builtin_inff();  // the frame of this wave's sums
   float seen = -__builtin_inff();  // the running maximum over every tile of the iterations before
@@ -469,7 +527,8 @@ sage_streams_kernel(const SageParams p) {
     stage_barrier<0>();  // this iteration's records landed, every read of the last one's (and of maxima) is done
     if (i + 1 < steps) copy_tiles<L, KS>(p, smem + ((i + 1) & 1) * kStage, bh, KS * (i + 1), tiles, wave, lane);
     const int t = KS * i + part;
-    const char* stage = smem + (i & 1) * kStage + part * L::kStageBytes;
+    char* stages = smem + (i & 1) * kStage;
+    char* stage = stages + part * L::kStageBytes;
     float ct[4];
     float x[32];
     float block_max = -__builtin_inff();
@@ -488,63 +547,45 @@ sage_streams_kernel(const SageParams p) {
       block_max = sage_block_raw<kCausal, kPerThread>(sc, ct, t, q0, n, h, p.key_length, x);
     }
     if (h == 0) maxima[wave][n] = block_max;  // both lane halves hold it
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    float frame = seen;
+    stream_barrier();  // every wave's maximum is there, every wave has read the K rows
+    float frames[KS];
+    float own = seen;  // this wave's tile's frame
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      const float m = maxima[k * kGroups + group][n];
-      seen = fmaxf(seen, m);
-      if (k <= part) frame = seen;
+    for (int j = 0; j < KS; ++j) {
+      seen = fmaxf(seen, maxima[j * kGroups + group][n]);
+      frames[j] = seen;
+      if (j <= part) own = seen;
     }
     if (t < wave_tiles) {
-      sage_frame<D>(frame, acc, den, mrun);
-      sage_block_tail<D, 4, false>(stage, x, ct, n, h, acc, den, mrun);
+      SageCodes codes;
+      v16f no_acc[kChunksD];  // not touched
+      float no_den = 0.0f;
+      sage_block_tail<D, 4, false, true>(stage, x, ct, n, h, no_acc, no_den, own, &codes);
+      char* slot = stage + group * SageExchange<D, KS>::kSlot;
+      *reinterpret_cast<uint4*>(slot + 16 * lane) = make_uint4(codes.pw[0], codes.pw[1], codes.pw[2], codes.pw[3]);
+      *reinterpret_cast<uint4*>(slot + 1024 + 16 * lane) = make_uint4(codes.pw[4], codes.pw[5], codes.pw[6], codes.pw[7]);
+      *reinterpret_cast<float*>(slot + SageExchange<D, KS>::kDen + 4 * lane) = codes.den;
     }
+    stream_barrier();  // every wave's block is there
+    sage_fold_blocks<D, KS>(stages, frames, KS * i, wave_tiles, group, part, lane, acc, den, mrun);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const float den_total = cross_half_sum(den);
-  __syncthreads();  // every wave is done with the stages
 
-  // every wave's sums: [wave][four-feature group][lane] float4, then [wave][lane] float2 (den, frame)
-  float4* sums = reinterpret_cast<float4*>(smem);
-  float2* stats = reinterpret_cast<float2*>(smem + 4 * D * 32 * 4);
-#pragma unroll
-  for (int j = 0; j < kChunksD; ++j)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      sums[(wave * 4 * kChunksD + 4 * j + g) * 64 + lane] =
-          make_float4(acc[j][4 * g + 0], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]);
-  stats[wave * 64 + lane] = make_float2(den_total, mrun);
-  __syncthreads();
+  const float total = cross_half_sum(den);
   const int query = q0 + n;
   if (!wave_live || query >= p.query_length) return;
-  float total = 0.0f;
-  float weight[KS];
-#pragma unroll
-  for (int k = 0; k < KS; ++k) {
-    const float2 st = stats[(k * kGroups + group) * 64 + lane];
-    weight[k] = st.y == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(st.y - seen);
-    total = fmaf(st.x, weight[k], total);
-  }
   const float rden = 1.0f / fmaxf(total, 1e-30f);
   const float* vscale = p.value_scale + static_cast<long>(bh) * D;
   const long out_row = (static_cast<long>(bh) * p.query_length + query) * D;
 #pragma unroll
-  for (int i = 0; i < kShare; ++i) {
-    const int four = part * kShare + i;  // this wave's share of the features: 4 j + g
-    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int c = 0; c < S::kChunks; ++c) {
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      const float4 v = sums[((k * kGroups + group) * 4 * kChunksD + four) * 64 + lane];
-      sum.x = fmaf(v.x, weight[k], sum.x);
-      sum.y = fmaf(v.y, weight[k], sum.y);
-      sum.z = fmaf(v.z, weight[k], sum.z);
-      sum.w = fmaf(v.w, weight[k], sum.w);
+    for (int g = 0; 4 * g < S::kRegs; ++g) {
+      const int d0 = 32 * (S::chunk(part) + c) + 16 * S::half(part) + 8 * g + 4 * h;
+      const float4 vs = *reinterpret_cast<const float4*>(vscale + d0);
+      store4<kOut>(p.output, out_row + d0, (acc[c][4 * g + 0] * vs.x) * rden, (acc[c][4 * g + 1] * vs.y) * rden,
+                   (acc[c][4 * g + 2] * vs.z) * rden, (acc[c][4 * g + 3] * vs.w) * rden);
     }
-    const int d0 = 8 * four + 4 * h;  // 32 j + 8 g + 4 h
-    const float4 vs = *reinterpret_cast<const float4*>(vscale + d0);
-    store4<kOut>(p.output, out_row + d0, (sum.x * vs.x) * rden, (sum.y * vs.y) * rden, (sum.z * vs.z) * rden,
-                 (sum.w * vs.w) * rden);
   }
 }
 

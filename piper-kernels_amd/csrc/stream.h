@@ -164,6 +164,24 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kInFlight) : "memory");
 }
 
+// A key-stream wave's share of the numerator: whole 32-feature chunks or, where there are more streams than
+// chunks, the 16 features that a permuted V^T row order brings into a chunk's first eight registers.
+template <int D, int KS>
+struct StreamShare {
+  static constexpr int kChunks = D / 32 >= KS ? D / 32 / KS : 1;
+  static constexpr int kRegs = D / 32 >= KS ? 16 : 8;
+  static constexpr int kSplit = D / 32 >= KS ? 1 : KS / (D / 32);  // waves per chunk
+  static_assert(kSplit <= 2, "halves of a chunk at most");
+  __device__ static int chunk(int part) { return kSplit == 1 ? part * kChunks : part / kSplit; }
+  __device__ static int half(int part) { return part % kSplit; }
+};
+
+// Barrier between the phases of a key-stream iteration: every wave's LDS reads and writes so far are done,
+// direct copies stay in flight.
+__device__ __forceinline__ void stream_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 template <class L>
 __device__ __forceinline__ void stage_barrier_keep_last(int wave) {
   if (wave < L::kFullWaves)

@@ -316,7 +316,7 @@ class NativeLibrary:
         )
 
     def attention_forward_balanced(self, args: PiperAttentionFusedArgs, stream: int) -> None:
-        """attention_forward_fused, free to run a small causal grid as key streams (equal to rounding)."""
+        """attention_forward_fused, free to run a small causal grid as key streams (the same bits)."""
         self._check(self._lib.piper_attention_forward_balanced(ctypes.byref(args), _ptr(stream)),
                     "piper_attention_forward_balanced")
 
@@ -336,7 +336,7 @@ class NativeLibrary:
         )
 
     def sage_attention_forward_balanced(self, args: PiperSageAttentionArgs, stream: int) -> None:
-        """sage_attention_forward, free to run a small grid as key streams (equal to rounding)."""
+        """sage_attention_forward, free to run a small grid as key streams (the same bits)."""
         self._check(self._lib.piper_sage_attention_forward_balanced(ctypes.byref(args), _ptr(stream)),
                     "piper_sage_attention_forward_balanced")
 

@@ -2,7 +2,9 @@
 edges -- fewer key tiles than streams, key tiles that do not divide, query rows past the end in one of a
 workgroup's groups, one row -- against the unsplit kernel and the oracle; the two-step and the fused
 entry points bit for bit alike.  The balanced entry points, which choose streams themselves (causal Piper
-Attention, SageAttention2++), against the others."""
+Attention, SageAttention2++), bit for bit the others, scores whose block maxima grow, leave the
+subtraction-free range or are not finite among them; a batch-head's output bit for bit the same alone and
+in a batch."""
 
 from __future__ import annotations
 
@@ -74,7 +76,7 @@ BALANCED = [
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("case", BALANCED, ids=str)
-def test_balanced_entry_points_equal_the_others_to_rounding(case, d, gfx950_device, monkeypatch) -> None:
+def test_balanced_entry_points_equal_the_others_bit_for_bit(case, d, gfx950_device, monkeypatch) -> None:
     from piper_kernels.attention.piper_attention.hip import _launch_piper_attention, _prepare_piper_attention
     from piper_kernels.attention.sage_attention_2pp.hip import _launch_sage_attention_2pp, _prepare_sage_attention_2pp
 
@@ -93,6 +95,59 @@ def test_balanced_entry_points_equal_the_others_to_rounding(case, d, gfx950_devi
             outs.append(_launch_piper_attention(prepared, output=out))
         else:
             outs.append(_launch_sage_attention_2pp(_prepare_sage_attention_2pp(q, k, v, d**-0.5, causal), output=out))
-    # every probability code is the same (an FP8 code off by one step would show as 1e-3); the FP32 sums
-    # enter in another order: a few ulps of a value of the outputs' size
-    assert (outs[0] - outs[1]).abs().max().item() <= 2e-6 * max(1.0, outs[0].abs().max().item())
+    assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("granularity", ["per_thread", "per_warp"])
+@pytest.mark.parametrize("operator", ["piper", "sage"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_growing_and_extreme_scores_bit_for_bit(d, operator, granularity, gfx950_device, monkeypatch) -> None:
+    """Keys that grow along the sequence (the frame moves in most tiles), rows of large queries (block maxima past
+    the subtraction-free range), an infinite and a NaN value: two and four streams against the other kernels."""
+    from piper_kernels.attention.sage_attention_2pp.hip import _launch_sage_attention_2pp, _prepare_sage_attention_2pp
+
+    log(f"[case] streams, extreme scores {operator} D={d} {granularity}")
+    g = torch.Generator().manual_seed(d)
+    lib = native.load_library()
+    for heads, causal, bad in ((2, False, False), (2, True, False), (9, True, False), (2, False, True), (2, True, True)):
+        if operator == "piper" and not causal:
+            continue
+        s = 1000
+        q = torch.randn((1, heads, s, d), generator=g)
+        q[:, :, 100:200] *= 60
+        k = torch.randn((1, heads, s, d), generator=g) * torch.linspace(0.1, 12, s).reshape(1, 1, s, 1)
+        v = torch.randn((1, heads, s, d), generator=g)
+        v[:, :, 37] *= 1000
+        if bad:
+            q[:, 0, 5, 3], v[:, 0, 300, 2], k[:, 1, 700, 1] = float("nan"), float("inf"), float("inf")
+        q, k, v = (x.to(torch.bfloat16).to(gfx950_device) for x in (q, k, v))
+        outs = []
+        for handle in (lib, _Balanced(lib)):
+            monkeypatch.setattr(native, "load_library", lambda *a, handle=handle: handle)
+            if operator == "sage":
+                out = torch.empty((1, heads, s, d), device=gfx950_device)
+                p = _prepare_sage_attention_2pp(q, k, v, d**-0.5, causal, qk_granularity=granularity)
+                outs.append(_launch_sage_attention_2pp(p, output=out))
+            else:
+                outs.append(gpu_attention(gpu_prepare(q, k, v, d**-0.5, causal, gfx950_device, quantize_query=False,
+                                                      qk_granularity=granularity)))
+        assert torch.allclose(outs[0], outs[1], rtol=0, atol=0, equal_nan=True)
+        assert bad or torch.isfinite(outs[0]).all()
+
+
+@pytest.mark.parametrize("operator", ["piper", "sage"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_a_batch_head_alone_and_in_a_batch(d, operator, gfx950_device) -> None:
+    """The public operators choose streams by the grid: four, two or none for one, six and many batch-heads."""
+    from piper_kernels import piper_attention, sage_attention_2pp
+
+    public = piper_attention if operator == "piper" else sage_attention_2pp
+    log(f"[case] batch against alone {operator} D={d}")
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (torch.randn((2, 40, 1031, d), generator=g).to(torch.float16).to(gfx950_device) for _ in range(3))
+    with torch.no_grad():
+        for causal in (True,) if operator == "piper" else (True, False):
+            want = public(q, k, v, is_causal=causal)
+            for heads in (1, 6, 14):
+                got = public(q[1:, :heads], k[1:, :heads], v[1:, :heads], is_causal=causal)
+                assert torch.equal(got, want[1:, :heads]), heads

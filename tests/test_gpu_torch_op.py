@@ -52,10 +52,7 @@ def test_native_call_equals_the_python_path(case, operator, gfx950_device) -> No
             got = public(q, k, v, scale=scale, is_causal=causal)
             want = python(q, k, v, d**-0.5 if scale is None else scale, causal)
             assert got.is_contiguous() and got.dtype is dtype
-            # the op may run key streams, whose FP32 sums differ by rounding (1e-5 as for the split plans)
-            # and can round to the neighbouring 16-bit value
-            step = 2.0 ** (-10 if dtype is torch.float16 else -7)
-            torch.testing.assert_close(got.float(), want.float(), rtol=step, atol=1e-5)
+            assert torch.equal(got, want)
 
 
 @pytest.mark.gpu
