@@ -89,10 +89,11 @@ constexpr int stream_workgroups(int head_dim, int streams) {
 // 29.7, not taken 448 31.4, 33.7; S1536 432 tiles 41.9, 40.5, not 504 42.1, 46.8; S2048 448 tiles 53.1, 50.3,
 // not 512 54.0, 55.8; S3072 not 504 75.7, 76.9; S4096 512 tiles 98.9, 95.4, not 768 114, 129.  D = 64: 512 tiles
 // of S1024 23.1, 23.3, of S2048 40.7, 33.9.  SageAttention2++ B1 H8 S1024 D64 18.2, 11.9 (4); B1 H16 S1024 D128
-// 24.3, 21.0 (2); causal B1 H16 S2048 43.1, 36.6 (2); B1 H32 S1024 D128 26.0, 22.5 (2); not taken: B1 H16 S2048
+// 24.3, 21.0 (2); B1 H24 Sq256 Sk16384 268, 166 (4); B1 H1 S8192 140, 87 (4); B1 H2 S6000 D64 84.6, 67.5 (2);
+// causal B1 H16 S2048 43.1, 36.6 (2); B1 H32 S1024 D128 26.0, 22.5 (2); B1 H1 S16384 276, 230 (2); not taken: B1 H16 S2048
 // 42.9, 45.1, causal B2 H16 S1531 36.8, 38.8.
 inline int small_grid_streams(bool sage, bool causal, int head_dim, long tiles, int key_tiles, int cus) {
-  if (key_tiles < 4 || (sage && key_tiles > 64)) return 1;
+  if (key_tiles < 4) return 1;
   if (4 * tiles <= cus) return 4;
   if (2 * tiles <= cus) return 2;
   if (!causal || key_tiles < 16) return 1;

@@ -71,6 +71,8 @@ BALANCED = [
     ("sage", 1, 5, 97, 300, False),
     ("sage", 1, 40, 257, 700, False),
     ("sage", 2, 40, 257, 700, False),
+    ("sage", 1, 2, 100, 8257, False),  # more than 128 key tiles
+    ("sage", 1, 1, 4500, 4500, True),
 ]
 
 
