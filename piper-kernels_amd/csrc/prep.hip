@@ -24,10 +24,12 @@ namespace piper {
 
 // K and V bytes up to which the two-pass prep, which reads them twice (the second time from the last-level
 // cache), beats the single pass, whose chunks wait for one another.  At D = 64 a chunk in flight is half
-// as large and the waits weigh more: B2 H24 S8192 (100 MB) 50.8 us against 54.7, B4 H24 S8192 (200 MB)
-// 106.6 against 103.8 (causal 104.8 against 89.3).  At D = 128 the two tie up to 50 MB (B1 H24 S2048 and
-// S4096) and the single pass wins from there: B2 H24 S4096 (100 MB) 45.3 us against 50.9,
-// SageAttention2++ 40.7 against 48.6.
+// as large and the waits weigh more.  us of the whole prep without the host, two-pass against single pass
+// (full, causal, SageAttention2++): D = 128, 25 MB (24 heads of 2048) 19.4-21.8, 17.9-19.1, 17.5-18.9; 34 MB (16 of
+// 4096) 23-24.8, 19.7-20.6, 20.7-20.4; 50 MB (24 of 4096) 29.8-30.5, 25.9-25.2, 26.7-25.4; 67 MB (16 of 8192)
+// 40.5-36.5, 34.1-28.7, 37.9-31.3; 101 MB (48 of 4096) 55.8-48.3, 46.0-40.7, 51.4-43.2.  D = 64, 42 MB (40 of
+// 4096) 26.8-32.7, 23.5-24.8, 23.6-27.2; 67 MB (64 of 4096) 39.2-39.8, 33.8-33.4, 35.8-35.2; 101 MB (48 of 8192)
+// 55.8-56.5, 48.2-47.3, 51.6-50.8; 201 MB (96 of 8192) 112-102, 90.2-84.3, 108-91.
 constexpr long two_pass_bytes(int head_dim) { return (head_dim == 64 ? 128L : 32L) << 20; }
 
 template <int D, bool kSage>
