@@ -243,17 +243,20 @@ def piper_heuristic_plan(batch: int, heads: int, query_length: int, is_causal: b
     waves per SIMD from three independent workgroups, one wave's MFMA, LDS and barrier waits are
     filled by the other two: measured 7-24% faster than the two-waves-per-SIMD plans at c2-c5.
     Non-causal grids too small or too ragged for whole rounds of resident workgroups split their key
-    range (``split_parts``).  Otherwise a non-causal grid of head size 128 whose 256-query tiles give
-    every CU exactly one runs two waves per SIMD either way; one 8-wave workgroup per CU is then 1-2%
-    faster (measured at r1, B1 H8 N8192; one 256-query tile more costs a round: B1 H10 N8192 474 us
-    against 320)."""
+    range (``split_parts``).  Otherwise a non-causal grid of head size 128 and at least 128 key tiles whose
+    256-query tiles give every CU exactly one runs two waves per SIMD either way, and one 8-wave workgroup
+    per CU is 0.3-0.8% faster (us, three per CU against wide: B1 H8 S8192 244.0, 243.2; B1 H4 S16384 473.4,
+    470.9; B1 H2 S32768 934.5, 927.3).  With fewer keys it is slower (B1 H16 S4096 128.8, 128.5 but B1 H32 S2048
+    69.2, 72.0; B1 H64 S1024 41.5, 43.5; Sk512 27.1, 28.5), and one 256-query tile more costs a round (B1 H10
+    S8192 320, 474)."""
     three = MI355XPlan(waves=4, three_per_cu=True)
     wide = MI355XPlan(waves=8)
     if not is_causal:
-        parts = split_parts(batch, heads, query_length, query_length if key_length is None else key_length, head_dim)
+        keys = query_length if key_length is None else key_length
+        parts = split_parts(batch, heads, query_length, keys, head_dim)
         if parts > 1:
             return MI355XPlan(waves=4, three_per_cu=True, key_parts=parts)
-        if head_dim == 128 and wide.workgroups(batch, heads, query_length) == COMPUTE_UNITS:
+        if head_dim == 128 and keys >= 128 * KEY_BLOCK and wide.workgroups(batch, heads, query_length) == COMPUTE_UNITS:
             return wide
     return three
 

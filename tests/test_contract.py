@@ -481,3 +481,13 @@ print(sorted(n for n in dir(torch.ops.piper_kernels) if n.startswith("piper_atte
     assert "duplicate registration refused" in result.stdout
     assert "'piper_attention', 'piper_attention_hip'" in result.stdout
 
+
+
+def test_wide_workgroups_need_long_keys() -> None:
+    """One 8-wave workgroup per CU only pays for grids of exactly one per CU whose key loop is long."""
+    from piper_kernels.attention.piper_attention import _plan
+
+    three = MI355XPlan(waves=4, three_per_cu=True)
+    for heads, sq, sk in ((16, 4096, 4096), (64, 1024, 1024), (256, 256, 512), (8, 8192, 8128), (17, 3800, 3800)):
+        assert _plan.piper_heuristic_plan(1, heads, sq, False, sk) == three
+    assert _plan.piper_heuristic_plan(1, 4, 16384, False, 16384) == MI355XPlan(waves=8)
