@@ -1,10 +1,10 @@
 // The operators' torch kernels (libpiper_torch.so): piper_kernels::piper_attention and
 // piper_kernels::sage_attention_2pp on GPU tensors, over the C ABI of libpiper_mi355x.so.
 //
-// Short calls are bound by the host: in Python, filling the argument structs, ten allocations and the
-// stream and device queries took 41 us of a 59 us call at B1 H4 Sq35 Sk67 D64 whose kernels take 14 us.
-// Here a call makes two allocations (the output, and one workspace that holds every prepared buffer) and
-// the library's two calls: the same call issues in 17 us.  The op's definition, its fake and its autograd stay in Python
+// Short calls are bound by the host: at B1 H4 Sq35 Sk67 D64, whose kernels take 13 us, the same two library
+// calls from Python, with their argument structs, ten allocations and stream and device queries, take 41 us
+// (calls in a row).  Here a call makes two allocations (the output, and one workspace that holds every prepared
+// buffer): the whole public call takes 17 us.  The op's definition, its fake and its autograd stay in Python
 // (torch.library.custom_op), which also runs calls under an explicit launch plan.
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
