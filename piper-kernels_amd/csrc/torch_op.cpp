@@ -90,14 +90,16 @@ struct Arena {
   }
 };
 
-// The kernels read key and value by the query's shape, type and device: what the public functions refuse is
-// refused here too, where a program can call the op itself.  Returns the device.
-c10::Device checked_device(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
+// The kernels read key and value by the query's shape and device, the value by the key's type and Piper
+// Attention's key by the query's: tensors that do not match are refused here too, where a program can call
+// the op itself.  Returns the device.
+c10::Device checked_device(Operator op, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
   TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4,
               "piper_kernels: tensors must have shape [batch, heads, sequence, head_dim]");
   TORCH_CHECK(k.device() == q.device() && v.device() == q.device(),
               "piper_kernels: query, key and value must share a device");
-  TORCH_CHECK(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type(),
+  // SageAttention2++'s prep reads no query: that has a type of its own, which is the output's
+  TORCH_CHECK(v.scalar_type() == k.scalar_type() && (op == kSage || k.scalar_type() == q.scalar_type()),
               "piper_kernels: query, key and value must share a dtype");
   TORCH_CHECK(k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(1) == q.size(1) && k.size(3) == q.size(3),
               "piper_kernels: batch, heads and head_dim must agree and key and value lengths match, got ", q.sizes(), ", ",
@@ -114,8 +116,8 @@ struct Call {
   c10::Stream stream;
   void* handle;
 
-  Call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v)
-      : guard(checked_device(q, k, v)),
+  Call(Operator op, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v)
+      : guard(checked_device(op, q, k, v)),
         query(native_input(q)),
         key(native_input(k)),
         value(native_input(v)),
@@ -137,7 +139,7 @@ struct Call {
 
 at::Tensor piper_attention(const at::Tensor& query, const at::Tensor& key, const at::Tensor& value, double scale,
                            bool is_causal) {
-  Call call(query, key, value);
+  Call call(kPiper, query, key, value);
   piper_layout layout;
   check(piper_prepared_layout(&call.shape, &layout), "piper_prepared_layout");  // refuses bad shapes
   const int32_t plan = plan_for(kPiper, call.shape, is_causal);
@@ -195,7 +197,7 @@ at::Tensor piper_attention(const at::Tensor& query, const at::Tensor& key, const
 
 at::Tensor sage_attention_2pp(const at::Tensor& query, const at::Tensor& key, const at::Tensor& value, double scale,
                               bool is_causal) {
-  Call call(query, key, value);
+  Call call(kSage, query, key, value);
   piper_sage_layout layout;
   check(piper_sage_prepared_layout(&call.shape, &layout), "piper_sage_prepared_layout");  // refuses bad shapes
   const int32_t plan = plan_for(kSage, call.shape, is_causal);

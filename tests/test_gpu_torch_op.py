@@ -114,12 +114,25 @@ def test_the_op_refuses_tensors_that_do_not_belong_together(operator, gfx950_dev
     for key, value, text in [
         (q, q[:, :, :7], "key and value lengths match"),
         (q[:, :1], q[:, :1], "heads and head_dim must agree"),
-        (q.bfloat16(), q.bfloat16(), "share a dtype"),
+        (q, q.bfloat16(), "share a dtype"),
+        *([(q.bfloat16(), q.bfloat16(), "share a dtype")] if operator == "piper_attention" else []),
         (q.cpu(), q.cpu(), "share a device"),
         (q[0], q[0], "must have shape"),
     ]:
         with pytest.raises(RuntimeError, match=text):
             op(q, key, value, 0.125, False)
+
+
+@pytest.mark.gpu
+def test_sage_query_of_another_type_than_the_keys(gfx950_device) -> None:
+    """Accepted by the op (the public function asks for one type): the output has the query's type."""
+    native.load_torch_kernels()
+    log("[case] torch op sage, fp16 query on bf16 keys")
+    q, k, v = _inputs(1, 2, 100, 300, 64, torch.bfloat16, gfx950_device)
+    with torch.no_grad():
+        got = torch.ops.piper_kernels.sage_attention_2pp(q.half(), k, v, 0.125, False)
+        assert got.dtype is torch.float16
+        assert torch.equal(got, _run_sage_attention_2pp(q.half(), k, v, 0.125, False))
 
 
 def test_plan_source_asks_the_package(monkeypatch) -> None:
@@ -173,7 +186,7 @@ library.load_torch_kernels()
 @pytest.mark.gpu
 def test_first_call_of_a_process_equals_the_next(gfx950_device) -> None:
     """A compiled graph, or the op itself, can be a process's first use; its bits are those of every later call
-    (shapes that run key streams, whose sums have an order of their own)."""
+    (shapes that run key streams)."""
     log("[case] first call of a process")
     program = """
 import sys
